@@ -189,7 +189,7 @@ class Life:
     dtype = "u8"
     bytes_per_lup = 2.0  # 1 B read + 1 B write of the uint8 cell format
 
-    def __init__(self, n=16384, generations=1000, seed=synthetic.DEFAULT_SEED, per_launch=31, variant=7, wrap=0):
+    def __init__(self, n=16384, generations=1000, seed=synthetic.DEFAULT_SEED, per_launch=25, variant=0, wrap=0):
         self.n, self.gens, self.seed, self.wrap = n, generations, seed, wrap
         self.tile = lgdhip.tile(steps_per_launch=per_launch, variant=variant)
         self.per_launch = per_launch
@@ -845,7 +845,7 @@ def main():
                     help="one workload (default: life, plus the secondary Jacobi and LBM entries)")
     ap.add_argument("--size", type=int, default=0, help="override the grid edge length")
     ap.add_argument("--iters", type=int, default=0, help="override generations / steps per run")
-    ap.add_argument("--per-launch", type=int, default=31, help="life: generations per launch")
+    ap.add_argument("--per-launch", type=int, default=25, help="life: generations per launch")
     ap.add_argument("--variant", type=int, default=-1, help="kernel variant id (-1: tuned default, 0: library default)")
     ap.add_argument("--by", type=int, default=0, help="jacobi/lbm: rows per work-group (0: default)")
     ap.add_argument("--bx", type=int, default=0, help="lbm: work-group width 64 or 256 (0: default)")
@@ -886,7 +886,7 @@ def main():
     if args.iters:
         kw["generations" if args.workload == "life" else "steps"] = args.iters
     if args.workload == "life":
-        kw.update(per_launch=args.per_launch, variant=7 if args.variant < 0 else args.variant, wrap=args.wrap)
+        kw.update(per_launch=args.per_launch, variant=max(0, args.variant), wrap=args.wrap)
     flags = (lgdhip.TILE_NO_XCD_SWIZZLE if args.no_xcd_swizzle else 0) | \
         (lgdhip.TILE_XCD_SWIZZLE if args.xcd_swizzle else 0) | (lgdhip.TILE_XCD_ROWS if args.xcd_rows else 0)
     if args.workload == "jacobi":

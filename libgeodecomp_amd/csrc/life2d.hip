@@ -17,6 +17,8 @@
 //    is packed once before and unpacked once after a run.
 #include "lgdhip_internal.h"
 
+#include <algorithm>
+
 namespace {
 
 // ---------------------------------------------------------------------------
@@ -59,12 +61,18 @@ __global__ __launch_bounds__(64 * BY) void life_u8_swar(const uint8_t *__restric
 }
 
 // ---------------------------------------------------------------------------
-// packing
+// packing: one word per thread, work-groups of 256 threads folded over as many
+// rows as keep them full (pack_block), so narrow grids run few work-groups
 // ---------------------------------------------------------------------------
+dim3 pack_block(int nw) {
+    unsigned x = 256;
+    while (x > 1 && x / 2 >= (unsigned)nw) x /= 2;
+    return dim3(x, 256 / x);
+}
 __global__ void life_pack(const uint8_t *__restrict__ grid, uint32_t *__restrict__ packed, int nx, int ny,
                           int nw, int64_t sx, int64_t origin) {
     const int w = blockIdx.x * blockDim.x + threadIdx.x;
-    const int y = blockIdx.y;
+    const int y = blockIdx.y * blockDim.y + threadIdx.y;
     if (w >= nw || y >= ny) return;
     const uint8_t *row = grid + origin + (int64_t)y * sx;
     const int x0 = 32 * w;
@@ -90,7 +98,7 @@ __global__ void life_pack(const uint8_t *__restrict__ grid, uint32_t *__restrict
 __global__ void life_unpack(const uint32_t *__restrict__ packed, uint8_t *__restrict__ grid, int nx, int ny,
                             int nw, int64_t sx, int64_t origin) {
     const int w = blockIdx.x * blockDim.x + threadIdx.x;
-    const int y = blockIdx.y;
+    const int y = blockIdx.y * blockDim.y + threadIdx.y;
     if (w >= nw || y >= ny) return;
     uint8_t *row = grid + origin + (int64_t)y * sx;
     const uint32_t bits = packed[(int64_t)y * nw + w];
@@ -264,43 +272,66 @@ __global__ __launch_bounds__(kLanes *kWavesPerBlock) void life_packed_tb(
 }
 
 // ---------------------------------------------------------------------------
-// stacked waves: NW waves of one work-group hold NW*R consecutive rows of the
-// same 64 word columns and hand their boundary rows to each other through
-// LDS every generation, so only the work-group's top and bottom K rows are
-// redundant halo (instead of 2K rows per wave).
+// stacked waves: NW waves of one work-group hold NW*R consecutive rows of 64
+// word columns and hand their boundary rows to each other through LDS every
+// generation, so only the work-group's top and bottom K rows are redundant
+// halo (instead of 2K rows per wave).
+//
+// The grid is cut into bands of NW*R - 2K output rows, and the bands' word
+// columns are laid end to end: each band contributes a span of nw + 1 columns
+// (one column of outside cells, then its nw words; nw + 2 on a wrapped x axis:
+// the periodic image at both ends), and work-group t takes the 64 columns
+// 62t - 1 .. 62t + 62 of that line, so a lane's band and column are its own.
+// A row of words that is no multiple of 62 then costs a work-group only where
+// the whole line ends (16384 cells: 512 words, 8.3 work-groups per band
+// instead of 9; 1000 cells: 32 words, one half instead of one).  The column of
+// outside cells keeps the neighbouring bands apart on an unwrapped axis; on a
+// wrapped one an image's outer neighbour is another band's cell, whose
+// influence has not crossed the image's 32 cells after 32 generations.
 // ---------------------------------------------------------------------------
 template <int R, int NW, bool WRAP>
 __global__ __launch_bounds__(kLanes *NW) void life_packed_stacked(const uint32_t *__restrict__ src,
                                                                   uint32_t *__restrict__ dst, int nw, int ny,
                                                                   uint32_t last_mask, uint32_t edge, int gens,
-                                                                  int halo_rows, int wrap_mask) {
+                                                                  int halo_rows, int span, int wrap_mask) {
     const int wrap = WRAP ? wrap_mask : 0;
     // [buffer][wave][0: first row, 1: last row][lane]
     __shared__ uint32_t xchg[2][NW][2][kLanes];
     const int lane = threadIdx.x & (kLanes - 1);
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / kLanes));
-    const int col = (int)blockIdx.x * kOutCols + lane - 1;
-    const int block_row0 = (int)blockIdx.y * (NW * R - 2 * halo_rows) - halo_rows;
-    if (block_row0 + halo_rows >= ny) return;  // block-uniform: no wave is left at a barrier
-    const int row0 = block_row0 + wave * R;
+    const int line = (int)blockIdx.x * kOutCols + lane - 1;
+    const int band = line < 0 ? 0 : line / span;
+    const int col = line < 0 ? -1 : line % span - 1;
+    const int valid = NW * R - 2 * halo_rows;
+    // bands past the grid (the end of the line) hold outside rows only
+    const int64_t band_row = (int64_t)band * valid;
+    const int row0 = (int)(band_row < ny ? band_row : (int64_t)ny) - halo_rows + wave * R;
 
     const bool col_in = col >= 0 && col < nw;
     const uint32_t cmask = (wrap & 1) ? 0xFFFFFFFFu : (col_in ? (col == nw - 1 ? last_mask : 0xFFFFFFFFu) : 0u);
-    const bool rows_edge = !(wrap & 2) && (row0 < 0 || row0 + R > ny);
-    const bool cols_edge = !(wrap & 1) && (blockIdx.x == 0 || (int)(blockIdx.x + 1) * kOutCols + 1 > nw - 1);
+    // does this wave hold cells outside an unwrapped grid boundary?
+    const bool rows_edge = !(wrap & 2) && __any(row0 < 0 || row0 + R > ny);
+    const bool cols_edge = !(wrap & 1) && __any(cmask != 0xFFFFFFFFu);
+    // register rows [ilo, ihi) lie inside the grid
     int ilo = row0 < 0 ? (-row0 < R ? -row0 : R) : 0;
     int ihi = ny - row0 < R ? (ny - row0 > 0 ? ny - row0 : 0) : R;
 
     const int colc = packed_col(col, nw, wrap);
     uint32_t v[R];
+    if (rows_edge || (wrap & 2)) {
 #pragma unroll
-    for (int i = 0; i < R; ++i) {
-        const uint32_t x = src[(int64_t)packed_row(row0 + i, ny, wrap) * nw + colc];
-        v[i] = ((wrap & 2) || (i >= ilo && i < ihi)) ? ((x & cmask) | (edge & ~cmask)) : edge;
+        for (int i = 0; i < R; ++i) {
+            const uint32_t x = src[(int64_t)packed_row(row0 + i, ny, wrap) * nw + colc];
+            v[i] = ((wrap & 2) || (i >= ilo && i < ihi)) ? ((x & cmask) | (edge & ~cmask)) : edge;
+        }
+    } else {
+        const uint32_t *p = src + (int64_t)row0 * nw + colc;
+#pragma unroll
+        for (int i = 0; i < R; ++i, p += nw) v[i] = (*p & cmask) | (edge & ~cmask);
     }
 
     for (int g = 0; g < gens; ++g) {
-        asm volatile("" : "+s"(ilo), "+s"(ihi));
+        asm volatile("" : "+v"(ilo), "+v"(ihi));
         const int buf = g & 1;
         xchg[buf][wave][0][lane] = v[0];
         xchg[buf][wave][1][lane] = v[R - 1];
@@ -314,10 +345,10 @@ __global__ __launch_bounds__(kLanes *NW) void life_packed_stacked(const uint32_t
         // The block's top wave has no neighbour above, so after generation g
         // its rows 0 .. g hold don't-care values (halo rows, read only by each
         // other and never stored); likewise rows R-1-g .. R-1 of the bottom
-        // wave.  Those rows skip the rule (8 of the 14 operations per row:
-        // about 7% of the block's work over a launch; the row sums stay, as
-        // skipping them too costs every row a register move).  The bounds
-        // are wave-uniform, so a skipped row is a scalar branch.
+        // wave.  Those rows skip the rule (8 of the 14 operations per row;
+        // the row sums stay, as skipping them too costs every row a register
+        // move).  The bounds are wave-uniform, so a skipped row is a scalar
+        // branch.
         auto generation = [&](int lo, int hi) {
             uint32_t sa, ca, sb, cb;
             row_sums<true>(above, sa, ca);
@@ -345,26 +376,25 @@ __global__ __launch_bounds__(kLanes *NW) void life_packed_stacked(const uint32_t
         }
     }
 
-    if (lane == 0 || lane == kLanes - 1 || !col_in) return;
-    // rows of this wave inside [block_row0 + K, block_row0 + NW*R - K) and the grid
-    const int lo = block_row0 + halo_rows - row0;
-    const int hi = block_row0 + NW * R - halo_rows - row0;
+    if (lane == 0 || lane == kLanes - 1 || !col_in || band_row >= ny) return;
+    // rows of this wave inside [band_row, band_row + valid) and the grid
+    const int lo = halo_rows - wave * R;
+    const int hi = lo + valid;
     const int iend = ihi < hi ? ihi : hi;
+    uint32_t *q = dst + (int64_t)row0 * nw + col;
 #pragma unroll
-    for (int i = 0; i < R; ++i) {
-        if (i >= lo && i < iend) dst[(int64_t)(row0 + i) * nw + col] = v[i];
+    for (int i = 0; i < R; ++i, q += nw) {
+        if (i >= lo && i < iend) *q = v[i];
     }
 }
 
-// variant ids of lgdhip_tile::variant for the packed kernel (0 = default)
+// variant ids of lgdhip_tile::variant for the packed kernel
+//   0: stacked waves, rows and generations per launch by life_plan
 //   1: independent waves, 128 register rows      2: same with ds_bpermute
 //   3: independent waves, 64 register rows       4: same with ds_bpermute
 //   5: 4 stacked waves x 64 rows                 6: 8 stacked waves x 64 rows
 //   7: 8 stacked waves x 32 rows                 8: 16 stacked waves x 32 rows
 constexpr int kNumVariants = 8;
-// tuned on MI355X for 16384^2 (8 waves x 32 rows, 31 generations per launch:
-// 4.9 ms for 1000 generations); see the variant sweep in the profiles
-constexpr int kDefaultVariant = 7;
 constexpr int kDefaultPerLaunch = 31;
 
 // register rows one work-group column holds for a variant
@@ -377,6 +407,58 @@ int rows_per_group(int variant) {
     case 7: return 8 * 32;
     default: return 16 * 32;
     }
+}
+
+// word columns of one band on the line of bands, and work-groups of a launch
+int64_t life_span(int nw, int wrap) { return (int64_t)nw + ((wrap & 1) ? 2 : 1); }
+int64_t life_groups(int nw, int ny, int wrap, int rows, int halo_rows) {
+    const int64_t valid = rows - 2 * halo_rows;
+    const int64_t columns = (ny + valid - 1) / valid * life_span(nw, wrap);
+    return (columns + kOutCols - 1) / kOutCols;
+}
+
+// Stacked waves, rows per wave and generations per launch of the default
+// variant, by the modelled time of the whole call: tall work-groups and 20-31
+// generations where the grid fills the chip's SIMDs evenly (16384^2: 16 x 20
+// rows, two work-groups on every CU, 4.13 us per generation against 4.59 with
+// 8 x 32 rows, whose 704 work-groups leave a quarter of the CUs a third idle),
+// 8 x 4 rows and 14 generations where it does not fill it at all (1000 x 777:
+// 0.67 us per generation on 104 CUs against 2.6 on 5).
+struct LifeShape {
+    int waves, rows, gens;
+};
+constexpr struct {
+    int waves, rows;
+} kLifeShapes[] = {{8, 4},  {8, 8},  {8, 12}, {8, 16},  {8, 24},  {8, 32},  {8, 40},  {8, 48}, {8, 64}, {8, 80},
+                   {16, 4}, {16, 6}, {16, 8}, {16, 12}, {16, 16}, {16, 20}, {16, 24}, {16, 32}};
+LifeShape life_plan(int nw, int ny, int wrap, int steps, int per_launch) {
+    LifeShape best{8, 32, per_launch > 0 ? per_launch : kDefaultPerLaunch};
+    double best_us = 1e300;
+    // Measured on MI355X (124 generations, every shape x 8-32 generations per
+    // launch on 256 x 200 .. 16384^2 grids; the model's choice is within 3% of
+    // the best on each).  A launch's fixed cost and its one pass over the state:
+    const double launch_us = 2.0 + 8.0 * nw * ny / 5.5e6;
+    for (const auto &shape : kLifeShapes) {
+        const int rows = shape.waves * shape.rows;
+        for (int gens = per_launch > 0 ? per_launch : 4; gens <= 32 && 2 * gens < rows; ++gens) {
+            const int64_t groups = life_groups(nw, ny, wrap, rows, gens);
+            if (groups <= INT32_MAX / kOutCols - 2) {
+                // A generation costs its exchange and barrier (0.25 us) and
+                // the rows of the busiest SIMD's waves: 14 operations of 4
+                // cycles each once there are many, but at two waves 162 cycles
+                // and at four 250, the waves' own latency.
+                const double waves = (double)((groups + lgdhip::kCUs - 1) / lgdhip::kCUs) * shape.waves / 4;
+                const double row_us = std::max(waves < 4 ? 0.0675 : 0.105, waves * (14 * 4 / 2400.0));
+                const double us = ((steps + gens - 1) / gens) * launch_us + steps * (0.25 + shape.rows * row_us);
+                if (us < best_us) {
+                    best_us = us;
+                    best = LifeShape{shape.waves, shape.rows, gens};
+                }
+            }
+            if (per_launch > 0) break;
+        }
+    }
+    return best;
 }
 
 template <int R>
@@ -401,26 +483,35 @@ void launch_rows(const uint32_t *src, uint32_t *dst, int nw, int ny, uint32_t la
 template <int R, int NW>
 void launch_stacked(const uint32_t *src, uint32_t *dst, int nw, int ny, uint32_t last_mask, uint32_t edge, int gens,
                     int halo_rows, int wrap, hipStream_t s) {
-    const int valid = NW * R - 2 * halo_rows;
-    dim3 grid((unsigned)((nw + kOutCols - 1) / kOutCols), (unsigned)((ny + valid - 1) / valid));
+    const unsigned groups = (unsigned)life_groups(nw, ny, wrap, NW * R, halo_rows);
+    const int span = (int)life_span(nw, wrap);
     if (wrap)
-        life_packed_stacked<R, NW, true><<<grid, kLanes * NW, 0, s>>>(src, dst, nw, ny, last_mask, edge, gens,
-                                                                      halo_rows, wrap);
+        life_packed_stacked<R, NW, true><<<groups, kLanes * NW, 0, s>>>(src, dst, nw, ny, last_mask, edge, gens,
+                                                                        halo_rows, span, wrap);
     else
-        life_packed_stacked<R, NW, false><<<grid, kLanes * NW, 0, s>>>(src, dst, nw, ny, last_mask, edge, gens,
-                                                                       halo_rows, 0);
+        life_packed_stacked<R, NW, false><<<groups, kLanes * NW, 0, s>>>(src, dst, nw, ny, last_mask, edge, gens,
+                                                                         halo_rows, span, 0);
 }
 
 int packed_launch(const uint32_t *src, uint32_t *dst, int nw, int ny, uint32_t last_mask, uint32_t edge,
-                  int gens, int halo_rows, int variant, int wrap, hipStream_t s) {
+                  int gens, int halo_rows, int variant, LifeShape shape, int wrap, hipStream_t s) {
     switch (variant) {
     case 1: case 2: launch_rows<128>(src, dst, nw, ny, last_mask, edge, gens, halo_rows, variant == 1, wrap, s); break;
     case 3: case 4: launch_rows<64>(src, dst, nw, ny, last_mask, edge, gens, halo_rows, variant == 3, wrap, s); break;
     case 5: launch_stacked<64, 4>(src, dst, nw, ny, last_mask, edge, gens, halo_rows, wrap, s); break;
-    case 6: launch_stacked<64, 8>(src, dst, nw, ny, last_mask, edge, gens, halo_rows, wrap, s); break;
-    case 7: launch_stacked<32, 8>(src, dst, nw, ny, last_mask, edge, gens, halo_rows, wrap, s); break;
-    default: launch_stacked<32, 16>(src, dst, nw, ny, last_mask, edge, gens, halo_rows, wrap, s); break;
+    case 6: shape = LifeShape{8, 64, halo_rows}; break;
+    case 7: shape = LifeShape{8, 32, halo_rows}; break;
+    case 8: shape = LifeShape{16, 32, halo_rows}; break;
+    default: break;
     }
+#define LGD_LIFE_CASE(NW, R)                                                                                    \
+    if ((variant == 0 || variant >= 6) && shape.waves == NW && shape.rows == R)                                 \
+        launch_stacked<R, NW>(src, dst, nw, ny, last_mask, edge, gens, halo_rows, wrap, s);
+    LGD_LIFE_CASE(8, 4) LGD_LIFE_CASE(8, 8) LGD_LIFE_CASE(8, 12) LGD_LIFE_CASE(8, 16) LGD_LIFE_CASE(8, 24)
+    LGD_LIFE_CASE(8, 32) LGD_LIFE_CASE(8, 40) LGD_LIFE_CASE(8, 48) LGD_LIFE_CASE(8, 64) LGD_LIFE_CASE(8, 80)
+    LGD_LIFE_CASE(16, 4) LGD_LIFE_CASE(16, 6) LGD_LIFE_CASE(16, 8) LGD_LIFE_CASE(16, 12) LGD_LIFE_CASE(16, 16)
+    LGD_LIFE_CASE(16, 20) LGD_LIFE_CASE(16, 24) LGD_LIFE_CASE(16, 32)
+#undef LGD_LIFE_CASE
     LGD_LAUNCHED("life_packed_tb");
     return 0;
 }
@@ -447,18 +538,17 @@ int packed_run(uint32_t *pa, uint32_t *pb, const lgdhip_grid *g, int edge_alive,
     LGD_REQUIRE(pa && pb && pa != pb, "need two distinct device buffers");
     LGD_REQUIRE(steps >= 0, "steps must be >= 0");
     LGD_REQUIRE(edge_alive == 0 || edge_alive == 1, "edge_alive must be 0 or 1");
-    int per_launch = kDefaultPerLaunch;
-    int variant = kDefaultVariant;
+    int per_launch = 0, variant = 0;
     if (tile) {
         if (tile->steps_per_launch > 0) per_launch = tile->steps_per_launch;
-        if (tile->variant != 0) variant = tile->variant;
+        variant = tile->variant;
     }
-    if (variant < 1 || variant > kNumVariants) return lgdhip::set_error(LGDHIP_ERR_UNSUPPORTED, "unknown life variant");
-    const int rows = rows_per_group(variant);
+    if (variant < 0 || variant > kNumVariants) return lgdhip::set_error(LGDHIP_ERR_UNSUPPORTED, "unknown life variant");
+    if (variant != 0 && per_launch == 0) per_launch = kDefaultPerLaunch;
     // a lane's neighbour word covers 32 cells, so at most 32 generations may
     // run before the halo lanes' garbage reaches an output column; the
     // register rows must keep at least one valid row per band
-    if (per_launch < 1 || per_launch > 32 || 2 * per_launch >= rows)
+    if (per_launch < 0 || per_launch > 32 || (variant != 0 && 2 * per_launch >= rows_per_group(variant)))
         return lgdhip::set_error(LGDHIP_ERR_UNSUPPORTED,
                                  "steps_per_launch must be in [1, 32] and below half the register rows");
     const int nw = (int)((g->nx + 31) / 32);
@@ -466,10 +556,15 @@ int packed_run(uint32_t *pa, uint32_t *pb, const lgdhip_grid *g, int edge_alive,
     const uint32_t last_mask = rem >= 32 ? 0xFFFFFFFFu : ((1u << rem) - 1u);
     const uint32_t edge = edge_alive ? 0xFFFFFFFFu : 0u;
     hipStream_t s = lgdhip::as_stream(stream);
+    LifeShape shape{0, 0, per_launch};
+    if (variant == 0) {
+        shape = life_plan(nw, (int)g->ny, wrap, steps, per_launch);
+        per_launch = shape.gens;
+    }
     uint32_t *cur = pa, *nxt = pb;
     for (int done = 0; done < steps;) {
         const int gens = (steps - done < per_launch) ? (steps - done) : per_launch;
-        rc = packed_launch(cur, nxt, nw, (int)g->ny, last_mask, edge, gens, per_launch, variant, wrap, s);
+        rc = packed_launch(cur, nxt, nw, (int)g->ny, last_mask, edge, gens, per_launch, variant, shape, wrap, s);
         if (rc) return rc;
         uint32_t *tmp = cur;
         cur = nxt;
@@ -518,8 +613,8 @@ int lgdhip_life2d_pack(const uint8_t *grid, const lgdhip_grid *g, uint32_t *pack
     LGD_REQUIRE(grid && packed, "NULL pointer");
     const int nw = (int)((g->nx + 31) / 32);
     LGD_REQUIRE(g->ny <= 65535, "ny must be <= 65535 (one grid row per launch row)");
-    dim3 grd(lgdhip::ceil_div(nw, 256), (unsigned)g->ny);
-    life_pack<<<grd, 256, 0, lgdhip::as_stream(stream)>>>(grid, packed, (int)g->nx, (int)g->ny, nw, g->sx,
+    const dim3 block = pack_block(nw), grd(lgdhip::ceil_div(nw, block.x), lgdhip::ceil_div(g->ny, block.y));
+    life_pack<<<grd, block, 0, lgdhip::as_stream(stream)>>>(grid, packed, (int)g->nx, (int)g->ny, nw, g->sx,
                                                          lgdhip::origin_index(*g));
     LGD_LAUNCHED("life_pack");
     return 0;
@@ -531,8 +626,8 @@ int lgdhip_life2d_unpack(const uint32_t *packed, const lgdhip_grid *g, uint8_t *
     LGD_REQUIRE(grid && packed, "NULL pointer");
     LGD_REQUIRE(g->ny <= 65535, "ny must be <= 65535 (one grid row per launch row)");
     const int nw = (int)((g->nx + 31) / 32);
-    dim3 grd(lgdhip::ceil_div(nw, 256), (unsigned)g->ny);
-    life_unpack<<<grd, 256, 0, lgdhip::as_stream(stream)>>>(packed, grid, (int)g->nx, (int)g->ny, nw, g->sx,
+    const dim3 block = pack_block(nw), grd(lgdhip::ceil_div(nw, block.x), lgdhip::ceil_div(g->ny, block.y));
+    life_unpack<<<grd, block, 0, lgdhip::as_stream(stream)>>>(packed, grid, (int)g->nx, (int)g->ny, nw, g->sx,
                                                            lgdhip::origin_index(*g));
     LGD_LAUNCHED("life_unpack");
     return 0;

@@ -275,6 +275,26 @@ def test_life_packed_periodic_bit_exact(hip, oracle, shape):
                 assert np.array_equal(out, exp), (wrap, edge, variant, per_launch)
 
 
+@pytest.mark.parametrize("nx,ny,steps,per_launch,wrap", [
+    (1000, 777, 100, 0, 0),     # low work-groups, two bands per wave
+    (1984, 40, 33, 0, 3),       # 62 words a row: a span of 64 columns, one band
+    (1999, 2051, 60, 0, 2),     # ragged last word, bands cut at every column
+    (4096, 4100, 45, 0, 0),     # 16 stacked waves, low bands
+    (8190, 8193, 27, 0, 0),     # taller ones, the last band almost empty
+    (8192, 8193, 27, 27, 1),    # images of the wrapped x axis inside a work-group
+    (16384, 16500, 26, 25, 0),  # the tallest work-groups
+])
+def test_life_packed_default_shapes(hip, oracle, nx, ny, steps, per_launch, wrap):
+    """The default variant's work-group heights and launch depths on grids
+    from a fraction of the chip to several rounds of it, both edge states."""
+    say("life default", nx, ny, "steps", steps, "wrap", wrap)
+    g0 = synthetic.life_initial(nx, ny, seed=nx + 11 * ny)
+    edge = (nx + ny) % 2
+    t = hip.tile(steps_per_launch=per_launch) if per_launch else None
+    exp = oracle.life2d(g0, steps, edge=edge, threads=16, wrap=wrap)
+    assert np.array_equal(gpu_life_packed_periodic(hip, g0, steps, wrap, edge=edge, tile=t), exp)
+
+
 def test_life_glider_on_gpu(hip):
     glider = [(11, 10), (12, 11), (10, 12), (11, 12), (12, 12)]
     g = place(glider, (300, 70))
