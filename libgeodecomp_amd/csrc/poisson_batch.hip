@@ -50,6 +50,16 @@ struct Tile {
     int32_t p, x0, y0, z0;
 };
 
+// A solve's state of one problem, kept on the device so that the decisions
+// between chunks (refresh, done) need no host round trip.  Kernels given the
+// states skip the problems they do not concern: sweeps the done ones, the
+// FP64 refresh all but the ones marked `refresh`.
+struct SolveState {
+    double ref, outer, inner;
+    int64_t sweeps;
+    int32_t outer_iters, done, refresh, pad;
+};
+
 __device__ __forceinline__ double block_sum(double v, double *lds) {
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
@@ -68,9 +78,11 @@ __global__ __launch_bounds__(kThreads) void poisson_residual_f64(const double *_
                                                                  const float *__restrict__ f,
                                                                  float *__restrict__ r32, const Tile *__restrict__ tiles,
                                                                  const ProblemDev *__restrict__ probs,
-                                                                 double *__restrict__ partial) {
+                                                                 double *__restrict__ partial,
+                                                                 const SolveState *__restrict__ state) {
     __shared__ double lds[kThreads / 64];
     const Tile t = tiles[blockIdx.x];
+    if (state && !state[t.p].refresh) return;
     const ProblemDev P = probs[t.p];
     const int n = P.n;
     const int x = t.x0 + (int)(threadIdx.x % kTX);
@@ -108,9 +120,11 @@ __global__ __launch_bounds__(kThreads) void poisson_sweep_f32(const float *__res
                                                               const float *__restrict__ r,
                                                               const Tile *__restrict__ tiles,
                                                               const ProblemDev *__restrict__ probs,
-                                                              double *__restrict__ partial, float omega) {
+                                                              double *__restrict__ partial, float omega,
+                                                              const SolveState *__restrict__ state) {
     __shared__ double lds[kThreads / 64];
     const Tile t = tiles[blockIdx.x];
+    if (state && state[t.p].done) return;
     const ProblemDev P = probs[t.p];
     const int n = P.n;
     const int x = t.x0 + (int)(threadIdx.x % kTX);
@@ -177,7 +191,8 @@ __global__ __launch_bounds__(64 * TY) void poisson_sweep_tb(const float *__restr
                                                             const Tile *__restrict__ tiles,
                                                             const ProblemDev *__restrict__ probs,
                                                             double *__restrict__ partial, int zchunk,
-                                                            unsigned ntiles, unsigned per, float omega) {
+                                                            unsigned ntiles, unsigned per, float omega,
+                                                            const SolveState *__restrict__ state) {
     constexpr int PF = 3;  // e planes in flight
     static_assert(K + 2 <= 6, "r ring of 6 slots holds planes p-K .. p+1");
     __shared__ float lds[2][K][TY][64];
@@ -187,6 +202,7 @@ __global__ __launch_bounds__(64 * TY) void poisson_sweep_tb(const float *__restr
     const unsigned tid = lgdhip::xcd_tile(blockIdx.x, per, true);
     if (tid >= ntiles) return;  // whole work-group, before any barrier
     const Tile t = tiles[tid];
+    if (state && state[t.p].done) return;
     const ProblemDev P = probs[t.p];
     const int n = P.n;
     const int tx = threadIdx.x, ty = threadIdx.y;
@@ -315,7 +331,8 @@ __global__ __launch_bounds__(64 * TY) void poisson_sweep_tb2(const float *__rest
                                                              const Tile *__restrict__ tiles,
                                                              const ProblemDev *__restrict__ probs,
                                                              double *__restrict__ partial, int zchunk,
-                                                             unsigned ntiles, unsigned per, float omega) {
+                                                             unsigned ntiles, unsigned per, float omega,
+                                                             const SolveState *__restrict__ state) {
     constexpr int PF = 3;
     constexpr int CY = R * TY;
     static_assert(K + 2 <= 6, "r ring of 6 slots holds planes p-K .. p+1");
@@ -325,6 +342,7 @@ __global__ __launch_bounds__(64 * TY) void poisson_sweep_tb2(const float *__rest
     const unsigned tid = lgdhip::xcd_tile(blockIdx.x, per, true);
     if (tid >= ntiles) return;  // whole work-group, before any barrier
     const Tile t = tiles[tid];
+    if (state && state[t.p].done) return;
     const ProblemDev P = probs[t.p];
     const int n = P.n;
     const int tx = threadIdx.x, ty = threadIdx.y;
@@ -462,11 +480,14 @@ __global__ __launch_bounds__(64 * TY) void poisson_sweep_tb2(const float *__rest
     }
 }
 
-// u += e over the interior and reset both correction buffers to zero
+// u += e over the interior and reset both correction buffers to zero, for the
+// problems marked `refresh`
 __global__ __launch_bounds__(kThreads) void poisson_update_f64(double *__restrict__ u, float *e, float *eother,
                                                                const Tile *__restrict__ tiles,
-                                                               const ProblemDev *__restrict__ probs) {
+                                                               const ProblemDev *__restrict__ probs,
+                                                               const SolveState *__restrict__ state) {
     const Tile t = tiles[blockIdx.x];
+    if (!state[t.p].refresh) return;
     const ProblemDev P = probs[t.p];
     const int n = P.n;
     const int x = t.x0 + (int)(threadIdx.x % kTX);
@@ -514,20 +535,61 @@ __global__ __launch_bounds__(kThreads) void poisson_sweep_f64(const double *__re
     }
 }
 
-// norms[k] = sum of partial over the tiles [begin[k], end[k])  (fixed order)
-__global__ __launch_bounds__(256) void poisson_reduce(const double *__restrict__ partial, const int *__restrict__ begin,
-                                                      const int *__restrict__ end, double *__restrict__ norms) {
+// sum of partial over [begin, end) by 256 threads in a fixed order, valid in
+// thread 0
+__device__ __forceinline__ double reduce_partials(const double *__restrict__ partial, int begin, int end) {
     __shared__ double lds[256];
-    const int k = blockIdx.x;
     double s = 0.0;
-    for (int i = begin[k] + (int)threadIdx.x; i < end[k]; i += 256) s += partial[i];
+    for (int i = begin + (int)threadIdx.x; i < end; i += 256) s += partial[i];
     lds[threadIdx.x] = s;
     __syncthreads();
     for (int w = 128; w > 0; w >>= 1) {
         if ((int)threadIdx.x < w) lds[threadIdx.x] += lds[threadIdx.x + w];
         __syncthreads();
     }
-    if (threadIdx.x == 0) norms[k] = lds[0];
+    return lds[0];
+}
+
+// norms[k] = sum of partial over the tiles [begin[k], end[k])
+__global__ __launch_bounds__(256) void poisson_reduce(const double *__restrict__ partial, const int *__restrict__ begin,
+                                                      const int *__restrict__ end, double *__restrict__ norms) {
+    const double s = reduce_partials(partial, begin[blockIdx.x], end[blockIdx.x]);
+    if (threadIdx.x == 0) norms[blockIdx.x] = s;
+}
+
+// After a chunk of `sweeps` sweeps: the inner residual norm of each problem of
+// the tile list (work-group k the problem of tiles [begin[k], end[k])), and
+// whether its correction has converged far enough for an FP64 refresh (by
+// theta, or to half the tolerance) or its sweeps are used up.
+__global__ __launch_bounds__(256) void poisson_decide_inner(const double *__restrict__ partial,
+                                                            const Tile *__restrict__ tiles,
+                                                            const int *__restrict__ begin,
+                                                            const int *__restrict__ end, SolveState *state, int sweeps,
+                                                            double theta, double rel_tol, int64_t max_sweeps) {
+    SolveState *q = state + tiles[begin[blockIdx.x]].p;
+    if (q->done) return;  // its sweeps were skipped; refresh is 0
+    const double s = reduce_partials(partial, begin[blockIdx.x], end[blockIdx.x]);
+    if (threadIdx.x != 0) return;
+    q->sweeps += sweeps;
+    q->inner = sqrt(s);
+    q->refresh = q->inner <= theta * q->outer || q->inner <= 0.5 * rel_tol * q->ref || q->sweeps >= max_sweeps;
+}
+
+// After the FP64 refresh: the outer residual norm of the refreshed problems,
+// and whether they are done.
+__global__ __launch_bounds__(256) void poisson_decide_outer(const double *__restrict__ partial,
+                                                            const Tile *__restrict__ tiles,
+                                                            const int *__restrict__ begin,
+                                                            const int *__restrict__ end, SolveState *state,
+                                                            double rel_tol, int64_t max_sweeps) {
+    SolveState *q = state + tiles[begin[blockIdx.x]].p;
+    if (!q->refresh) return;
+    const double s = reduce_partials(partial, begin[blockIdx.x], end[blockIdx.x]);
+    if (threadIdx.x != 0) return;
+    q->outer = sqrt(s);
+    q->outer_iters += 1;
+    q->refresh = 0;
+    q->done = q->outer <= rel_tol * q->ref || q->sweeps >= max_sweeps;
 }
 
 // faces into the halo of u (edges and corners are never read)
@@ -658,6 +720,7 @@ struct Workspace {
     double *faces;
     Tile *tb_tiles;  // temporal-blocking sweep tiles of the active set
     int *tb_begin, *tb_end;
+    SolveState *state;
     size_t bytes;
 };
 
@@ -685,6 +748,7 @@ Workspace carve(void *base, int64_t pool, int64_t ntiles, int64_t ntb, int count
     w.tb_tiles = (Tile *)take(ntb * sizeof(Tile));
     w.tb_begin = (int *)take((size_t)count * 4);
     w.tb_end = (int *)take((size_t)count * 4);
+    w.state = (SolveState *)take((size_t)count * sizeof(SolveState));
     w.bytes = off;
     return w;
 }
@@ -741,36 +805,39 @@ int upload_tb_set(const Workspace &w, const lgdhip_poisson_problem *probs, const
 
 template <bool DAMPED>
 void launch_tb_kind(TbShape sh, const float *a, float *b, const float *r, const Workspace &w, int64_t ntiles,
-                    int zchunk, double *partial, float omega, hipStream_t s) {
+                    int zchunk, double *partial, float omega, const SolveState *state, hipStream_t s) {
     const unsigned nt = (unsigned)ntiles, per = lgdhip::xcd_per(nt), groups = lgdhip::xcd_groups(nt);
     if (sh.rows == 3)
         poisson_sweep_tb2<4, 16, 3, DAMPED><<<groups, dim3(64, 16), 0, s>>>(a, b, r, w.tb_tiles, w.probs, partial,
-                                                                            zchunk, nt, per, omega);
+                                                                            zchunk, nt, per, omega, state);
     else if (sh.rows == 2 && sh.ty == 16)
         poisson_sweep_tb2<4, 16, 2, DAMPED><<<groups, dim3(64, 16), 0, s>>>(a, b, r, w.tb_tiles, w.probs, partial,
-                                                                            zchunk, nt, per, omega);
+                                                                            zchunk, nt, per, omega, state);
     else if (sh.rows == 2)
         poisson_sweep_tb2<4, 8, 2, DAMPED><<<groups, dim3(64, 8), 0, s>>>(a, b, r, w.tb_tiles, w.probs, partial, zchunk,
-                                                                          nt, per, omega);
+                                                                          nt, per, omega, state);
     else if (sh.k == 2)
         poisson_sweep_tb<2, 16, DAMPED><<<groups, dim3(64, 16), 0, s>>>(a, b, r, w.tb_tiles, w.probs, partial, zchunk, nt,
-                                                                        per, omega);
+                                                                        per, omega, state);
     else
         poisson_sweep_tb<4, 16, DAMPED><<<groups, dim3(64, 16), 0, s>>>(a, b, r, w.tb_tiles, w.probs, partial, zchunk, nt,
-                                                                        per, omega);
+                                                                        per, omega, state);
 }
 
 // one launch of K blocked sweeps a -> b over the uploaded tile list (z
 // chunks of `zchunk` planes, as uploaded); omega > 0 runs weighted sweeps
 // e' = e + omega (J(e) - e)
 void launch_tb(TbShape sh, const float *a, float *b, const float *r, const Workspace &w, int64_t ntiles,
-               int zchunk, double *partial, hipStream_t s, float omega = 0.0f) {
+               int zchunk, double *partial, hipStream_t s, float omega = 0.0f, const SolveState *state = nullptr) {
     if (ntiles <= 0) return;
     if (omega > 0.0f)
-        launch_tb_kind<true>(sh, a, b, r, w, ntiles, zchunk, partial, omega, s);
+        launch_tb_kind<true>(sh, a, b, r, w, ntiles, zchunk, partial, omega, state, s);
     else
-        launch_tb_kind<false>(sh, a, b, r, w, ntiles, zchunk, partial, 0.0f, s);
+        launch_tb_kind<false>(sh, a, b, r, w, ntiles, zchunk, partial, 0.0f, state, s);
 }
+
+// chunks of a solve enqueued between two looks at the problems' states
+constexpr int kChunksPerLook = 4;
 
 // Uploads problem descriptors and the tile list of the problems in `set`;
 // begin/end index the tiles of set[k].
@@ -794,7 +861,7 @@ int upload_set(const Workspace &w, const lgdhip_poisson_problem *probs, const st
 int residual_norms(const double *u, const float *f, const Workspace &w, const std::vector<Tile> &tiles, int nset,
                    std::vector<double> *norms, hipStream_t s) {
     if (tiles.empty()) return 0;
-    poisson_residual_f64<<<(unsigned)tiles.size(), kThreads, 0, s>>>(u, f, w.r, w.tiles, w.probs, w.partial);
+    poisson_residual_f64<<<(unsigned)tiles.size(), kThreads, 0, s>>>(u, f, w.r, w.tiles, w.probs, w.partial, nullptr);
     LGD_LAUNCHED("poisson_residual_f64");
     poisson_reduce<<<(unsigned)nset, 256, 0, s>>>(w.partial, w.begin, w.end, w.norms);
     LGD_LAUNCHED("poisson_reduce");
@@ -839,10 +906,10 @@ int run_sweeps_in(float *ea, float *eb, const float *r, const lgdhip_poisson_pro
     for (; t < sweeps; ++t) {
         if (omega > 0.0f)
             poisson_sweep_f32<true>
-                <<<(unsigned)tiles.size(), kThreads, 0, s>>>(cur, nxt, r, w.tiles, w.probs, nullptr, omega);
+                <<<(unsigned)tiles.size(), kThreads, 0, s>>>(cur, nxt, r, w.tiles, w.probs, nullptr, omega, nullptr);
         else
             poisson_sweep_f32<false>
-                <<<(unsigned)tiles.size(), kThreads, 0, s>>>(cur, nxt, r, w.tiles, w.probs, nullptr, 1.0f);
+                <<<(unsigned)tiles.size(), kThreads, 0, s>>>(cur, nxt, r, w.tiles, w.probs, nullptr, 1.0f, nullptr);
         LGD_LAUNCHED("poisson_sweep_f32");
         std::swap(cur, nxt);
     }
@@ -1117,16 +1184,10 @@ int lgdhip_poisson_batch_solve(double *u, const float *f, const lgdhip_poisson_p
     rc = residual_norms(u, f, w, tiles, count, &rn, s);
     if (rc) return rc;
 
-    struct State {
-        double ref, outer, inner;
-        int64_t sweeps, inner_sweeps;
-        int outer_iters;
-        bool done;
-    };
-    std::vector<State> st(count);
+    std::vector<SolveState> st(count);
     for (int k = 0; k < count; ++k) {
         const double ref = (opt->reference_norms && opt->reference_norms[k] > 0) ? opt->reference_norms[k] : rn[k];
-        st[k] = State{ref, rn[k], rn[k], 0, 0, 0, rn[k] <= opt->rel_tol * ref};
+        st[k] = SolveState{ref, rn[k], rn[k], 0, 0, rn[k] <= opt->rel_tol * ref, 0, 0};
     }
 
     float *ecur = w.e0, *enxt = w.e1;  // every problem's correction lives in ecur between chunks
@@ -1161,17 +1222,15 @@ int lgdhip_poisson_batch_solve(double *u, const float *f, const lgdhip_poisson_p
             }
             for (; t < smooth; ++t) {
                 poisson_sweep_f32<true><<<(unsigned)tiles.size(), kThreads, 0, s>>>(
-                    ecur, enxt, w.r, w.tiles, w.probs, nullptr, opt->smooth_omega);
+                    ecur, enxt, w.r, w.tiles, w.probs, nullptr, opt->smooth_omega, nullptr);
                 LGD_LAUNCHED("poisson_sweep_f32");
                 std::swap(ecur, enxt);
             }
-            for (int k : active) {
-                st[k].sweeps += smooth;
-                st[k].inner_sweeps += smooth;
-            }
+            for (int k : active) st[k].sweeps += smooth;
         }
     }
-    // the chunk graph, destroyed on every return path
+    LGD_HIP(hipMemcpyAsync(w.state, st.data(), (size_t)count * sizeof(SolveState), hipMemcpyHostToDevice, s));
+    // the graph of one block of chunks, destroyed on every return path
     struct GraphExec {
         hipGraphExec_t h = nullptr;
         void reset() {
@@ -1180,7 +1239,6 @@ int lgdhip_poisson_batch_solve(double *u, const float *f, const lgdhip_poisson_p
         }
         ~GraphExec() { reset(); }
     } graph;
-    bool graph_valid = false;
     while (true) {
         active.clear();
         for (int k = 0; k < count; ++k)
@@ -1195,89 +1253,61 @@ int lgdhip_poisson_batch_solve(double *u, const float *f, const lgdhip_poisson_p
             rc = upload_tb_set(w, probs, active, sh, &ntb, &zc, s);
             if (rc) return rc;
         }
-        graph_valid = false;
-
-        bool set_changed = false;
-        while (!set_changed) {
-            // one chunk of C sweeps whose last sweep also reports the inner
-            // residual of its input iterate; the chunk leaves the correction
-            // in ecur, so the captured graph stays valid from chunk to chunk
-            auto enqueue = [&](float *a, float *b) -> int {
-                if (sh.k > 0) {
-                    for (int t = 0; t < C; t += sh.k) {
-                        launch_tb(sh, a, b, w.r, w, ntb, zc, t + sh.k == C ? w.partial : nullptr, s);
-                        std::swap(a, b);
-                    }
-                    poisson_reduce<<<(unsigned)active.size(), 256, 0, s>>>(w.partial, w.tb_begin, w.tb_end,
-                                                                           w.norms);
-                    return 0;
-                }
-                for (int t = 0; t < C; ++t) {
-                    poisson_sweep_f32<false><<<(unsigned)tiles.size(), kThreads, 0, s>>>(
-                        a, b, w.r, w.tiles, w.probs, t == C - 1 ? w.partial : nullptr, 1.0f);
+        const unsigned nt = (unsigned)tiles.size(), na = (unsigned)active.size();
+        // One chunk: C sweeps whose last one also reports the inner residual of
+        // its input iterate (the correction is back in ecur after them), then
+        // an FP64 update u += e with a fresh FP64 residual for the problems
+        // whose correction has converged far enough, which restart from e = 0.
+        // Which ones is decided on the device, so chunks follow each other
+        // without the host.
+        auto enqueue_chunk = [&]() {
+            float *a = ecur, *b = enxt;
+            if (sh.k > 0) {
+                for (int t = 0; t < C; t += sh.k) {
+                    launch_tb(sh, a, b, w.r, w, ntb, zc, t + sh.k == C ? w.partial : nullptr, s, 0.0f, w.state);
                     std::swap(a, b);
                 }
-                poisson_reduce<<<(unsigned)active.size(), 256, 0, s>>>(w.partial, w.begin, w.end, w.norms);
-                return 0;
-            };
-            if (graphs) {
-                if (!graph_valid) {
-                    graph.reset();
-                    LGD_HIP(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
-                    enqueue(ecur, enxt);
-                    hipGraph_t g = nullptr;
-                    LGD_HIP(hipStreamEndCapture(s, &g));
-                    hipError_t e = hipGraphInstantiate(&graph.h, g, nullptr, nullptr, 0);
-                    hipGraphDestroy(g);
-                    if (e != hipSuccess) {
-                        graph.h = nullptr;
-                        return lgdhip::hip_fail(e, "hipGraphInstantiate");
-                    }
-                    graph_valid = true;
+            } else {
+                for (int t = 0; t < C; ++t) {
+                    poisson_sweep_f32<false><<<nt, kThreads, 0, s>>>(a, b, w.r, w.tiles, w.probs,
+                                                                     t == C - 1 ? w.partial : nullptr, 1.0f, w.state);
+                    std::swap(a, b);
                 }
+            }
+            poisson_decide_inner<<<na, 256, 0, s>>>(w.partial, sh.k > 0 ? w.tb_tiles : w.tiles,
+                                                    sh.k > 0 ? w.tb_begin : w.begin, sh.k > 0 ? w.tb_end : w.end,
+                                                    w.state, C, theta, opt->rel_tol, opt->max_sweeps);
+            poisson_update_f64<<<nt, kThreads, 0, s>>>(u, ecur, enxt, w.tiles, w.probs, w.state);
+            poisson_residual_f64<<<nt, kThreads, 0, s>>>(u, f, w.r, w.tiles, w.probs, w.partial, w.state);
+            poisson_decide_outer<<<na, 256, 0, s>>>(w.partial, w.tiles, w.begin, w.end, w.state, opt->rel_tol,
+                                                    opt->max_sweeps);
+        };
+        // Blocks of chunks until a problem is done, then new tile lists without
+        // it.  A look at the states costs the GPU about 25 us of idling, a
+        // chunk of work-groups that find their problem done about 25 us too.
+        graph.reset();
+        for (bool changed = false; !changed;) {
+            if (graphs && !graph.h) {
+                LGD_HIP(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
+                for (int c = 0; c < kChunksPerLook; ++c) enqueue_chunk();
+                hipGraph_t g = nullptr;
+                LGD_HIP(hipStreamEndCapture(s, &g));
+                hipError_t e = hipGraphInstantiate(&graph.h, g, nullptr, nullptr, 0);
+                hipGraphDestroy(g);
+                if (e != hipSuccess) {
+                    graph.h = nullptr;
+                    return lgdhip::hip_fail(e, "hipGraphInstantiate");
+                }
+            }
+            if (graphs) {
                 LGD_HIP(hipGraphLaunch(graph.h, s));
             } else {
-                enqueue(ecur, enxt);
-                LGD_LAUNCHED("poisson_sweep_f32");
+                for (int c = 0; c < kChunksPerLook; ++c) enqueue_chunk();
+                LGD_LAUNCHED("poisson chunk");
             }
-            std::vector<double> inner(active.size());
-            LGD_HIP(hipMemcpyAsync(inner.data(), w.norms, inner.size() * 8, hipMemcpyDeviceToHost, s));
+            LGD_HIP(hipMemcpyAsync(st.data(), w.state, (size_t)count * sizeof(SolveState), hipMemcpyDeviceToHost, s));
             LGD_HIP(hipStreamSynchronize(s));
-
-            // problems whose correction has converged far enough get an
-            // FP64 update u += e and a fresh FP64 residual
-            std::vector<int> refresh;
-            for (size_t a = 0; a < active.size(); ++a) {
-                State &q = st[active[a]];
-                q.sweeps += C;
-                q.inner_sweeps += C;
-                q.inner = std::sqrt(inner[a]);
-                const bool inner_ok = q.inner <= theta * q.outer || q.inner <= 0.5 * opt->rel_tol * q.ref;
-                if (inner_ok || q.sweeps >= opt->max_sweeps) refresh.push_back(active[a]);
-            }
-            if (refresh.empty()) continue;
-            std::vector<Tile> rt;
-            rc = upload_set(w, probs, refresh, &rt, s);
-            if (rc) return rc;
-            poisson_update_f64<<<(unsigned)rt.size(), kThreads, 0, s>>>(u, ecur, enxt, w.tiles, w.probs);
-            LGD_LAUNCHED("poisson_update_f64");
-            rc = residual_norms(u, f, w, rt, (int)refresh.size(), &rn, s);
-            if (rc) return rc;
-            for (size_t a = 0; a < refresh.size(); ++a) {
-                State &q = st[refresh[a]];
-                q.outer = rn[a];
-                q.outer_iters += 1;
-                q.inner_sweeps = 0;
-                if (q.outer <= opt->rel_tol * q.ref || q.sweeps >= opt->max_sweeps) {
-                    q.done = true;
-                    set_changed = true;
-                }
-            }
-            // the refreshed problems restart their correction from zero; the
-            // tile list on the device was replaced, so re-upload the active set
-            rc = upload_set(w, probs, active, &tiles, s);
-            if (rc) return rc;
-            graph_valid = false;
+            for (int k : active) changed = changed || st[k].done;
         }
     }
     graph.reset();

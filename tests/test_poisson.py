@@ -150,10 +150,11 @@ class Batch:
         self.f.upload(f_host)
         hip.call("lgdhip_poisson_set_faces", self.u.ptr, self.probs, self.count, self.ws.ptr, self.ws_bytes, None)
 
-    def solve(self, rel_tol=1e-6, chunk=32, use_graph=1, reference=None, stream=None, sweep_variant=0, polish=0):
+    def solve(self, rel_tol=1e-6, chunk=32, use_graph=1, reference=None, stream=None, sweep_variant=0, polish=0,
+              max_sweeps=2_000_000):
         hip = self.hip
         opt = hip.lgdhip_poisson_options()
-        opt.rel_tol, opt.chunk, opt.max_sweeps, opt.use_graph = rel_tol, chunk, 2_000_000, use_graph
+        opt.rel_tol, opt.chunk, opt.max_sweeps, opt.use_graph = rel_tol, chunk, max_sweeps, use_graph
         opt.sweep_variant = sweep_variant
         opt.final_fp64_sweeps = polish
         ref = None
@@ -307,6 +308,37 @@ def test_gpu_ensemble_solve(hip, oracle, use_graph, variant):
         assert np.linalg.norm(ublock - uo) <= 1.01 * bound + 1e-12
         print(f"  n={n}: sweeps gpu {res[k].sweeps} oracle {sweeps_o}, outer {res[k].outer_iterations}, "
               f"rel residual {rk / r0:.3e}", flush=True)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("chunks,use_graph,variant", [(1, 0, 0), (3, 0, 0), (5, 1, 0), (6, 1, 1), (4, 0, 3)])
+def test_gpu_solve_stops_at_its_sweeps(hip, oracle, chunks, use_graph, variant):
+    """max_sweeps used up at every place of a block of chunks: the sweeps
+    reported and run are the chunks' (none after the stop), u the FP64
+    Jacobi iterate of that many sweeps; a problem that is solved before (it
+    starts at its solution) is left alone."""
+    problems = synthetic.poisson_ensemble(3, sizes=(12, 17, 31), seed=11 + chunks)
+    k = 8 * chunks
+    guesses = [padded(n, faces, oracle) for n, faces, _ in problems]
+    oracle.poisson_jacobi(guesses[0], problems[0][2], 1e-9, max_sweeps=100000, check=100)
+    print("poisson max sweeps", k, use_graph, variant, flush=True)
+    e = Batch(hip, problems, guesses)
+    reference = [oracle.poisson_residual_norm(padded(n, faces, oracle), f) for n, faces, f in problems]
+    stream = hip.Stream()
+    res = e.solve(1e-7, chunk=8, use_graph=use_graph, sweep_variant=variant, max_sweeps=k, reference=reference,
+                  stream=stream.h)
+    u = e.u_blocks()
+    for j, (n, faces, f) in enumerate(problems):
+        if j == 0:
+            assert res[j].converged and res[j].sweeps == 0 and np.array_equal(u[j][1:-1, 1:-1, 1:-1], guesses[j][1:-1, 1:-1, 1:-1])
+            continue
+        assert not res[j].converged and res[j].sweeps == k
+        exp = padded(n, faces, oracle)
+        oracle.poisson_jacobi(exp, f, 1e-300, max_sweeps=k, check=k)
+        # FP32 sweeps of a correction about as large as u: a sweep adds at most 8
+        # roundings of 2^-24 and amplifies none
+        err = np.abs(u[j] - exp)[1:-1, 1:-1, 1:-1].max()
+        assert err <= 8 * k * 2.0 ** -24 * max(1.0, np.abs(exp).max())
 
 
 @pytest.mark.gpu
