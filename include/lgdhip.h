@@ -370,7 +370,9 @@ typedef struct lgdhip_poisson_options {
                                     fell by this factor (0: 1e-2)                 */
     int32_t use_graph;           /* replay chunks as a captured hipGraph           */
     int32_t sweep_variant;       /* 0 default (6 for active sets of at least
-                                    2048 of its tiles, else 3), 1 plain sweeps,
+                                    2048 of its tiles, whole planes on chip for
+                                    sets of problems below 64^3 where that is
+                                    faster, else 3), 1 plain sweeps,
                                     2 / 3 temporal blocking with 2 / 4 sweeps per
                                     launch, 4 / 5 4 sweeps with two rows per
                                     thread (32- / 16-row tiles), 6 with three
@@ -437,7 +439,8 @@ int lgdhip_poisson_sweeps_f64(double *ua, double *ub, const float *f, const lgdh
                               lgdhip_stream_t stream);
 
 /* The blocked sweep variant a launch over these problems uses for
- * `requested` (0: the default, resolved by launch size; 1-6 are kept).  No
+ * `requested` (0: the default, resolved by launch size; 1-6 are kept; 7 names
+ * the kernel of small problem sets, which holds whole planes on chip).  No
  * device work; for tools.  No counterpart in the reference (the ensemble
  * solver is new with this library). */
 int lgdhip_poisson_sweep_plan(const lgdhip_poisson_problem *probs, int count, int requested, int *variant);

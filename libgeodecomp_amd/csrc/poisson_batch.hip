@@ -480,6 +480,140 @@ __global__ __launch_bounds__(64 * TY) void poisson_sweep_tb2(const float *__rest
     }
 }
 
+// K FP32 sweeps per launch for small problems, without a march: a work-group
+// holds whole x-y planes of one problem, the NP planes z0 - K .. z0 + NP - K - 1
+// of e and r in registers (a lane one x, RY adjacent rows), and runs level after
+// level on all of them at once, a plane fewer at both ends per level; it writes
+// its NP - 2K middle planes.  x neighbours come from the adjacent lanes (rows of
+// LX lanes: n < LX, so the zero lane past a row's end is also the next row's
+// left neighbour), y neighbours of a thread's first and last row through LDS,
+// z neighbours are the thread's own.  Cells, sum order, zero halo and residual
+// partials as in poisson_sweep_tb: bit-exact with K launches of
+// poisson_sweep_f32.
+//
+// A small set is bound by latency: the marching kernel needs a chunk plus 2K
+// dependent plane steps per launch, each with its barrier and level chain,
+// this one K levels with one barrier each (one more where the planes do not
+// fit LDS twice), every level's planes independent of each other.
+template <int LX, int RY, int NP, int K, bool DAMPED>
+__global__ __launch_bounds__(1024) void poisson_sweep_slab(const float *__restrict__ e, float *__restrict__ e2,
+                                                           const float *__restrict__ r,
+                                                           const Tile *__restrict__ tiles,
+                                                           const ProblemDev *__restrict__ probs,
+                                                           double *__restrict__ partial, unsigned ntiles, unsigned per,
+                                                           float omega, const SolveState *__restrict__ state) {
+    constexpr int NG = 16 * 64 / LX;         // row groups of RY rows
+    constexpr int NS = RY > 1 ? 2 : 1;       // rows a group publishes: first, last
+    constexpr int kPlane = (NG + 1) * NS * LX;
+    constexpr int NB = 2 * NP * kPlane * 4 <= 160 * 1024 ? 2 : 1;  // LDS buffers
+    __shared__ float lds[NB][NP][NG + 1][NS][LX];  // group g at index g + 1, zeros at 0
+    __shared__ double red[16];
+    const unsigned tid = lgdhip::xcd_tile(blockIdx.x, per, true);
+    if (tid >= ntiles) return;  // whole work-group, before any barrier
+    const Tile t = tiles[tid];
+    if (state && state[t.p].done) return;
+    const ProblemDev P = probs[t.p];
+    const int n = P.n;
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int x = lane % LX, grp = wave * (64 / LX) + lane / LX;
+    const int y0 = grp * RY;
+    const bool idle = wave * (64 / LX) * RY >= n;  // no row of the wave inside: its planes stay zero
+    const int64_t sx = n + 2, sxy = sx * sx;
+    const int zb = t.z0 - K;  // plane 0
+    float ev[NP][RY], rv[NP][RY];
+    bool live[RY];
+    const int64_t col = P.base + (int64_t)(y0 + 1) * sx + (x + 1);
+#pragma unroll
+    for (int j = 0; j < RY; ++j) live[j] = x < n && y0 + j < n;
+#pragma unroll
+    for (int p = 0; p < NP; ++p) {
+        const bool zin = (unsigned)(zb + p) < (unsigned)n;
+        const int64_t at = col + (int64_t)(zb + p + 1) * sxy;
+#pragma unroll
+        for (int j = 0; j < RY; ++j) {
+            ev[p][j] = zin && live[j] ? e[at + j * sx] : 0.0f;
+            rv[p][j] = p > 0 && p < NP - 1 && zin && live[j] ? r[at + j * sx] : 0.0f;
+        }
+    }
+    if (grp == 0) {
+#pragma unroll
+        for (int b = 0; b < NB; ++b)
+#pragma unroll
+            for (int p = 0; p < NP; ++p)
+#pragma unroll
+                for (int q = 0; q < NS; ++q) lds[b][p][0][q][x] = 0.0f;
+    }
+    const int below = grp < NG - 1 ? grp + 2 : grp + 1;  // the last group's last row is never live
+    double acc = 0.0;
+    for (int l = 1; l <= K; ++l) {
+        const int b = NB == 2 ? (l & 1) : 0;
+#pragma unroll
+        for (int p = 1; p < NP - 1; ++p)
+            if (p >= l && p < NP - l) {
+                lds[b][p][grp + 1][0][x] = ev[p][0];
+                if (RY > 1) lds[b][p][grp + 1][NS - 1][x] = ev[p][RY - 1];
+            }
+        __syncthreads();
+        if (!idle) {
+            float before[RY];
+#pragma unroll
+            for (int j = 0; j < RY; ++j) before[j] = ev[0][j];
+#pragma unroll
+            for (int p = 1; p < NP - 1; ++p) {
+                if (p >= l && p < NP - l) {
+                    const bool zin = (unsigned)(zb + p) < (unsigned)n;
+                    const float first = lds[b][p][grp][NS - 1][x], last = lds[b][p][below][0][x];
+                    float up = first;  // the row above, before this level
+#pragma unroll
+                    for (int j = 0; j < RY; ++j) {
+                        const float c = ev[p][j];
+                        float sum = before[j];               // ( 0,  0, -1)
+                        sum += up;                           // ( 0, -1,  0)
+                        sum += lane_prev(c);                 // (-1,  0,  0)
+                        sum += lane_next(c);                 // ( 1,  0,  0)
+                        sum += j < RY - 1 ? ev[p][j + 1 < RY ? j + 1 : j] : last;  // ( 0,  1,  0)
+                        sum += ev[p + 1][j];                 // ( 0,  0,  1)
+                        sum += rv[p][j];
+                        const float jv = DAMPED ? __builtin_fmaf(omega, __builtin_fmaf(sum, 1.0f / 6.0f, -c), c)
+                                                : sum * (1.0f / 6.0f);
+                        if (partial && l == K && zin && live[j]) {
+                            const double rr = (double)sum - 6.0 * (double)c;
+                            acc += rr * rr;
+                        }
+                        ev[p][j] = zin && live[j] ? jv : 0.0f;
+                        before[j] = c;
+                        up = c;
+                    }
+                } else {
+#pragma unroll
+                    for (int j = 0; j < RY; ++j) before[j] = ev[p][j];
+                }
+            }
+        }
+        if (NB == 1) __syncthreads();
+    }
+#pragma unroll
+    for (int p = K; p < NP - K; ++p)
+        if (zb + p < n) {
+            const int64_t at = col + (int64_t)(zb + p + 1) * sxy;
+#pragma unroll
+            for (int j = 0; j < RY; ++j)
+                if (live[j]) e2[at + j * sx] = ev[p][j];
+        }
+    if (partial) {
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) acc += __shfl_xor(acc, o, 64);
+        if (lane == 0) red[wave] = acc;
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            double sum = 0.0;
+            for (int k = 0; k < 16; ++k) sum += red[k];
+            partial[tid] = sum;
+        }
+    }
+}
+
 // u += e over the interior and reset both correction buffers to zero, for the
 // problems marked `refresh`
 __global__ __launch_bounds__(kThreads) void poisson_update_f64(double *__restrict__ u, float *e, float *eother,
@@ -630,6 +764,8 @@ void append_tiles(std::vector<Tile> *out, int p, int n) {
 // tiles, tb_zchunk)
 struct TbShape {
     int k, ty, rows;  // sweeps per launch, work-group rows, tile rows per work-group row
+    int slab = 0;     // poisson_sweep_slab: its output planes per work-group
+    int lanes = 0;    // and lanes per row
 };
 constexpr int kTbZ = 64;
 // the default: 4 sweeps per launch, three rows per thread in 48-row tiles
@@ -645,6 +781,7 @@ constexpr int kDefaultSweepVariant = 6;
 constexpr int kSmallSweepVariant = 3;
 constexpr int64_t kTallMinTiles = 2048;
 constexpr int kSweepVariants = 6;
+constexpr int kSlabVariant = 7;  // named by the plan only
 TbShape tb_shape(int variant) {
     switch (variant) {
     case 2: return {2, 16, 1};
@@ -657,11 +794,16 @@ TbShape tb_shape(int variant) {
 }
 
 int64_t tb_tiles_of(int n, TbShape sh, int zchunk = kTbZ) {
+    if (sh.slab) return (n + sh.slab - 1) / sh.slab;
     const int ox = 64 - 2 * sh.k, oy = sh.ty * sh.rows - 2 * sh.k;
     return (int64_t)((n + ox - 1) / ox) * ((n + oy - 1) / oy) * ((n + zchunk - 1) / zchunk);
 }
 
 void append_tb_tiles(std::vector<Tile> *out, int p, int n, TbShape sh, int zchunk) {
+    if (sh.slab) {
+        for (int z = 0; z < n; z += sh.slab) out->push_back(Tile{p, 0, 0, z});
+        return;
+    }
     const int ox = 64 - 2 * sh.k, oy = sh.ty * sh.rows - 2 * sh.k;
     for (int z = 0; z < n; z += zchunk)
         for (int y = 0; y < n; y += oy)
@@ -685,19 +827,58 @@ int tb_zchunk(const lgdhip_poisson_problem *probs, const std::vector<int> &set, 
         for (int k : set) t += tb_tiles_of(probs[k].n, sh, zc);
         return t;
     };
-    int zc = kTbZ;
-    while (zc > 4 && tiles(zc) < kTbMinGroups) zc /= 2;
+    int zc = sh.slab ? sh.slab : kTbZ;
+    while (!sh.slab && zc > 4 && tiles(zc) < kTbMinGroups) zc /= 2;
     return zc;
 }
 
-// the blocked sweep shape of a launch over the problems in `set`: the
-// requested variant, or for 0 the default by launch size
+// Slab shapes, all of 4 sweeps: output planes, lanes and rows per thread.
+constexpr TbShape kSlabShapes[] = {{4, 16, 1, 8, 32}, {4, 16, 1, 2, 32}, {4, 16, 3, 4, 64},
+                                   {4, 16, 3, 2, 64}, {4, 16, 4, 4, 64}, {4, 16, 4, 2, 64}};
+
+// The blocked sweep shape of a launch over the problems in `set`: the
+// requested variant, or for 0 the default by launch size: a slab shape where it
+// is modelled faster, else three rows per thread for large launches and one row
+// for small ones.  Measured per launch of 4 sweeps (MI355X, slab / one row):
+// 1 x 31^3 7.5 / 8.9 us, 16 x 31^3 7.9 / 12.6, 64 x 31^3 12.1 / 22.1, 16 x 40^3
+// 14.3 / 20.0, 16 x 63^3 21.6 / 32.8, but 1 x 40^3 11.9 / 9.4, 1 x 63^3
+// 13.6 / 9.5.  8 sweeps per launch in 18 planes took 16.0 us at 16 x 31^3, no
+// less per sweep.
 TbShape sweep_shape(int requested, const lgdhip_poisson_problem *probs, const std::vector<int> &set) {
     if (requested >= 1 && requested <= kSweepVariants) return tb_shape(requested);
-    const TbShape tall = tb_shape(kDefaultSweepVariant);
+    const TbShape tall = tb_shape(kDefaultSweepVariant), flat = tb_shape(kSmallSweepVariant);
+    int nmax = 0;
     int64_t tiles = 0;
-    for (int k : set) tiles += tb_tiles_of(probs[k].n, tall);
-    return tiles >= kTallMinTiles ? tall : tb_shape(kSmallSweepVariant);
+    for (int k : set) {
+        nmax = std::max(nmax, (int)probs[k].n);
+        tiles += tb_tiles_of(probs[k].n, tall);
+    }
+    if (tiles >= kTallMinTiles) return tall;
+    if (set.empty() || nmax >= 64) return flat;
+    // the one-row kernel: 0.65 us a plane step, 0.9 us with two work-groups on
+    // a CU, which holds no more
+    const int zc = tb_zchunk(probs, set, flat);
+    int64_t groups = 0;
+    for (int k : set) groups += tb_tiles_of(probs[k].n, flat, zc);
+    TbShape best = flat;
+    double best_us = 1.5 + (double)((groups + 2 * lgdhip::kCUs - 1) / (2 * lgdhip::kCUs)) * (zc + 2 * flat.k) *
+                               (groups > (int64_t)lgdhip::kCUs ? 0.9 : 0.65);
+    for (const TbShape &sh : kSlabShapes) {
+        if (nmax >= std::min(sh.lanes, 16 * sh.rows * 64 / sh.lanes)) continue;
+        int64_t slabs = 0;
+        for (int k : set) slabs += tb_tiles_of(probs[k].n, sh);
+        if (slabs > kTbSmallListTiles && sh.slab < 8) continue;  // the tile lists' capacity
+        // a slab kernel: one work-group per CU; loads, levels' barriers and
+        // the planes of all levels at 0.09 us per 1024 cells
+        const double planes = sh.k * sh.slab + sh.k * (sh.k - 1);
+        const double us = 5.0 + 0.3 * sh.k +
+                          (double)((slabs + lgdhip::kCUs - 1) / lgdhip::kCUs) * planes * sh.rows * 0.09;
+        if (us < best_us) {
+            best_us = us;
+            best = sh;
+        }
+    }
+    return best;
 }
 
 int check_problems(const lgdhip_poisson_problem *probs, int count) {
@@ -807,6 +988,16 @@ template <bool DAMPED>
 void launch_tb_kind(TbShape sh, const float *a, float *b, const float *r, const Workspace &w, int64_t ntiles,
                     int zchunk, double *partial, float omega, const SolveState *state, hipStream_t s) {
     const unsigned nt = (unsigned)ntiles, per = lgdhip::xcd_per(nt), groups = lgdhip::xcd_groups(nt);
+#define LGD_SLAB_CASE(K, ZS, LX, RY)                                                                           \
+    if (sh.k == K && sh.slab == ZS && sh.lanes == LX && sh.rows == RY) {                                                   \
+        poisson_sweep_slab<LX, RY, ZS + 2 * K, K, DAMPED><<<groups, 1024, 0, s>>>(a, b, r, w.tb_tiles, w.probs, \
+                                                                                  partial, nt, per, omega,     \
+                                                                                  state);                      \
+        return;                                                                                                \
+    }
+    LGD_SLAB_CASE(4, 8, 32, 1) LGD_SLAB_CASE(4, 2, 32, 1) LGD_SLAB_CASE(4, 4, 64, 4)
+    LGD_SLAB_CASE(4, 2, 64, 4) LGD_SLAB_CASE(4, 4, 64, 3) LGD_SLAB_CASE(4, 2, 64, 3)
+#undef LGD_SLAB_CASE
     if (sh.rows == 3)
         poisson_sweep_tb2<4, 16, 3, DAMPED><<<groups, dim3(64, 16), 0, s>>>(a, b, r, w.tb_tiles, w.probs, partial,
                                                                             zchunk, nt, per, omega, state);
@@ -1134,7 +1325,7 @@ int lgdhip_poisson_sweep_plan(const lgdhip_poisson_problem *probs, int count, in
     std::vector<int> all(count);
     for (int k = 0; k < count; ++k) all[k] = k;
     const TbShape sh = sweep_shape(0, probs, all);
-    *variant = sh.rows > 1 ? kDefaultSweepVariant : kSmallSweepVariant;
+    *variant = sh.slab ? kSlabVariant : (sh.rows > 1 ? kDefaultSweepVariant : kSmallSweepVariant);
     return 0;
 }
 

@@ -222,6 +222,48 @@ def test_gpu_sweeps_bit_exact(hip, oracle, variant, sweeps):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("sizes", [[31, 1, 2, 17, 30], [31] * 60 + [9] * 9, [44, 47, 8, 33] * 4, [40, 47, 1] * 8,
+                                   [63, 62, 61, 48, 2], [63, 62, 5, 50] * 5], ids=lambda s: f"{len(s)}x{max(s)}")
+def test_gpu_small_problem_sweeps_bit_exact(hip, sizes):
+    """The kernels that hold a small problem's planes on chip, one set for each
+    shape (rows of 32 or 64 lanes, 1, 3 or 4 rows per thread, 2, 4 or 8 output
+    planes): plain and weighted sweeps, counts with remainders, noise in r's
+    halo, equal to single sweeps bit for bit, both through a workspace and
+    through the static scratch."""
+    rng = np.random.default_rng(len(sizes))
+    b = Batch(hip, [(n, np.zeros(6), np.zeros((n + 2,) * 3, np.float32)) for n in sizes])
+    plan = C.c_int(-1)
+    hip.call("lgdhip_poisson_sweep_plan", b.probs, b.count, 0, C.byref(plan))
+    assert plan.value == 7
+    e_host = np.zeros(b.elems, np.float32)
+    for k, n in enumerate(sizes):
+        e = np.zeros((n + 2,) * 3, np.float32)
+        e[1:-1, 1:-1, 1:-1] = rng.standard_normal((n, n, n))
+        e_host[b.probs[k].offset:][:e.size] = e.ravel()
+    ea, eb, r = (hip.DeviceBuffer(b.elems * 4) for _ in range(3))
+    r.upload(rng.standard_normal(b.elems).astype(np.float32))
+
+    def run(name, sweeps, *extra, variant, ws=True):
+        ea.upload(e_host)
+        eb.upload(np.zeros(b.elems, np.float32))
+        in_b, tile = C.c_int(-1), hip.tile(variant=variant)
+        print("[case]", name, len(sizes), max(sizes), sweeps, variant, flush=True)
+        hip.call(name, ea.ptr, eb.ptr, r.ptr, b.probs, b.count, sweeps, *extra, C.byref(tile),
+                 *((b.ws.ptr, b.ws_bytes) if ws else ()), C.byref(in_b), None)
+        hip.call("lgdhip_device_synchronize")
+        out = np.empty(b.elems, np.float32)
+        (eb if in_b.value else ea).download(out)
+        return out
+
+    for sweeps in (4, 9, 16):
+        plain = run("lgdhip_poisson_sweeps_f32", sweeps, variant=1)
+        assert np.array_equal(run("lgdhip_poisson_sweeps_f32", sweeps, variant=0), plain)
+        assert np.array_equal(run("lgdhip_poisson_sweeps_f32_noalloc", sweeps, variant=0, ws=False), plain)
+        damped = run("lgdhip_poisson_damped_sweeps_f32", sweeps, 2.0 / 3.0, variant=1)
+        assert np.array_equal(run("lgdhip_poisson_damped_sweeps_f32", sweeps, 2.0 / 3.0, variant=0), damped)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("variant,sweeps", [(1, 3), (3, 9), (4, 10), (5, 8), (0, 12), (6, 9)])
 def test_gpu_damped_sweeps_bit_exact(hip, oracle, variant, sweeps):
     """Weighted sweeps (omega = 2/3, the smoothing phase's) through every
