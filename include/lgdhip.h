@@ -243,8 +243,9 @@ int lgdhip_grid_store(const void *grid, const lgdhip_grid *g, void *host,
 /* Runs `steps` sweeps ping-ponging between a and b (both carry the edge
  * value in their halo).  *result_in_b is set to 1 when the final state is
  * in b, 0 when it is in a (tile->variant 4-10 run K = 2-4 sweeps per launch
- * and swap once per launch, so this is not steps % 2 there; 11 and 12 run
- * the same tile pipelines for one sweep per launch). */
+ * and swap once per launch, so this is not steps % 2 there, nor for the
+ * default, which runs 4 sweeps per launch and a last launch of steps % 4; 11
+ * and 12 run the same tile pipelines for one sweep per launch). */
 int lgdhip_jacobi3d_f64_run(double *a, double *b, const lgdhip_grid *g, int steps,
                             const lgdhip_tile *tile, int *result_in_b,
                             lgdhip_stream_t stream);
@@ -272,8 +273,9 @@ int lgdhip_jacobi3d_f64_run_zrange(const double *src, double *dst, const lgdhip_
  * geometry/topologies.h:225-247,267-280: a neighbour past a wrapped face is
  * the cell on the opposite face; past an unwrapped face it is `edge`).  The
  * temporal-blocking variants take the wrapped neighbours straight from the
- * interior; steps % K are single sweeps after a periodic halo refresh
- * (lgdhip_grid_fill_halo).  Both buffers' halos are rewritten.  A wrapped z
+ * interior; the default's steps % K are one blocked launch too, a requested
+ * variant's single sweeps after a periodic halo refresh
+ * (lgdhip_grid_fill_halo).  Both buffers' halos may be rewritten.  A wrapped z
  * axis shorter than 8 cells runs single sweeps throughout.  Results equal
  * `steps` single sweeps of the periodic stencil bit for bit; *result_in_b
  * as for lgdhip_jacobi3d_f64_run.  Views are refused. */

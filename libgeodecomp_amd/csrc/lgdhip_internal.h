@@ -54,6 +54,10 @@ __host__ __device__ __forceinline__ void static_for(F &&f) {
 // Views (LGDHIP_GRID_VIEW) are rejected unless allow_view.
 int check_grid(const lgdhip_grid *g, int dim, int elem_bytes, int members, bool allow_view = false);
 
+// lgdhip_grid_fill_halo for `grid` and, in the same launch, `other` (NULL: none)
+int fill_halos(void *grid, void *other, const lgdhip_grid *g, const void *edge, int wrap_mask,
+               lgdhip_stream_t stream);
+
 inline int64_t plane_elems(const lgdhip_grid &g) { return g.sx * g.sy * g.sz; }
 // element strides between members and between z slices (LGDHIP_LAYOUT_*)
 inline int64_t member_stride(const lgdhip_grid &g) {

@@ -107,22 +107,43 @@ __global__ void lgd_fill_edge_kernel(T *__restrict__ plane, T edge, int64_t sx, 
 // outside the box along an unwrapped axis, the edge value -- the rule of
 // Topology::normalize + isOutOfBounds.  Reads only interior cells, writes
 // only halo cells.
-template <typename T>
-__global__ void lgd_fill_halo_kernel(T *__restrict__ plane, T edge, int64_t sx, int64_t zs, int64_t ox, int64_t oy,
-                                     int64_t oz, int64_t nx, int64_t ny, int64_t nz, int h, int dim, int wrap) {
-    const int64_t ex = nx + 2 * h, ey = ny + 2 * h, ez = dim == 3 ? nz + 2 * h : 1;
-    const int64_t total = ex * ey * ez;
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < total;
-         i += (int64_t)gridDim.x * blockDim.x) {
-        const int64_t x = i % ex - h, y = (i / ex) % ey - h, z = dim == 3 ? i / (ex * ey) - h : 0;
-        if (x >= 0 && x < nx && y >= 0 && y < ny && z >= 0 && z < nz) continue;
-        int64_t wx = x, wy = y, wz = z;
-        if (wrap & 1) wx = ((x % nx) + nx) % nx;
-        if (wrap & 2) wy = ((y % ny) + ny) % ny;
-        if ((wrap & 4) && dim == 3) wz = ((z % nz) + nz) % nz;
+// Threads run over the shell only, first the z layers (whole padded planes),
+// then the y layers of the other planes, then the x layers of the rest (over
+// the whole padded box, with 64-bit divisions, a 150 x 101 x 77 grid took
+// 11.3 us); I: 32-bit indices while the shell has fewer than 2^31 cells.
+template <typename T, typename I>
+__global__ void lgd_fill_halo_kernel(T *plane0, T *plane1, T edge, int64_t sx, int64_t zs, int64_t ox, int64_t oy,
+                                     int64_t oz, I nx, I ny, I nz, I h, int dim, int wrap) {
+    T *__restrict__ plane = blockIdx.y ? plane1 : plane0;
+    const I ex = nx + 2 * h, ey = ny + 2 * h, h2 = 2 * h;
+    const I zcells = dim == 3 ? h2 * ex * ey : 0, ycells = nz * h2 * ex, total = zcells + ycells + nz * ny * h2;
+    auto layer = [h](I k, I n) { return k < h ? k - h : n + (k - h); };  // layer k of 2h around [0, n)
+    auto image = [](I c, I n) { return ((c % n) + n) % n; };
+    for (int64_t at = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; at < (int64_t)total;
+         at += (int64_t)gridDim.x * blockDim.x) {
+        I i = (I)at, x, y, z;
+        if (i < zcells) {
+            x = i % ex - h;
+            i /= ex;
+            y = i % ey - h;
+            z = layer(i / ey, nz);
+        } else if ((i -= zcells) < ycells) {
+            x = i % ex - h;
+            i /= ex;
+            y = layer(i % h2, ny);
+            z = i / h2;
+        } else {
+            i -= ycells;
+            x = layer(i % h2, nx);
+            i /= h2;
+            y = i % ny;
+            z = i / ny;
+        }
+        const I wx = (wrap & 1) ? image(x, nx) : x, wy = (wrap & 2) ? image(y, ny) : y;
+        const I wz = (wrap & 4) && dim == 3 ? image(z, nz) : z;
         const bool inside = wx >= 0 && wx < nx && wy >= 0 && wy < ny && wz >= 0 && wz < nz;
-        const T v = inside ? plane[(wz + oz) * zs + (wy + oy) * sx + (wx + ox)] : edge;
-        plane[(z + oz) * zs + (y + oy) * sx + (x + ox)] = v;
+        const T v = inside ? plane[((int64_t)wz + oz) * zs + ((int64_t)wy + oy) * sx + (wx + ox)] : edge;
+        plane[((int64_t)z + oz) * zs + ((int64_t)y + oy) * sx + (x + ox)] = v;
     }
 }
 
@@ -132,6 +153,55 @@ static unsigned fill_blocks(size_t n) {
     if (b == 0) b = 1;
     return (unsigned)b;
 }
+
+namespace lgdhip {
+// the halo of one grid, or of two of the same shape by one launch
+int fill_halos(void *grid, void *other, const lgdhip_grid *g, const void *edge, int wrap_mask,
+               lgdhip_stream_t stream) {
+    int rc = check_grid(g, 0, 0, 0);
+    if (rc) return rc;
+    LGD_REQUIRE(grid && edge, "NULL pointer");
+    LGD_REQUIRE(wrap_mask >= 0 && wrap_mask <= 7, "wrap_mask must be a combination of bits 1, 2, 4");
+    const int64_t n = member_stride(*g);
+    const int h = g->halo;
+    const double ex = g->nx + 2.0 * h, ey = g->ny + 2.0 * h;
+    const double cells = 2.0 * h * ((g->dim == 3 ? ex * ey : 0.0) + (double)g->nz * ex + (double)g->nz * g->ny);
+    LGD_REQUIRE(cells < 9e18, "halo too large");
+    const int64_t shell = (int64_t)cells;
+    const bool small = shell < INT32_MAX;
+    const dim3 blocks(fill_blocks((size_t)shell), other ? 2 : 1);
+    hipStream_t s = as_stream(stream);
+    const int64_t zs = z_stride(*g);
+    for (int m = 0; m < g->members; ++m) {
+        const uint8_t *ev = (const uint8_t *)edge + (size_t)m * g->elem_bytes;
+        const size_t at = (size_t)m * n * g->elem_bytes;
+        char *plane = (char *)grid + at, *plane1 = other ? (char *)other + at : plane;
+#define LGD_HALO_CASE(BYTES, T)                                                                                   \
+    case BYTES: {                                                                                                 \
+        T v;                                                                                                      \
+        std::memcpy(&v, ev, BYTES);                                                                               \
+        if (small)                                                                                                \
+            lgd_fill_halo_kernel<T, int32_t><<<blocks, 256, 0, s>>>((T *)plane, (T *)plane1, v, g->sx, zs, g->ox, g->oy, g->oz, \
+                                                                    (int32_t)g->nx, (int32_t)g->ny, (int32_t)g->nz, \
+                                                                    h, g->dim, wrap_mask);                        \
+        else                                                                                                      \
+            lgd_fill_halo_kernel<T, int64_t><<<blocks, 256, 0, s>>>((T *)plane, (T *)plane1, v, g->sx, zs, g->ox, g->oy, g->oz, \
+                                                                    g->nx, g->ny, g->nz, h, g->dim, wrap_mask);   \
+        break;                                                                                                    \
+    }
+        switch (g->elem_bytes) {
+            LGD_HALO_CASE(1, uint8_t)
+            LGD_HALO_CASE(2, uint16_t)
+            LGD_HALO_CASE(4, uint32_t)
+            LGD_HALO_CASE(8, uint64_t)
+        default: return set_error(LGDHIP_ERR_UNSUPPORTED, "element size must be 1, 2, 4 or 8 bytes");
+        }
+#undef LGD_HALO_CASE
+        LGD_LAUNCHED("lgdhip_grid_fill_halo");
+    }
+    return 0;
+}
+} // namespace lgdhip
 
 // ---------------------------------------------------------------------------
 // C-ABI
@@ -442,38 +512,7 @@ int64_t lgdhip_grid_bytes(const lgdhip_grid *g) {
 
 int lgdhip_grid_fill_halo(void *grid, const lgdhip_grid *g, const void *edge, int wrap_mask,
                           lgdhip_stream_t stream) {
-    int rc = check_grid(g, 0, 0, 0);
-    if (rc) return rc;
-    LGD_REQUIRE(grid && edge, "NULL pointer");
-    LGD_REQUIRE(wrap_mask >= 0 && wrap_mask <= 7, "wrap_mask must be a combination of bits 1, 2, 4");
-    const int64_t n = member_stride(*g);
-    const int h = g->halo;
-    const int64_t shell = (g->nx + 2 * h) * (g->ny + 2 * h) * (g->dim == 3 ? g->nz + 2 * h : 1);
-    const unsigned blocks = fill_blocks((size_t)shell);
-    hipStream_t s = as_stream(stream);
-    const int64_t zs = z_stride(*g);
-    for (int m = 0; m < g->members; ++m) {
-        const uint8_t *ev = (const uint8_t *)edge + (size_t)m * g->elem_bytes;
-        char *plane = (char *)grid + (size_t)m * n * g->elem_bytes;
-#define LGD_HALO_CASE(BYTES, T)                                                                                   \
-    case BYTES: {                                                                                                 \
-        T v;                                                                                                      \
-        std::memcpy(&v, ev, BYTES);                                                                               \
-        lgd_fill_halo_kernel<T><<<blocks, 256, 0, s>>>((T *)plane, v, g->sx, zs, g->ox, g->oy, g->oz, g->nx,     \
-                                                       g->ny, g->nz, h, g->dim, wrap_mask);                       \
-        break;                                                                                                    \
-    }
-        switch (g->elem_bytes) {
-            LGD_HALO_CASE(1, uint8_t)
-            LGD_HALO_CASE(2, uint16_t)
-            LGD_HALO_CASE(4, uint32_t)
-            LGD_HALO_CASE(8, uint64_t)
-        default: return set_error(LGDHIP_ERR_UNSUPPORTED, "element size must be 1, 2, 4 or 8 bytes");
-        }
-#undef LGD_HALO_CASE
-        LGD_LAUNCHED("lgdhip_grid_fill_halo");
-    }
-    return 0;
+    return lgdhip::fill_halos(grid, nullptr, g, edge, wrap_mask, stream);
 }
 
 int lgdhip_grid_fill_edge(void *grid, const lgdhip_grid *g, const void *edge, lgdhip_stream_t stream) {

@@ -140,6 +140,22 @@ def test_jacobi_periodic_bit_exact(hip, oracle, shape, steps):
             assert np.array_equal(got, exp), (wrap, variant, bz)
 
 
+@pytest.mark.parametrize("shape,steps", [((70, 45, 40), (1, 2, 3, 6, 7)), ((129, 33, 9), (2, 7)), ((5, 3, 8), (3, 5)),
+                                         ((257, 256, 256), (1, 5))])
+def test_jacobi_default_remainders_bit_exact(hip, oracle, shape, steps):
+    """The default's last launch of 1, 2 or 3 sweeps on Cube and periodic grids
+    (the fourth shape is large enough to end with a single sweep after a halo
+    refresh instead)."""
+    nx, ny, nz = shape
+    a = synthetic.jacobi_initial(nx, ny, nz, seed=nx + ny)
+    for k in steps:
+        for wrap in (0, 7, 1, 6):
+            say("jacobi remainder", shape, k, "wrap", wrap)
+            exp = oracle.jacobi3d(a, k, edge=0.5, threads=16, wrap=wrap)
+            got = gpu_jacobi_periodic(hip, a, k, wrap, edge=0.5) if wrap else gpu_jacobi(hip, a, k, edge=0.5)
+            assert np.array_equal(got, exp), (k, wrap)
+
+
 def test_jacobi_zrange_launch_writes_only_its_planes(hip, oracle):
     """lgdhip_jacobi3d_f64_run_zrange: one blocked launch writes the planes
     [z0, z1) of dst, equal to K oracle sweeps there, and leaves every other
