@@ -20,6 +20,7 @@
 #include <hip/hip_bf16.h>
 
 #include <algorithm>
+#include <cmath>
 
 namespace {
 
@@ -222,12 +223,6 @@ __device__ __forceinline__ uint4 load_global16(gh_ptr p) {
     const u32x4 v = *(gq_ptr)p;
     return make_uint4(v.x, v.y, v.z, v.w);
 }
-// one 4-byte word (two BF16) where only that word is used: a 16-byte load
-// of which the code reads one word would still write all four registers,
-// and the compiler, reusing the three it considers dead, then waits for
-// the load before going on
-typedef const unsigned int __attribute__((address_space(1))) *gw_ptr;
-__device__ __forceinline__ unsigned load_global4(gh_ptr p) { return *(gw_ptr)p; }
 
 // IN: how the input is staged -- kInVec, 16-byte loads (cin % 8 == 0);
 // kInMasked, 16-byte loads of a row whose channels past cin (< 8) are
@@ -984,246 +979,228 @@ __global__ __launch_bounds__(256) void conv3d_wgrad_mfma(const u16 *__restrict__
     }
 }
 
-// channels-last (ld, off, C) -> voxel-blocked [nvox / 8][C][8] (C, ld, off
-// and nvox multiples of 8): element (v, c) at ((v / 8) C + c) 8 + v % 8, so
-// a channel's 8 consecutive voxels are 16 contiguous bytes and the 16
-// channels of an MFMA fragment at one 8-voxel group 256 contiguous bytes.
-// A work-group takes 256 voxels and 8 channels: coalesced 16-byte reads of
-// each voxel's 8 channels, a transpose through LDS, 16-byte writes of each
-// channel's 8 voxels (128 contiguous bytes per 8 lanes).
-__global__ __launch_bounds__(256) void to_voxel_blocked(const u16 *__restrict__ src, int64_t nvox, int ld, int off,
-                                                        int C, u16 *__restrict__ dst) {
-    __shared__ uint4 tile[256];  // [voxel of the block][8 channels]
-    const int64_t v0 = (int64_t)blockIdx.x * 256;
-    const int g = blockIdx.y;  // channels 8g .. 8g + 7
-    const int t = threadIdx.x;
-    if (v0 + t < nvox) tile[t] = *(const uint4 *)(src + (v0 + t) * ld + off + 8 * g);
-    __syncthreads();
-    const int vg = t >> 3, c = t & 7;  // voxel group of the block, channel
-    const int64_t vb = v0 + 8 * vg;
-    if (vb >= nvox) return;  // after the only barrier; nvox % 8 == 0
-    const u16 *tl = reinterpret_cast<const u16 *>(tile);
-    Frag f;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) f.h[e] = tl[(8 * vg + e) * 8 + c];
-    *reinterpret_cast<uint4 *>(dst + (((vb >> 3) * C + 8 * g + c) << 3)) = f.q;
-}
+// dW partials of a 3x3x3 layer straight from the channels-last tensors:
+// P[chunk][co][tap*cin + ci] = sum over the chunk's voxels v of dY[v][co] X[v + tap][ci].
+// A work-group owns a 16 x 8 column of voxels and marches a chunk of z planes;
+// TI ci tiles and TO co tiles of 16 channels pass through LDS as one X plane
+// (18 x 10 voxels with halo) and one dY plane per step, double buffered.  The
+// products sum over voxels, so both MFMA operands need 8 voxels of one channel
+// per lane: ds_read_b64_tr_b16 transposes 4 voxels x 16 channels while reading
+// them, so no transposed copy of the tensors is made.  Wave (ti, to, ks) takes
+// one pair of channel tiles and every KS-th of the plane's four 32-voxel steps
+// (two 16-voxel rows): per step and X plane z it reads 9 X fragments (the dy, dx
+// taps) and one new dY fragment, that of plane z + 1; with the kept ones of
+// planes z and z - 1 they make all 27 taps' products (an X plane serves dz = -1,
+// 0, 1 for the dY planes z + 1, z, z - 1).  108 accumulator registers per wave;
+// the KS waves of a tile pair are summed through LDS in a fixed order.
+//
+// Per MFMA (16 cycles) the wave reads 10/27 of a fragment (8 LDS cycles), so the
+// matrix cores, not LDS, bound the loop; at 16 channels the launch is bound by
+// its one pass over memory.  MI355X, reduction included: 128^3 16 -> 16 42 us
+// (voxel-blocked copies and a kernel reading them: 207), 48 -> 16 104 us (570),
+// 64^3 96 -> 32 59 us (154); with one plane in flight instead of two 73 + 6 us
+// and 106 + 12 us at 128^3.  Volumes of n % 8 != 0 had the gather kernel only
+// (60^3 32 -> 32: 30 us, 250 before).
+typedef short s16x4 __attribute__((ext_vector_type(4)));
+typedef s16x4 __attribute__((address_space(3))) *ls_ptr;
+constexpr int kWgX = 18, kWgVox = 18 * 10, kWgOut = 16 * 8;
 
-// 8 BF16 of one channel's voxels shifted by one voxel: dx = -1 gives
-// element e = c[e-1] with element 0 from the previous 8 (their last word,
-// elements 6 and 7: prev_w); dx = +1 gives c[e+1] with element 7 from the
-// next 8 (their first word, elements 0 and 1: next_x); little-endian
-// halves, so each 32-bit word is an alignbit of two neighbours
-__device__ __forceinline__ uint4 shift_from_prev(uint4 c, unsigned prev_w) {
-    return make_uint4(__builtin_amdgcn_alignbit(c.x, prev_w, 16), __builtin_amdgcn_alignbit(c.y, c.x, 16),
-                      __builtin_amdgcn_alignbit(c.z, c.y, 16), __builtin_amdgcn_alignbit(c.w, c.z, 16));
-}
-__device__ __forceinline__ uint4 shift_from_next(uint4 c, unsigned next_x) {
-    return make_uint4(__builtin_amdgcn_alignbit(c.y, c.x, 16), __builtin_amdgcn_alignbit(c.z, c.y, 16),
-                      __builtin_amdgcn_alignbit(c.w, c.z, 16), __builtin_amdgcn_alignbit(next_x, c.w, 16));
-}
+template <int TI, int TO, int KS, int IN>
+__global__ __launch_bounds__(64 * TI * TO * KS, TI * TO * KS == 4 ? 3 : 1) void conv3d_wgrad_zm(const u16 *__restrict__ X, int n, int ldx,
+                                                                     int offx, int cin, const u16 *__restrict__ dY,
+                                                                     int ldy, int offy, int cout, int Kp, int zchunk,
+                                                                     int bx, int by, int gi, int go,
+                                                                     float *__restrict__ P, unsigned groups,
+                                                                     unsigned per) {
+    constexpr int T = 64 * TI * TO * KS;
+    constexpr int PX = kWgVox * 2 * TI, PY = kWgOut * 2 * TO;  // 16-byte pieces of a plane
+    constexpr int PERX = (PX + T - 1) / T, PERY = (PY + T - 1) / T;
+    constexpr int NKS = 4 / KS;                                // 32-voxel steps per wave and plane
+    constexpr int kStage = 2 * (PX + PY);                      // uint4: [X buffers][dY buffers]
+    constexpr int kRed = KS > 1 ? KS / 2 * TI * TO * 9 * 64 : 0;  // uint4 (4 floats): a dz's accumulators of half the waves
+    __shared__ uint4 smem[kStage > kRed ? kStage : kRed];
+    uint4 *const xs = smem, *const ys = smem + 2 * PX;
+    unsigned b = lgdhip::xcd_tile(blockIdx.x, per, true);
+    if (b >= groups) return;  // whole work-group, before any barrier
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int ks = wave % KS, ti = wave / KS % TI, to = wave / KS / TI;
+    const int x0 = (int)(b % bx) * 16;
+    b /= bx;
+    const int y0 = (int)(b % by) * 8;
+    b /= by;
+    const int ig = (int)(b % gi);
+    b /= gi;
+    const int og = (int)(b % go);
+    const int zc = (int)(b / go);
+    const int zs = zc * zchunk, ze = min(zs + zchunk, n);
+    const int ci0 = ig * TI * 16, co0 = og * TO * 16;
 
-// dW partial from voxel-blocked copies: P[chunk][co][tap*cin + ci] =
-// sum over the chunk's voxels v of G[co][v] X[ci][v + tap].  One wave per
-// (chunk, taps, group of CT co tiles, group of IT ci tiles).  A wave's
-// taps: DXT = 3 takes the three x-shifted taps of a (dz, dy) row, whose B
-// fragments come from the row's centre 8 voxels and one word of each
-// neighbouring 8; DYT = 3 (with DXT = 3) takes the three rows of one dz as
-// well, so 9 taps share the A fragment, the voxel stepping and the
-// validity tests (per MFMA about a third of the bookkeeping of one row);
-// DXT = 1: one tap.  Per 32 voxels (4 groups of 8 consecutive voxels of one
-// x row, n % 8 == 0) every fragment is one 16-byte load per lane, the 16
-// lanes of a voxel group reading 256 contiguous bytes of the voxel-blocked
-// copy.  Needs ksize 3, cin and cout multiples of 16, chunk_vox a multiple
-// of 32.  Work-groups (4 waves) run in XCD order: XCD c takes the
-// contiguous range [c per, (c + 1) per), so the waves of one chunk and of
-// the chunks above and beside it (whose rows its dz / dy taps read) share
-// one L2 instead of every XCD fetching every chunk's rows.
-template <int CT, int IT, int DXT, int DYT>
-__global__ __launch_bounds__(256) void conv3d_wgrad_cf(const u16 *__restrict__ Xc, const u16 *__restrict__ Gc, int n,
-                                                       int cin, int cout, int Kp, int chunk_vox, int cotg, int citg,
-                                                       float *__restrict__ P, unsigned per) {
-    static_assert(DYT == 1 || DXT == 3, "three y rows take the three x taps of each");
-    constexpr int kGroups = 27 / (DXT * DYT);  // dz planes, (dz, dy) rows or single taps
-    const int lane = threadIdx.x & 63;
-    const int64_t nvox = (int64_t)n * n * n;
-    const int64_t chunks = (nvox + chunk_vox - 1) / chunk_vox;
-    const int64_t tasks = (int64_t)kGroups * cotg * citg;
-    const int64_t wave = (int64_t)lgdhip::xcd_tile(blockIdx.x, per, true) * 4 + threadIdx.x / 64;
-    if (wave >= chunks * tasks) return;  // no barriers in this kernel
-    const int64_t chunk = wave / tasks;
-    int64_t rem = wave % tasks;
-    const int grp = (int)(rem % kGroups);  // taps fastest: neighbouring waves share the G fragments
-    rem /= kGroups;
-    const int cig = (int)(rem % citg), cog = (int)(rem / citg);
-    const int tap0 = grp * DXT * DYT;  // taps tap0 + 3 r + e: row dy + r, x offset e - 1 (DXT = 3)
-    int dz, dy, dx0;
-    tap_offset(tap0, 3, dz, dy, dx0);
-    const int i = lane & 15, q = lane >> 4;
-    f32x4 acc[DYT][DXT][CT][IT];
-#pragma unroll
-    for (int r = 0; r < DYT; ++r)
-#pragma unroll
-        for (int d = 0; d < DXT; ++d)
-#pragma unroll
-            for (int t = 0; t < CT; ++t)
-#pragma unroll
-                for (int u = 0; u < IT; ++u) acc[r][d][t][u] = f32x4{0.f, 0.f, 0.f, 0.f};
-
-    const int64_t v_begin = chunk * chunk_vox;
-    const int64_t v_end = v_begin + chunk_vox < nvox ? v_begin + chunk_vox : nvox;
-    // the fetch front's voxel v = vb + 8q of this lane group and its
-    // coordinates, stepped along with v (32 voxels per step) instead of
-    // divided out each time
-    int x, y, z;
-    {
-        const int64_t v0 = v_begin + 8 * q;
-        x = (int)(v0 % n);
-        const int64_t r0 = v0 / n;
-        y = (int)(r0 % n);
-        z = (int)(r0 / n);
-    }
-    // One 32-voxel step's fragments: dY (A) and each X row's centre 8 with
-    // the adjacent words of its left and right neighbours.  Loads outside
-    // the volume read a zero block instead of being skipped, so they need
-    // no branch.  Addresses are stepped, not recomputed: the voxel-blocked
-    // copies put the front's 8-voxel group g at element (g C + channel) 8,
-    // a step is 4 groups, tap (dz, dy) reads group g + (dz n^2 + dy n) / 8
-    // (exact, n % 8 == 0) and the next row n cin elements further; the
-    // coordinates only decide which loads are inside the volume.
+    // staging: piece k is half g % 2 of tile g / 2 of voxel k / (2 T.): consecutive
+    // threads read consecutive 16 bytes of a voxel's channels
     const gh_ptr zero = (gh_ptr)(const void *)kZero16;
-    struct Step {
-        uint4 a[CT], c[DYT][IT];
-        unsigned prev[DYT][IT], next[DYT][IT];  // the neighbouring 8 voxels' adjacent word
-    };
-    const int64_t g0 = (v_begin + 8 * q) >> 3;
-    const int64_t tap_groups = ((int64_t)dz * n * n + (int64_t)dy * n) >> 3;
-    const int64_t row_elems = (int64_t)n * cin;
-    gh_ptr pa[CT], px[IT];
+    const gh_ptr xg = (gh_ptr)X + offx, yg = (gh_ptr)dY + offy;
+    int xofs[PERX], yofs[PERY];
+    bool xok[PERX], yok[PERY];
 #pragma unroll
-    for (int t = 0; t < CT; ++t) pa[t] = (gh_ptr)Gc + ((g0 * cout + (cog * CT + t) * 16 + i) << 3);
-#pragma unroll
-    for (int u = 0; u < IT; ++u) px[u] = (gh_ptr)Xc + (((g0 + tap_groups) * cin + (cig * IT + u) * 16 + i) << 3);
-    const int64_t step_a = (int64_t)32 * cout, step_x = (int64_t)32 * cin;  // 4 groups of 8 voxels
-    auto fetch = [&](Step &f) {
-#pragma unroll
-        for (int t = 0; t < CT; ++t) f.a[t] = load_global16(pa[t]);
-        const bool zok = (unsigned)(z + dz) < (unsigned)n;
-        const bool xlo = (DXT == 3 || dx0 < 0) && x > 0;
-        const bool xhi = (DXT == 3 || dx0 > 0) && x + 8 < n;
-#pragma unroll
-        for (int r = 0; r < DYT; ++r) {
-            const bool rowok = zok && (unsigned)(y + dy + r) < (unsigned)n;
-            const bool lo = rowok && xlo, hi = rowok && xhi;
-#pragma unroll
-            for (int u = 0; u < IT; ++u) {
-                const gh_ptr pr = px[u] + r * row_elems;
-                f.c[r][u] = load_global16(rowok ? pr : zero);
-                f.prev[r][u] = load_global4(lo ? pr - 8 * cin + 6 : zero);
-                f.next[r][u] = load_global4(hi ? pr + 8 * cin : zero);
-            }
-        }
-    };
-    // 32 voxels on: at most 32 / n <= 4 row wraps (n >= 8) and one plane
-    // wrap (n^2 >= 64), as selects -- no data-dependent loop between a
-    // step's loads and the MFMAs that wait for them
-    auto advance = [n](int &xa, int &ya, int &za) {
-        xa += 32;
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const bool w = xa >= n;
-            xa = w ? xa - n : xa;
-            ya = w ? ya + 1 : ya;
-        }
-        const bool wz = ya >= n;
-        ya = wz ? ya - n : ya;
-        za = wz ? za + 1 : za;
-    };
-    // Two step buffers, unrolled by two with fixed roles: step k + 1's
-    // loads go out before step k's MFMAs, and step k + 2's before step
-    // k + 1's, so a step's loads have a whole other step to arrive (a copy
-    // from a "next" buffer would wait for them at the end of every step).
-    // The fetch front stops at the chunk's last step, which later fetches
-    // re-load; an odd step count ends with one step of a zero A fragment
-    // (adding exact zeros), so the body has no branch.
-    const int S = (int)((v_end - v_begin) / 32);
-    int front = 0;  // step the next fetch loads
-    auto fetch_front = [&](Step &f) {
-        fetch(f);
-        const bool on = front + 1 < S;
-        int xa = x, ya = y, za = z;
-        advance(xa, ya, za);
-        front += on ? 1 : 0;
-        x = on ? xa : x;
-        y = on ? ya : y;
-        z = on ? za : z;
-#pragma unroll
-        for (int t = 0; t < CT; ++t) pa[t] += on ? step_a : 0;
-#pragma unroll
-        for (int u = 0; u < IT; ++u) px[u] += on ? step_x : 0;
-    };
-    auto compute = [&](const Step &cur, bool live) {
-        Frag a[CT];
-#pragma unroll
-        for (int t = 0; t < CT; ++t) a[t].q = live ? cur.a[t] : make_uint4(0u, 0u, 0u, 0u);
-#pragma unroll
-        for (int r = 0; r < DYT; ++r) {
-            Frag b[DXT][IT];
-#pragma unroll
-            for (int u = 0; u < IT; ++u) {
-                if (DXT == 3) {
-                    b[0][u].q = shift_from_prev(cur.c[r][u], cur.prev[r][u]);
-                    b[1 % DXT][u].q = cur.c[r][u];
-                    b[2 % DXT][u].q = shift_from_next(cur.c[r][u], cur.next[r][u]);
-                } else {
-                    b[0][u].q = dx0 == 0 ? cur.c[r][u]
-                                         : (dx0 < 0 ? shift_from_prev(cur.c[r][u], cur.prev[r][u])
-                                                    : shift_from_next(cur.c[r][u], cur.next[r][u]));
-                }
-            }
-#pragma unroll
-            for (int e = 0; e < DXT; ++e)
-#pragma unroll
-                for (int t = 0; t < CT; ++t)
-#pragma unroll
-                    for (int u = 0; u < IT; ++u)
-                        acc[r][e][t][u] =
-                            __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[t].v, b[e][u].v, acc[r][e][t][u], 0, 0, 0);
-        }
-    };
-    Step s0, s1;
-    fetch_front(s0);
-    for (int k = 0; k < S; k += 2) {
-        fetch_front(s1);  // step k + 1
-        compute(s0, true);
-        fetch_front(s0);  // step k + 2
-        compute(s1, k + 1 < S);
+    for (int p = 0; p < PERX; ++p) {
+        const int k = tid + T * p, v = k / (2 * TI), c = ci0 + 8 * (k % (2 * TI));
+        const int xx = x0 + v % kWgX - 1, yy = y0 + v / kWgX - 1;
+        xok[p] = k < PX && c < cin && (unsigned)xx < (unsigned)n && (unsigned)yy < (unsigned)n;
+        xofs[p] = xok[p] ? (yy * n + xx) * ldx + c : 0;
     }
-    // D lane layout: row (co) 4*(lane/16) + e, column (ci) lane % 16
 #pragma unroll
-    for (int r = 0; r < DYT; ++r)
+    for (int p = 0; p < PERY; ++p) {
+        const int k = tid + T * p, v = k / (2 * TO), c = co0 + 8 * (k % (2 * TO));
+        const int xx = x0 + v % 16, yy = y0 + v / 16;
+        yok[p] = k < PY && c < cout && xx < n && yy < n;
+        yofs[p] = yok[p] ? (yy * n + xx) * ldy + c : 0;
+    }
+    uint4 sx[2][PERX], sy[2][PERY];  // two planes in flight
+    auto load_x = [&](int set, int z) {
+        const bool ok = (unsigned)z < (unsigned)n;
+        const gh_ptr base = xg + (int64_t)(ok ? z : 0) * n * n * ldx;
 #pragma unroll
-        for (int d = 0; d < DXT; ++d)
+        for (int p = 0; p < PERX; ++p) {
+            Frag f;
+            f.q = load_global16(ok && xok[p] ? base + xofs[p] : zero);
+            if (IN == kInMasked) {
 #pragma unroll
-            for (int t = 0; t < CT; ++t)
+                for (int e = 0; e < 8; ++e)
+                    if (e >= cin) f.h[e] = 0;
+            }
+            sx[set][p] = f.q;
+        }
+    };
+    auto load_y = [&](int set, int z) {  // planes outside the chunk hold zeros
+        const bool ok = z >= zs && z < ze;
+        const gh_ptr base = yg + (int64_t)(ok ? z : 0) * n * n * ldy;
 #pragma unroll
-                for (int u = 0; u < IT; ++u)
+        for (int p = 0; p < PERY; ++p) sy[set][p] = load_global16(ok && yok[p] ? base + yofs[p] : zero);
+    };
+    auto store_xy = [&](int set, int buf) {
 #pragma unroll
-                    for (int e = 0; e < 4; ++e) {
-                        const int co = (cog * CT + t) * 16 + 4 * q + e;
-                        const int ci = (cig * IT + u) * 16 + i;
-                        P[((int64_t)chunk * cout + co) * Kp + (tap0 + 3 * r + d) * cin + ci] = acc[r][d][t][u][e];
-                    }
+        for (int p = 0; p < PERX; ++p) {
+            const int k = tid + T * p, v = k / (2 * TI), g = k % (2 * TI);
+            if (k < PX) xs[buf * PX + ((g >> 1) * kWgVox + v) * 2 + (g & 1)] = sx[set][p];
+        }
+#pragma unroll
+        for (int p = 0; p < PERY; ++p) {
+            const int k = tid + T * p, v = k / (2 * TO), g = k % (2 * TO);
+            if (k < PY) ys[buf * PY + ((g >> 1) * kWgOut + v) * 2 + (g & 1)] = sy[set][p];
+        }
+    };
+    // a fragment's 8 voxels: lane group q = lane / 16 takes x 4 (q & 1) .. + 3 and
+    // 8 further of row q / 2 of the step's two, the same for X and dY; lane t of
+    // the group addresses voxel t / 4, channels 4 (t % 4) .. + 3
+    const int q = lane >> 4, t = lane & 15;
+    const int xv = 4 * (q & 1) + (t >> 2), row = q >> 1;
+    typedef const char __attribute__((address_space(3))) *lc_ptr;
+    const lc_ptr xlane = (lc_ptr)(void *)xs + (ti * kWgVox + row * kWgX + xv) * 32 + (t & 3) * 8;
+    const lc_ptr ylane = (lc_ptr)(void *)ys + (to * kWgOut + row * 16 + xv) * 32 + (t & 3) * 8;
+    auto frag = [](lc_ptr p) {
+        union {
+            s16x4 s[2];
+            Frag f;
+        } u;
+        u.s[0] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((ls_ptr)p);
+        u.s[1] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((ls_ptr)(p + 8 * 32));
+        return u.f;
+    };
+
+    f32x4 acc[3][9];
+#pragma unroll
+    for (int d = 0; d < 3; ++d)
+#pragma unroll
+        for (int e = 0; e < 9; ++e) acc[d][e] = f32x4{0.f, 0.f, 0.f, 0.f};
+    Frag a[3][NKS];  // dY of planes z + 1, z, z - 1
+#pragma unroll
+    for (int d = 0; d < 3; ++d)
+#pragma unroll
+        for (int s = 0; s < NKS; ++s) a[d][s].q = make_uint4(0u, 0u, 0u, 0u);
+
+    load_x(0, zs - 1);
+    load_y(0, zs);
+    load_x(1, zs);
+    load_y(1, zs + 1);
+    store_xy(0, 0);
+    __syncthreads();
+    // step at X plane z (dY plane z + 1) in buffer PH: the planes of step z + 2 go
+    // out, those of z + 1 (in flight for a whole step) are stored after the products
+    auto plane = [&](auto ph_c, int z) __attribute__((always_inline)) {
+        constexpr int PH = decltype(ph_c)::value;
+        load_x(PH, z + 2);
+        load_y(PH, z + 3);
+#pragma unroll
+        for (int s = 0; s < NKS; ++s) {
+            const int step = ks + KS * s;  // rows 2 step, 2 step + 1
+            a[2][s] = a[1][s];
+            a[1][s] = a[0][s];
+            a[0][s] = frag(ylane + PH * PY * 16 + step * 2 * 16 * 32);
+            const lc_ptr xp = xlane + PH * PX * 16 + step * 2 * kWgX * 32;
+#pragma unroll
+            for (int e = 0; e < 9; ++e) {  // tap (dy, dx) = (e / 3 - 1, e % 3 - 1)
+                const Frag f = frag(xp + ((e / 3) * kWgX + e % 3) * 32);
+#pragma unroll
+                for (int d = 0; d < 3; ++d)
+                    acc[d][e] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[d][s].v, f.v, acc[d][e], 0, 0, 0);
+            }
+        }
+        store_xy(PH ^ 1, PH ^ 1);
+        __syncthreads();
+    };
+    int z = zs - 1;
+    for (; z + 1 <= ze; z += 2) {
+        plane(lgdhip::ic<0>{}, z);
+        plane(lgdhip::ic<1>{}, z + 1);
+    }
+    if (z <= ze) plane(lgdhip::ic<0>{}, z);
+    // sum the KS waves of each tile pair, one dz at a time: the upper half of the
+    // waves writes, the lower half adds
+    if (KS > 1) {
+        f32x4 *red = reinterpret_cast<f32x4 *>(smem);
+        const int pair = to * TI + ti;
+#pragma unroll
+        for (int d = 0; d < 3; ++d)
+#pragma unroll
+            for (int half = KS / 2; half >= 1; half /= 2) {
+                if (ks >= half && ks < 2 * half) {
+#pragma unroll
+                    for (int e = 0; e < 9; ++e) red[((pair * (KS / 2) + ks - half) * 9 + e) * 64 + lane] = acc[d][e];
+                }
+                __syncthreads();
+                if (ks < half) {
+#pragma unroll
+                    for (int e = 0; e < 9; ++e) acc[d][e] += red[((pair * (KS / 2) + ks) * 9 + e) * 64 + lane];
+                }
+                __syncthreads();
+            }
+        if (ks != 0) return;
+    }
+    // D lane layout: row (co) 4 (lane / 16) + e, column (ci) lane % 16
+    const int64_t chunk = ((int64_t)zc * by + y0 / 8) * bx + x0 / 16;
+    const int ci = ci0 + ti * 16 + t;
+    if (ci >= cin) return;
+#pragma unroll
+    for (int d = 0; d < 3; ++d)
+#pragma unroll
+        for (int k = 0; k < 9; ++k)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const int co = co0 + to * 16 + 4 * q + e;
+                if (co < cout) P[(chunk * cout + co) * Kp + (9 * d + k) * cin + ci] = acc[d][k][e];
+            }
 }
 
 // dW[co][k] = sum over chunks of P (fixed order) for k < K; the padding
 // columns k >= K stay zero
-// A work-group of 64 x 4 threads takes 64 consecutive outputs; thread row j
-// sums the chunks j, j + 4, j + 8, ... (eight loads in flight, coalesced
-// across the 64 outputs) and the four row sums are added in row order:
-// a fixed order for every output.
-constexpr int kWgradReduceOutputs = 64, kWgradReduceRows = 4;
-__global__ __launch_bounds__(256) void conv3d_wgrad_reduce(const float *__restrict__ P, int chunks, int cout, int Kp,
+// A work-group of 64 x 16 threads takes 64 consecutive outputs; thread row j
+// sums the chunks j, j + 16, j + 32, ... (eight loads in flight, coalesced
+// across the 64 outputs) and the row sums are added in row order: a fixed
+// order for every output.  (With 4 rows the 108 work-groups of a 16 -> 16
+// layer's 512 chunks took 20.5 us.)
+constexpr int kWgradReduceOutputs = 64, kWgradReduceRows = 16;
+__global__ __launch_bounds__(kWgradReduceOutputs * kWgradReduceRows) void conv3d_wgrad_reduce(const float *__restrict__ P, int chunks, int cout, int Kp,
                                                            int K, float *__restrict__ dW, int accumulate) {
     __shared__ float part[kWgradReduceRows][kWgradReduceOutputs];
     const int total = cout * Kp;  // < 2^31: cout <= 192, Kp <= 27 * 192 + 31
@@ -1247,25 +1224,9 @@ __global__ __launch_bounds__(256) void conv3d_wgrad_reduce(const float *__restri
     dW[o] = accumulate ? dW[o] + r : r;
 }
 
-// db from the voxel-blocked gradient (C channels): partial sums of each
-// channel over chunks of 8192 voxels, then a fixed-order sum of the chunks
+// db: channel sums over chunks of 8192 voxels, then a fixed-order sum of the
+// chunks
 constexpr int kBiasChunk = 8192;
-__global__ __launch_bounds__(256) void row_sum_partial(const u16 *__restrict__ Gc, int64_t nvox, float *__restrict__ Pb,
-                                                       int bchunks, int C) {
-    __shared__ float red[256];
-    const int co = blockIdx.x, c = blockIdx.y;
-    const int64_t v0 = (int64_t)c * kBiasChunk;
-    const int64_t v1 = v0 + kBiasChunk < nvox ? v0 + kBiasChunk : nvox;
-    float s = 0.0f;
-    for (int64_t v = v0 + threadIdx.x; v < v1; v += 256) s += bf2f(Gc[((((v >> 3) * C) + co) << 3) + (v & 7)]);
-    red[threadIdx.x] = s;
-    __syncthreads();
-    for (int w = 128; w > 0; w >>= 1) {
-        if ((int)threadIdx.x < w) red[threadIdx.x] += red[threadIdx.x + w];
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) Pb[co * bchunks + c] = red[0];
-}
 __global__ void row_sum_final(const float *__restrict__ Pb, int bchunks, int cout, float *__restrict__ db,
                               int accumulate) {
     const int co = blockIdx.x * blockDim.x + threadIdx.x;
@@ -1593,40 +1554,63 @@ bool vec8(const void *a, const void *b, int c, int lda, int offa, int ldb, int o
            ((uintptr_t)a & 15) == 0 && ((uintptr_t)b & 15) == 0;
 }
 
-// shapes the voxel-blocked weight gradient (conv3d_wgrad_cf) handles
-bool wgrad_cf_shape(int n, int cin, int ksize, int cout) {
-    return ksize == 3 && cin % 16 == 0 && cout % 16 == 0 && n % 8 == 0;
-}
-
-// conv3d_wgrad_cf's tiling: CT x IT tiles of 16 co x 16 ci per wave, the
-// three x taps of a row at once (DXT = 3) while the accumulators stay
-// within 48 registers, and for a single tile the three rows of a dz too
-// (DYT = 3, 36 accumulator registers)
-struct CfTiling {
-    int CT, IT, DXT, DYT, cotg, citg;
-    int tasks() const { return 27 / (DXT * DYT) * cotg * citg; }  // waves per chunk
+// Launch of conv3d_wgrad_zm: tile pairs TI x TO and KS waves per pair, channel
+// groups, z planes per chunk and chunks of the volume.
+struct ZmWgrad {
+    int ti, to, ks, gi, go, bx, by, zchunk, chunks;
+    int64_t groups() const { return (int64_t)chunks * gi * go; }
 };
-CfTiling cf_tiling(int cin, int cout) {
-    const int cot = cout / 16, cit = cin / 16;
-    CfTiling t;
-    t.CT = cot % 4 == 0 ? 4 : (cot % 2 == 0 ? 2 : 1);
-    t.IT = cit % 4 == 0 ? 4 : (cit % 2 == 0 ? 2 : 1);
-    t.cotg = cot / t.CT;
-    t.citg = cit / t.IT;
-    t.DXT = t.CT * t.IT <= 4 ? 3 : 1;
-    t.DYT = t.CT * t.IT == 1 ? 3 : 1;  // one co and one ci tile: all three rows of a dz
-    return t;
+constexpr struct {
+    int ti, to, ks;
+} kZmWgrad[] = {{1, 1, 4}, {1, 2, 4}, {2, 1, 4}, {3, 1, 4}, {2, 2, 2}, {3, 2, 1}, {2, 4, 1}, {4, 2, 1}};
+// 3x3x3 layers whose 8-channel pieces are whole (or, for the network's first
+// layer, one masked row); the partials index rows of channels with 32 bits
+bool wgrad_zm_shape(int cin, int ksize, int cout) { return ksize == 3 && (cin % 8 == 0 || cin < 8) && cout % 8 == 0; }
+ZmWgrad wgrad_zm_plan(int n, int cin, int cout) {
+    const int cit = (cin + 15) / 16, cot = (cout + 15) / 16;
+    ZmWgrad best{};
+    double best_us = 1e300;
+    for (const auto &c : kZmWgrad) {
+        if (cin < 8 && c.ti > 1) continue;  // the masked row has the one-tile kernels
+        if (cin < 8 && c.to > 2) continue;
+        ZmWgrad w{c.ti, c.to, c.ks, (cit + c.ti - 1) / c.ti, (cot + c.to - 1) / c.to, (n + 15) / 16, (n + 7) / 8, 0, 0};
+        const int waves = c.ti * c.to * c.ks, resident = waves == 4 ? 3 : 1;
+        for (int zc = 2; zc <= 64; zc *= 2) {
+            w.zchunk = zc;
+            w.chunks = w.bx * w.by * ((n + zc - 1) / zc);
+            // Modelled time (us): a plane step of the CU's resident work-groups
+            // takes its memory latency (0.7) or its products (27 MFMAs of 16
+            // cycles per wave and 32-voxel step, at 0.7 of issue), a chunk two
+            // halo planes and its start and reduction (4); the partials' round
+            // trip at 4 TB/s and the tensors' (X with its halo) at 4.5 TB/s.
+            const double on_cu = (double)((w.groups() + lgdhip::kCUs - 1) / lgdhip::kCUs);
+            const double together = std::min<double>(on_cu, resident), rounds = std::ceil(on_cu / resident);
+            const double products = std::max(1.0, together * waves / 4) * (4 / c.ks) * 27 * 16 / 2400.0 / 0.7;
+            const double march = rounds * ((zc + 2) * std::max(0.7, products) + 4.0);
+            const double partials = 2.0 * w.chunks * cout * lgdhip_conv3d_kpad(cin, 3) * 4 / 4e6;
+            const double tensors = 2.0 * n * n * n * (1.4 * (zc + 2) / zc * w.go * cin + (double)w.gi * cout) / 4.5e6;
+            const double us = std::max(march, tensors) + partials;
+            if (us < best_us) {
+                best_us = us;
+                best = w;
+            }
+        }
+    }
+    return best;
 }
 
-// Voxels per chunk when the caller leaves it to the library (chunk_vox <=
-// 0): the largest power of two <= 4096 (and >= 128) that still gives the
-// launch 2048 waves (8 per CU), since each wave marches its chunk 32 voxels
-// per dependent step.  4096 at 128^3 (16 channels: 4608 waves of 128
-// steps); the 32^3 and 16^3 levels would otherwise run 54-162 work-groups.
+// Voxels per chunk of the general kernel when the caller leaves it to the
+// library (chunk_vox <= 0): the largest power of two <= 4096 (and >= 128) that
+// still gives the launch 2048 waves (8 per CU) in its wave split, since each
+// wave marches its chunk 32 voxels per dependent step.
 int wgrad_chunk(int n, int cin, int ksize, int cout) {
     const int64_t nvox = (int64_t)n * n * n;
-    const int64_t tasks = wgrad_cf_shape(n, cin, ksize, cout) ? cf_tiling(cin, cout).tasks()
-                                                               : lgdhip_conv3d_kpad(cin, ksize) / 16;
+    int64_t tasks = lgdhip_conv3d_kpad(cin, ksize) / 16;
+    if (ksize == 3 && cin % 16 == 0 && cout % 16 == 0 && n % 8 == 0) {
+        const int cot = cout / 16, cit = cin / 16;
+        const int ct = cot % 4 == 0 ? 4 : (cot % 2 == 0 ? 2 : 1), it = cit % 4 == 0 ? 4 : (cit % 2 == 0 ? 2 : 1);
+        tasks = 27 / (ct * it <= 4 ? (ct * it == 1 ? 9 : 3) : 1) * (cot / ct) * (cit / it);
+    }
     int c = 4096;
     while (c > 128 && (nvox + c - 1) / c * tasks < 2048) c /= 2;
     return c;
@@ -1802,11 +1786,11 @@ size_t lgdhip_conv3d_wgrad_workspace_bytes(int n, int cin, int ksize, int cout, 
     if (chunk_vox <= 0) chunk_vox = wgrad_chunk(n, cin, ksize, cout);
     const int64_t nvox = (int64_t)n * n * n;
     const int64_t chunks = (nvox + chunk_vox - 1) / chunk_vox;
-    // [P: chunk partials][bias partials][x and dy voxel-blocked copies]
-    size_t bytes = (size_t)(chunks * cout * lgdhip_conv3d_kpad(cin, ksize) * 4);
-    bytes += (size_t)cout * (size_t)((nvox + kBiasChunk - 1) / kBiasChunk) * 4;
-    if (wgrad_cf_shape(n, cin, ksize, cout)) bytes += 256 + (size_t)(cin + cout) * (size_t)nvox * 2;
-    return bytes;
+    // [P: chunk partials][bias partials], for whichever kernel the tensors allow
+    int64_t partials = chunks;
+    if (wgrad_zm_shape(cin, ksize, cout)) partials = std::max<int64_t>(partials, wgrad_zm_plan(n, cin, cout).chunks);
+    return (size_t)(partials * cout * lgdhip_conv3d_kpad(cin, ksize) * 4) +
+           (size_t)cout * (size_t)((nvox + kBiasChunk - 1) / kBiasChunk) * 4;
 }
 
 int lgdhip_conv3d_bf16_wgrad(const void *x, int n, int ldx, int offx, int cin, int ksize, const void *dy, int ldy,
@@ -1829,82 +1813,59 @@ int lgdhip_conv3d_bf16_wgrad(const void *x, int n, int ldx, int offx, int cin, i
     const int chunks = (int)((nvox + chunk_vox - 1) / chunk_vox);
     hipStream_t s = lgdhip::as_stream(stream);
     float *P = (float *)workspace;
-    const bool cf = wgrad_cf_shape(n, cin, ksize, cout) && ldx % 8 == 0 && offx % 8 == 0 && ldy % 8 == 0 &&
-                    offy % 8 == 0 && (uintptr_t)x % 16 == 0 && (uintptr_t)dy % 16 == 0;
-    if (cf) {
-        // voxel-blocked copies: every MFMA fragment becomes one 16-byte load per lane
-        const int bchunks0 = (int)((nvox + kBiasChunk - 1) / kBiasChunk);
-        float *Pb = P + (size_t)chunks * cout * Kp;
-        char *base = (char *)(Pb + (size_t)cout * bchunks0);
-        base += (256 - (uintptr_t)base % 256) % 256;
-        u16 *Xc = (u16 *)base;
-        u16 *Gc = Xc + (size_t)cin * nvox;
-        to_voxel_blocked<<<dim3(blocks_for(nvox), cin / 8), 256, 0, s>>>((const u16 *)x, nvox, ldx, offx, cin, Xc);
-        to_voxel_blocked<<<dim3(blocks_for(nvox), cout / 8), 256, 0, s>>>((const u16 *)dy, nvox, ldy, offy, cout, Gc);
-        LGD_LAUNCHED("to_voxel_blocked");
-        const CfTiling tl = cf_tiling(cin, cout);
-        const int CT = tl.CT, IT = tl.IT, DXT = tl.DXT, DYT = tl.DYT, cotg = tl.cotg, citg = tl.citg;
-        const int64_t waves = (int64_t)chunks * tl.tasks();
+    int parts = chunks;
+    const bool zm = wgrad_zm_shape(cin, ksize, cout) && ldx % 8 == 0 && offx % 8 == 0 && ldy % 8 == 0 &&
+                    offy % 8 == 0 && (cin >= 8 || offx + 8 <= ldx) && (uintptr_t)x % 16 == 0 &&
+                    (uintptr_t)dy % 16 == 0 && (int64_t)n * n * std::max(ldx, ldy) < INT32_MAX;
+    if (zm) {
+        const ZmWgrad w = wgrad_zm_plan(n, cin, cout);
+        parts = w.chunks;
+        const unsigned groups = (unsigned)w.groups(), per = lgdhip::xcd_per(groups);
+#define LGD_ZW_CASE(TI, TO, KS, IN)                                                                            \
+    if (w.ti == TI && w.to == TO && w.ks == KS && (cin < 8) == (IN == kInMasked))                              \
+        conv3d_wgrad_zm<TI, TO, KS, IN><<<lgdhip::xcd_groups(groups), 64 * TI * TO * KS, 0, s>>>(              \
+            (const u16 *)x, n, ldx, offx, cin, (const u16 *)dy, ldy, offy, cout, Kp, w.zchunk, w.bx, w.by,     \
+            w.gi, w.go, P, groups, per);
+        LGD_ZW_CASE(1, 1, 4, kInVec) LGD_ZW_CASE(1, 2, 4, kInVec) LGD_ZW_CASE(2, 1, 4, kInVec)
+        LGD_ZW_CASE(3, 1, 4, kInVec) LGD_ZW_CASE(2, 2, 2, kInVec) LGD_ZW_CASE(3, 2, 1, kInVec)
+        LGD_ZW_CASE(2, 4, 1, kInVec) LGD_ZW_CASE(4, 2, 1, kInVec)
+        LGD_ZW_CASE(1, 1, 4, kInMasked) LGD_ZW_CASE(1, 2, 4, kInMasked)
+#undef LGD_ZW_CASE
+        LGD_LAUNCHED("conv3d_wgrad_zm");
+    } else {
+        const int64_t waves = (int64_t)chunks * (Kp / 16);
         const unsigned wgs = (unsigned)((waves + 3) / 4);
         const unsigned per = lgdhip::xcd_per(wgs), grid = lgdhip::xcd_groups(wgs);
-#define LGD_CF_CASE(A, B, D, R)                                                                              \
-    if (CT == A && IT == B && DXT == D && DYT == R)                                                          \
-        conv3d_wgrad_cf<A, B, D, R><<<grid, 256, 0, s>>>(Xc, Gc, n, cin, cout, Kp, chunk_vox, cotg, citg, P, per);
-        LGD_CF_CASE(1, 1, 3, 3)
-        LGD_CF_CASE(1, 2, 3, 1)
-        LGD_CF_CASE(1, 4, 3, 1)
-        LGD_CF_CASE(2, 1, 3, 1)
-        LGD_CF_CASE(2, 2, 3, 1)
-        LGD_CF_CASE(2, 4, 1, 1)
-        LGD_CF_CASE(4, 1, 3, 1)
-        LGD_CF_CASE(4, 2, 1, 1)
-        LGD_CF_CASE(4, 4, 1, 1)
-#undef LGD_CF_CASE
-        LGD_LAUNCHED("conv3d_wgrad_cf");
-        conv3d_wgrad_reduce<<<(unsigned)((cout * Kp + kWgradReduceOutputs - 1) / kWgradReduceOutputs),
-                              dim3(kWgradReduceOutputs, kWgradReduceRows), 0, s>>>(P, chunks, cout, Kp, K, dw,
-                                                                                    accumulate);
-        LGD_LAUNCHED("conv3d_wgrad_reduce");
-        if (db) {
-            const int bchunks = (int)((nvox + kBiasChunk - 1) / kBiasChunk);
-            row_sum_partial<<<dim3(cout, bchunks), 256, 0, s>>>(Gc, nvox, Pb, bchunks, cout);
-            row_sum_final<<<blocks_for(cout), 256, 0, s>>>(Pb, bchunks, cout, db, accumulate);
-            LGD_LAUNCHED("row_sum");
-        }
-        return 0;
-    }
-    const int64_t waves = (int64_t)chunks * (Kp / 16);
-    const unsigned wgs = (unsigned)((waves + 3) / 4);
-    const unsigned per = lgdhip::xcd_per(wgs), grid = lgdhip::xcd_groups(wgs);
-    const int nt = (cout + 15) / 16;
+        const int nt = (cout + 15) / 16;
 #define LGD_WG_CASE(T)                                                                                       \
     case T:                                                                                                  \
         conv3d_wgrad_mfma<T><<<grid, 256, 0, s>>>((const u16 *)x, n, ldx, offx, cin, ksize, (const u16 *)dy, \
                                                   ldy, offy, cout, Kp, chunk_vox, P, per);                   \
         break;
-    switch (nt) {
-        LGD_WG_CASE(1)
-        LGD_WG_CASE(2)
-        LGD_WG_CASE(3)
-        LGD_WG_CASE(4)
-        LGD_WG_CASE(5)
-        LGD_WG_CASE(6)
-        LGD_WG_CASE(7)
-        LGD_WG_CASE(8)
-        LGD_WG_CASE(9)
-        LGD_WG_CASE(10)
-        LGD_WG_CASE(11)
-        LGD_WG_CASE(12)
-    }
+        switch (nt) {
+            LGD_WG_CASE(1)
+            LGD_WG_CASE(2)
+            LGD_WG_CASE(3)
+            LGD_WG_CASE(4)
+            LGD_WG_CASE(5)
+            LGD_WG_CASE(6)
+            LGD_WG_CASE(7)
+            LGD_WG_CASE(8)
+            LGD_WG_CASE(9)
+            LGD_WG_CASE(10)
+            LGD_WG_CASE(11)
+            LGD_WG_CASE(12)
+        }
 #undef LGD_WG_CASE
-    LGD_LAUNCHED("conv3d_wgrad_mfma");
+        LGD_LAUNCHED("conv3d_wgrad_mfma");
+    }
     conv3d_wgrad_reduce<<<(unsigned)((cout * Kp + kWgradReduceOutputs - 1) / kWgradReduceOutputs),
-                              dim3(kWgradReduceOutputs, kWgradReduceRows), 0, s>>>(P, chunks, cout, Kp, K, dw,
+                              dim3(kWgradReduceOutputs, kWgradReduceRows), 0, s>>>(P, parts, cout, Kp, K, dw,
                                                                                     accumulate);
     LGD_LAUNCHED("conv3d_wgrad_reduce");
     if (db) {
         const int bchunks = (int)((nvox + kBiasChunk - 1) / kBiasChunk);
-        float *Pb = P + (size_t)chunks * cout * Kp;
+        float *Pb = P + (size_t)parts * cout * Kp;
         bias_grad_partial<<<bchunks, 256, 0, s>>>((const u16 *)dy, nvox, ldy, offy, cout, Pb, bchunks);
         row_sum_final<<<blocks_for(cout), 256, 0, s>>>(Pb, bchunks, cout, db, accumulate);
         LGD_LAUNCHED("bias_grad");

@@ -352,9 +352,8 @@ def test_conv_dgrad_vs_oracle(hip, oracle, n, cin, cout):
                                               (8, 192, 128, 3), (8, 32, 16, 3), (8, 64, 16, 3),
                                               (8, 16, 32, 3), (8, 32, 32, 3), (8, 16, 64, 3)])
 def test_conv_wgrad_vs_oracle(hip, oracle, n, cin, cout, ksize):
-    """Element-gather kernel (odd channel counts, 1x1x1, n % 8 != 0) and the
-    voxel-blocked kernel (3x3x3, channels multiples of 16, n % 8 == 0, every
-    tile grouping CT x IT in {1, 2, 4}^2 reached by some case)."""
+    """Element-gather kernel (odd channel counts, 1x1x1) and the column kernel
+    (3x3x3, channels multiples of 8) on small volumes."""
     run_wgrad_case(hip, oracle, n, cin, cout, ksize, 256)
 
 
@@ -404,6 +403,43 @@ def run_wgrad_case(hip, oracle, n, cin, cout, ksize, chunk):
     assert np.all(out[:, taps * cin:] == 0)
     assert np.all(np.abs(got - ref) <= (n ** 3 + 64) * 2.0 ** -24 * mag + 1e-30)
     assert np.allclose(outb, refb, rtol=1e-5, atol=1e-3)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,cin,cout", [(17, 16, 16), (13, 24, 40), (33, 3, 16), (20, 3, 48), (31, 64, 128), (53, 192, 48),
+                                        (30, 96, 128), (35, 64, 128), (45, 48, 128), (47, 64, 128), (68, 64, 96),
+                                        (1, 16, 16)])
+def test_conv_wgrad_columns_vs_gather(hip, n, cin, cout):
+    """The column kernel (every tile grouping, ragged columns and z chunks,
+    channel counts that fill half a tile, one masked row) against the gather
+    kernel, which the same values in rows of an odd stride take, with a second
+    call accumulating."""
+    print("[case] conv wgrad columns", n, cin, cout, flush=True)
+    rng = np.random.default_rng(n * cin + cout)
+    x = rng.standard_normal((n ** 3, cin)).astype(np.float32)
+    g = rng.standard_normal((n ** 3, cout)).astype(np.float32)
+    lib = hip.load()
+    kp = lib.lgdhip_conv3d_kpad(cin, 3)
+    wsb = lib.lgdhip_conv3d_wgrad_workspace_bytes(n, cin, 3, cout, 0)
+    ws, dw = hip.DeviceBuffer(wsb), hip.DeviceBuffer(cout * kp * 4)
+
+    def run(x, g, ldx, calls=1):
+        xs = np.full((n ** 3, ldx), 7.0, np.float32)  # channels past cin are another tensor's
+        xs[:, :cin] = x
+        xb, gb = dev(hip, to_bf16_bits(xs)), dev(hip, to_bf16_bits(g))
+        for k in range(calls):
+            hip.call("lgdhip_conv3d_bf16_wgrad", xb.ptr, n, ldx, 0, cin, 3, gb.ptr, cout, 0, cout, dw.ptr, None, k, 0,
+                     ws.ptr, wsb, None)
+        out = np.empty((cout, kp), np.float32)
+        dw.download(out)
+        return out
+
+    got, ref = run(x, g, max(cin, 8)), run(x, g, cin | 1 if cin % 2 == 0 else cin + 2)
+    mag = run(np.abs(x), np.abs(g), cin | 1 if cin % 2 == 0 else cin + 2)
+    assert np.all(np.abs(got - ref) <= 2 * (n ** 3 + 64) * 2.0 ** -24 * mag + 1e-30)
+    assert np.all(got[:, 27 * cin:] == 0)
+    twice = run(x, g, max(cin, 8), calls=2)
+    assert np.array_equal(twice, got + got)
 
 
 @pytest.mark.gpu
