@@ -525,6 +525,11 @@ int lgdhip_upsample2_concat_bf16(const void *x, int m, int ldx, int offx, int cu
                                  int offs, int cs, void *y, int ldy, int offy, lgdhip_stream_t stream);
 /* FP32 field -> one BF16 channel of a channels-last tensor */
 int lgdhip_pack_bf16(const float *src, int64_t nvox, void *y, int ldy, int offy, lgdhip_stream_t stream);
+/* `count` (<= 8) FP32 fields (a host array of device pointers) -> channels
+ * 0 .. count-1 of y's rows, channels count .. 7 zero; rows 16-byte aligned, ldy
+ * a multiple of 8.  No counterpart in the reference. */
+int lgdhip_pack_rows_bf16(const float *const *src, int count, int64_t nvox, void *y, int ldy,
+                          lgdhip_stream_t stream);
 /* MSE: grad[v*ldg] = 2 (pred - target) / nvox (BF16), partial[b] = per-block
  * sums of squared errors (lgdhip_mse_partials(nvox) entries) */
 int64_t lgdhip_mse_partials(int64_t nvox);

@@ -810,6 +810,64 @@ __global__ __launch_bounds__(256) void conv1x1_to1(const u16 *__restrict__ X, in
     if (Y32) Y32[v * ld32] = o;
 }
 
+// 1x1x1 convolution of a single input channel (the output layer's input
+// gradient): y[v][co] = x[v] w[co], 8 output channels per thread.  One product
+// each, so the same values as an MFMA tile with 31 zero products, which took
+// 52 us at 128^3 x 16 for one pass over 71 MB.  W rows are Kp apart.
+__global__ __launch_bounds__(256) void conv1x1_from1(const u16 *__restrict__ X, uint32_t items, int ldx, int offx,
+                                                     const u16 *__restrict__ W, int Kp,
+                                                     const float *__restrict__ bias, int c8, u16 *__restrict__ Y,
+                                                     int ldy, int offy, int relu) {
+    const uint32_t i = blockIdx.x * 256u + threadIdx.x;
+    if (i >= items) return;
+    const uint32_t v = i / (uint32_t)c8;
+    const int co = 8 * (int)(i - v * (uint32_t)c8);
+    const float xv = bf2f(X[(int64_t)v * ldx + offx]);
+    Frag f;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+        float o = xv * bf2f(W[(int64_t)(co + e) * Kp]) + (bias ? bias[co + e] : 0.0f);
+        if (relu) o = o > 0.0f ? o : 0.0f;
+        f.h[e] = f2bf(o);
+    }
+    *reinterpret_cast<uint4 *>(Y + (int64_t)v * ldy + offy + co) = f.q;
+}
+
+// Weight gradient of a 1x1x1 layer with one output channel: P[chunk][ci] = sum
+// over the chunk's voxels of dY[v] X[v][ci].  Thread (lane, piece) sums 8
+// channels of every (256 / c8)-th voxel in FP32; the lanes' sums are added in a
+// fixed tree.  One pass over X (an MFMA tile of 16 output channels with element
+// gathers took 77 us at 128^3 x 16).
+__global__ __launch_bounds__(256) void conv1x1_to1_wgrad(const u16 *__restrict__ X, int64_t nvox, int ldx, int offx,
+                                                         const u16 *__restrict__ dY, int ldy, int offy, int c8,
+                                                         int Kp, int chunk_vox, float *__restrict__ P) {
+    __shared__ float red[256][9];
+    const int t = threadIdx.x, lanes = 256 / c8;  // c8 a power of two
+    const int piece = t % c8, lane = t / c8;
+    const int64_t v0 = (int64_t)blockIdx.x * chunk_vox;
+    const int64_t v1 = v0 + chunk_vox < nvox ? v0 + chunk_vox : nvox;
+    float s[8] = {};
+    for (int64_t v = v0 + lane; v < v1; v += lanes) {
+        Frag f;
+        f.q = *reinterpret_cast<const uint4 *>(X + v * ldx + offx + 8 * piece);
+        const float g = bf2f(dY[v * ldy + offy]);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) s[e] += g * bf2f(f.h[e]);
+    }
+#pragma unroll
+    for (int e = 0; e < 8; ++e) red[t][e] = s[e];
+    __syncthreads();
+    for (int w = lanes / 2; w > 0; w >>= 1) {
+        if (lane < w) {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) red[t][e] += red[t + w * c8][e];
+        }
+        __syncthreads();
+    }
+    // the row of Kp weights: 8 c8 channels, the rest zero
+    if (t < Kp) P[(int64_t)blockIdx.x * Kp + t] = t < 8 * c8 ? red[t / 8][t % 8] : 0.0f;
+}
+
 // the LDS-staged kernel takes 3x3x3 layers with up to 32 output channels on
 // volumes of at least 16^3
 constexpr int kLdsMinN = 16;
@@ -1361,6 +1419,27 @@ struct alignas(16) Bf8 {
 __device__ __forceinline__ Bf8 ld8(const u16 *p) { return *reinterpret_cast<const Bf8 *>(p); }
 __device__ __forceinline__ void st8(u16 *p, const Bf8 &v) { *reinterpret_cast<Bf8 *>(p) = v; }
 
+// g *= (y > 0), 8 channels per thread; items = voxels * c8 < 2^31.  Dense
+// tensors (c8 0: both strides the channel count) need no division.  At 128^3 x
+// 16 channels one element per thread with a 64-bit division took 74 us.
+__global__ void relu_backward_v8(u16 *__restrict__ g, int ldg, int offg, const u16 *__restrict__ y, int ldy, int offy,
+                                 int c8, uint32_t items) {
+    const uint32_t i = blockIdx.x * 256u + threadIdx.x;
+    if (i >= items) return;
+    int64_t ig = (int64_t)i * 8, iy = ig;
+    if (c8 > 0) {
+        const uint32_t v = i / (uint32_t)c8, ch = 8 * (i - v * (uint32_t)c8);
+        ig = (int64_t)v * ldg + offg + ch;
+        iy = (int64_t)v * ldy + offy + ch;
+    }
+    const Bf8 a = ld8(y + iy);
+    Bf8 o = ld8(g + ig);
+#pragma unroll
+    for (int k = 0; k < 8; ++k)
+        if (!(bf2f(a.h[k]) > 0.0f)) o.h[k] = 0;
+    st8(g + ig, o);
+}
+
 // Thread coordinates of the 8-channel resampling kernels over a w^3 volume:
 // a launch row_grid(w, c8) gives each (y, z) row blockIdx.y / .z, and the
 // threads along x cover its (x, channel chunk) pairs, the chunk fastest
@@ -1497,6 +1576,21 @@ __global__ void upsample2_backward_v8(const u16 *__restrict__ dY, int m, int ldy
 __global__ void pack_bf16(const float *__restrict__ src, int64_t nvox, u16 *Y, int ldy, int offy) {
     const int64_t v = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (v < nvox) Y[v * ldy + offy] = f2bf(src[v]);
+}
+
+// up to 8 FP32 fields -> whole 8-channel rows, the channels past them zero (a
+// fill and one pass per field, each writing 2 of every 16 bytes, took 47 us at
+// 128^3 with three fields)
+struct PackFields {
+    const float *f[8];
+};
+__global__ void pack_rows_bf16(PackFields src, int count, int64_t nvox, u16 *__restrict__ Y, int ldy) {
+    const int64_t v = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (v >= nvox) return;
+    Bf8 o;
+#pragma unroll
+    for (int k = 0; k < 8; ++k) o.h[k] = k < count ? f2bf(src.f[k][v]) : (u16)0;
+    st8(Y + v * ldy, o);
 }
 
 // MSE loss: L = mean((pred - target)^2); grad = 2 (pred - target) / N as BF16;
@@ -1674,6 +1768,14 @@ int lgdhip_conv3d_bf16_forward_ws(const void *x, int n, int ldx, int offx, int c
         LGD_LAUNCHED("conv1x1_to1");
         return 0;
     }
+    if (ksize == 1 && cin == 1 && cout % 8 == 0 && y && !y32 && !accumulate && (ldy & 7) == 0 && (offy & 7) == 0 &&
+        ((uintptr_t)y & 15) == 0 && nvox * (cout / 8) < INT32_MAX) {
+        const uint32_t items = (uint32_t)(nvox * (cout / 8));
+        conv1x1_from1<<<(unsigned)((items + 255u) / 256u), 256, 0, s>>>(X, items, ldx, offx, Wb, Kp, bias, cout / 8, Y,
+                                                                      ldy, offy, relu);
+        LGD_LAUNCHED("conv1x1_from1");
+        return 0;
+    }
     // z-marching kernel: 16 output channels written as plain BF16 into an
     // aligned slice, input of at most 6 groups of 8 channels (or a masked
     // row of fewer than 8).  Wider outputs on volumes of at least
@@ -1832,6 +1934,11 @@ int lgdhip_conv3d_bf16_wgrad(const void *x, int n, int ldx, int offx, int cin, i
         LGD_ZW_CASE(1, 1, 4, kInMasked) LGD_ZW_CASE(1, 2, 4, kInMasked)
 #undef LGD_ZW_CASE
         LGD_LAUNCHED("conv3d_wgrad_zm");
+    } else if (ksize == 1 && cout == 1 && cin % 8 == 0 && (cin & (cin - 1)) == 0 && ldx % 8 == 0 && offx % 8 == 0 &&
+               (uintptr_t)x % 16 == 0 && cin <= 192) {
+        conv1x1_to1_wgrad<<<(unsigned)chunks, 256, 0, s>>>((const u16 *)x, nvox, ldx, offx, (const u16 *)dy, ldy, offy,
+                                                           cin / 8, Kp, chunk_vox, P);
+        LGD_LAUNCHED("conv1x1_to1_wgrad");
     } else {
         const int64_t waves = (int64_t)chunks * (Kp / 16);
         const unsigned wgs = (unsigned)((waves + 3) / 4);
@@ -1887,6 +1994,14 @@ int lgdhip_conv3d_dgrad_weights(const void *w, int cin, int cout, int ksize, voi
 int lgdhip_relu_backward_bf16(void *g, int ldg, int offg, const void *y, int ldy, int offy, int c, int64_t nvox,
                               lgdhip_stream_t stream) {
     LGD_REQUIRE(g && y && c > 0 && nvox > 0, "bad arguments");
+    if (vec8(g, y, c, ldg, offg, ldy, offy) && nvox * (c / 8) < INT32_MAX) {
+        const bool dense = ldg == c && ldy == c && offg == 0 && offy == 0;
+        const uint32_t items = (uint32_t)(nvox * (c / 8));
+        relu_backward_v8<<<blocks_for(items), 256, 0, lgdhip::as_stream(stream)>>>(
+            (u16 *)g, ldg, offg, (const u16 *)y, ldy, offy, dense ? 0 : c / 8, items);
+        LGD_LAUNCHED("relu_backward_v8");
+        return 0;
+    }
     relu_backward<<<blocks_for(nvox * c), 256, 0, lgdhip::as_stream(stream)>>>((u16 *)g, ldg, offg, (const u16 *)y,
                                                                                ldy, offy, c, nvox);
     LGD_LAUNCHED("relu_backward");
@@ -1975,6 +2090,19 @@ int lgdhip_pack_bf16(const float *src, int64_t nvox, void *y, int ldy, int offy,
     LGD_REQUIRE(src && y && nvox > 0, "bad arguments");
     pack_bf16<<<blocks_for(nvox), 256, 0, lgdhip::as_stream(stream)>>>(src, nvox, (u16 *)y, ldy, offy);
     LGD_LAUNCHED("pack_bf16");
+    return 0;
+}
+
+int lgdhip_pack_rows_bf16(const float *const *src, int count, int64_t nvox, void *y, int ldy, lgdhip_stream_t stream) {
+    LGD_REQUIRE(src && y && nvox > 0 && count >= 1 && count <= 8, "bad arguments");
+    LGD_REQUIRE(ldy >= 8 && ldy % 8 == 0 && ((uintptr_t)y & 15) == 0, "rows must be 16-byte aligned, ldy a multiple of 8");
+    PackFields f{};
+    for (int k = 0; k < count; ++k) {
+        LGD_REQUIRE(src[k], "NULL pointer");
+        f.f[k] = src[k];
+    }
+    pack_rows_bf16<<<blocks_for(nvox), 256, 0, lgdhip::as_stream(stream)>>>(f, count, nvox, (u16 *)y, ldy);
+    LGD_LAUNCHED("pack_rows_bf16");
     return 0;
 }
 

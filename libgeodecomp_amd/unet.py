@@ -216,9 +216,11 @@ class UNet3D:
 
     def load_input(self, fields: list):
         """fields: FP32 device buffers (n^3 each) -> input tensor channels."""
-        self.x.zero(self.stream)
-        for c, buf in enumerate(fields):
-            lgdhip.call("lgdhip_pack_bf16", buf.ptr, self.n ** 3, self.x.ptr, self.x.ld, c, self.stream)
+        if not fields:
+            self.x.zero(self.stream)
+            return
+        src = (C.c_void_p * len(fields))(*[getattr(buf.ptr, "value", buf.ptr) for buf in fields])
+        lgdhip.call("lgdhip_pack_rows_bf16", src, len(fields), self.n ** 3, self.x.ptr, self.x.ld, self.stream)
 
     def forward(self):
         c0, c1, c2, c3 = self.ch

@@ -566,6 +566,79 @@ def test_upsample_concat(hip, cu, cs, ldx, offx, lds, offs, ldy, offy):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("c,ldg,offg,ldy,offy", [(16, 16, 0, 16, 0), (24, 40, 8, 32, 0), (8, 8, 0, 8, 0), (3, 5, 1, 3, 0),
+                                                 (16, 17, 0, 16, 0)])
+def test_relu_backward_rows(hip, c, ldg, offg, ldy, offy):
+    """Dense and strided rows by 16-byte pieces, odd channel counts and strides
+    by elements; zeros, negative zero and NaN masks; the channels beside the
+    range stay as they are."""
+    nvox = 777
+    rng = np.random.default_rng(c + ldg)
+    g = to_bf16_bits(rng.standard_normal((nvox, ldg)))
+    y = rng.standard_normal((nvox, ldy)).astype(np.float32)
+    y[::7] = 0.0
+    y[::11] = -0.0
+    y[::13] = np.nan
+    yb = to_bf16_bits(np.nan_to_num(y, nan=1.0))
+    yb[::13] = 0x7FC0
+    gb, db = dev(hip, g), dev(hip, yb)
+    hip.call("lgdhip_relu_backward_bf16", gb.ptr, ldg, offg, db.ptr, ldy, offy, c, nvox, None)
+    out = np.empty_like(g)
+    gb.download(out)
+    exp = g.copy()
+    keep = from_bf16_bits(yb)[:, offy:offy + c] > 0
+    exp[:, offg:offg + c] = np.where(keep, exp[:, offg:offg + c], 0)
+    assert np.array_equal(out, exp)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("count,ld", [(1, 8), (3, 8), (8, 16)])
+def test_pack_rows(hip, count, ld):
+    """Whole rows from separate fields: BF16 values, zeros past them, nothing
+    written past the eighth channel."""
+    nvox = 1000
+    rng = np.random.default_rng(count)
+    f = [rng.standard_normal(nvox).astype(np.float32) for _ in range(count)]
+    bufs = [dev(hip, v) for v in f]
+    y = dev(hip, np.full((nvox, ld), 0x1234, np.uint16))
+    src = (C.c_void_p * count)(*[b.ptr.value for b in bufs])
+    hip.call("lgdhip_pack_rows_bf16", src, count, nvox, y.ptr, ld, None)
+    out = np.empty((nvox, ld), np.uint16)
+    y.download(out)
+    exp = np.full((nvox, ld), 0x1234, np.uint16)
+    exp[:, :8] = 0
+    for k in range(count):
+        exp[:, k] = to_bf16_bits(f[k])
+    assert np.array_equal(out, exp)
+    assert hip.load().lgdhip_pack_rows_bf16(src, 9, nvox, y.ptr, ld, None) == -1
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,cout,relu", [(9, 16, 0), (5, 40, 1)])
+def test_conv_from_one_channel(hip, n, cout, relu):
+    """1x1x1 convolution of one channel: each value one rounded product (plus
+    bias), so exact."""
+    rng = np.random.default_rng(n)
+    x = bf16_round(rng.standard_normal((n ** 3, 3)).astype(np.float32))
+    w = bf16_round(rng.standard_normal((cout, 1)).astype(np.float32))
+    b = rng.standard_normal(cout).astype(np.float32)
+    kp = hip.load().lgdhip_conv3d_kpad(1, 1)
+    wp = np.zeros((cout, kp), np.uint16)
+    wp[:, :1] = to_bf16_bits(w)
+    xb, wb, bb = dev(hip, to_bf16_bits(x)), dev(hip, wp), dev(hip, b)
+    for bias in (None, bb.ptr):
+        y = dev(hip, np.zeros((n ** 3, cout + 8), np.uint16))
+        hip.call("lgdhip_conv3d_bf16_forward", xb.ptr, n, 3, 1, 1, 1, wb.ptr, bias, cout, y.ptr, cout + 8, 8, None, 1,
+                 relu, 0, None)
+        out = np.empty((n ** 3, cout + 8), np.uint16)
+        y.download(out)
+        # the product of two BF16 values is exact in FP32
+        exp = x[:, 1:2] * w[:, 0] + (b if bias is not None else np.float32(0))
+        exp = np.maximum(exp, 0) if relu else exp
+        assert np.array_equal(from_bf16_bits(out[:, 8:]), bf16_round(exp)) and np.all(out[:, :8] == 0)
+
+
+@pytest.mark.gpu
 def test_relu_mse_adam(hip):
     rng = np.random.default_rng(4)
     n, c = 8, 16
