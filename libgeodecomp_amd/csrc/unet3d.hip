@@ -219,9 +219,16 @@ __device__ __align__(16) const unsigned int kZero16[4] = {0u, 0u, 0u, 0u};
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 typedef const u32x4 __attribute__((address_space(1))) *gq_ptr;
 typedef const u16 __attribute__((address_space(1))) *gh_ptr;
+typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
+typedef const u32x2 __attribute__((address_space(1))) *gd_ptr;
 __device__ __forceinline__ uint4 load_global16(gh_ptr p) {
     const u32x4 v = *(gq_ptr)p;
     return make_uint4(v.x, v.y, v.z, v.w);
+}
+
+__device__ __forceinline__ uint2 load_global8(gh_ptr p) {
+    const u32x2 v = *(gd_ptr)p;
+    return make_uint2(v.x, v.y);
 }
 
 // IN: how the input is staged -- kInVec, 16-byte loads (cin % 8 == 0);
@@ -446,38 +453,74 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     }
 }
 
-// Z-marching LDS convolution for 3x3x3 layers with up to 16 output channels
-// and cin = 8 G input channels (G <= 6; G = 1 also takes cin < 8 rows, see
-// IN).  A work-group owns a 16 x 8 column of output voxels and marches z
-// over a chunk of ZC planes.  Input planes (18 x 10 voxels with their halo,
-// all cin channels) pass through a ring of 4 LDS slots: output plane z reads
-// input planes z-1, z, z+1 while plane z+2, loaded into registers one step
-// earlier, is written into the fourth slot -- every input voxel is fetched
-// once per column, whole channel rows together (the tile kernel above takes
-// the channels 8 at a time, re-reading each voxel's row G times).  The G x 7
-// weight fragments of the lane stay in registers for the whole march; wave w
-// computes output rows y0 + 2w and y0 + 2w + 1 of each plane.  The output
-// plane goes out through LDS as 16-byte stores one step later.  k order as
-// conv3d_fwd_lds (group-major, then tap).
-constexpr int kZmChunk = 32;  // output planes per work-group (16: forward 731 us, 32: 705 us at 128^3; 8: 782 us)
+// Z-marching LDS convolution for 3x3x3 layers with cin = 8 G input channels (G
+// <= 6; G = 1 also takes cin < 8 rows, see IN) and slices of NT x 16 output
+// channels.  A work-group owns a 16 x 8 column of output voxels and one slice and
+// marches z over a chunk of planes.  Input planes (18 x 10 voxels with their
+// halo, all cin channels) pass through a ring of 4 LDS slots: output plane z
+// reads input planes z-1, z, z+1 while plane z+2 is written into the fourth
+// slot; up to two planes' loads are in flight in registers, so a load has a whole
+// step to arrive.  Every input voxel is fetched once per column and slice, whole
+// channel rows together (the tile kernel above takes the channels 8 at a time,
+// re-reading each voxel's row G times).  Wave w computes output rows y0 + 2w and
+// y0 + 2w + 1 of each plane.  The G x 7 x NT weight fragments of the lane stay in
+// registers for the whole march; a plane step is bound by the LDS reads of the
+// input fragments, so each feeds NT products.  Work-groups run in XCD order,
+// slices of a column together: neighbouring columns' halos come from one L2.
+//
+// The k order is that of the kernel that takes the layer when this one does not
+// (accumulation, unaligned rows), so a layer's result has the same bits either
+// way.  SPLIT = 0: conv3d_fwd_lds's, group-major, 4 taps of one group per step.
+// SPLIT = 1: conv3d_fwd_gemm's, the weights' tap-major rows, 4 groups (of one
+// tap or two) per step.  SPLIT = 2: the same in conv3d_fwd_gemm's two slices of
+// its stages, each summed from zero and then added.
+//
+// Measured (us; the launch this one replaces in brackets: one 16-channel slice
+// per launch with the outputs re-tiled in LDS; the GEMM-tiled kernel and its
+// reduction; the LDS-tile kernel): 128^3 16 -> 16 41 [48], 3 -> 16 36 [47], 48 ->
+// 16 114 [127], 16 -> 48 102 [147], 32 -> 32 115 [145]; 100^3 64 -> 16 168 [tile
+// 237]; 64^3 32 -> 96 54 [GEMM 143], 64 -> 64 92 [GEMM 124], 32 -> 32 21.5 [tile
+// 24.6]; 60^3 16 -> 16 11 [34], 32 -> 32 20 [GEMM 67], 48 -> 32 33 [GEMM 89]; 32^3
+// 32 -> 64 9.5 [GEMM 25], 64 -> 64 21 [GEMM 31]; 16^3 16 -> 16 6 [18].
+// work-groups per CU (and waves per SIMD), by registers and, from 7 groups on, LDS
+constexpr int zm_waves(int g, int nt) { return g * nt <= 2 ? 3 : (g * nt <= 6 ? 2 : 1); }
+// planes in flight: one where the weight fragments leave no registers for two
+constexpr int zm_ahead(int g, int nt) { return g * nt == 5 || g * nt == 6 ? 1 : 2; }
+// k steps of 32, and the one a SPLIT = 2 launch's second slice begins with
+constexpr int zm_steps(int g, int split) { return split ? (27 * g + 3) / 4 : 7 * g; }
+constexpr int zm_second(int g) { return (zm_steps(g, 2) + 1) / 2 / 2 * 2; }
+// fragment reads in flight (at 6 groups the weights leave room for three: 48 ->
+// 16 at 128^3 133 us with six, 115 with three)
+constexpr int zm_reads(int g) { return g == 6 ? 3 : 6; }
 
-template <int G, int IN>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void conv3d_fwd_zm(
-    const u16 *__restrict__ X, int n, int ldx, int offx, int cin, const u16 *__restrict__ W, int Kp,
-    const float *__restrict__ bias, int cout, u16 *Y, int ldy, int offy, int relu, int bx, int by) {
+template <int G, int IN, int NT, int SPLIT>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(zm_waves(G, NT), zm_waves(G, NT)))) void
+conv3d_fwd_zm(const u16 *__restrict__ X, int n, int ldx, int offx, int cin, const u16 *__restrict__ W, int Kp,
+              const float *__restrict__ bias, u16 *Y, int ldy, int offy, float *Y32, int ld32, int relu,
+              int bx, int by, int slices, int zchunk, unsigned groups, unsigned per) {
     constexpr int SX = 18, SY = 10, PV = SX * SY;  // staged voxels per plane
     constexpr int CHUNKS = PV * G;                 // 16-byte pieces per plane
     constexpr int PER = (CHUNKS + 255) / 256;
-    __shared__ uint4 ring[4][CHUNKS];               // [slot][group][voxel]
-    __shared__ u16 oplane[2][8 * 16 * 16];          // [y][x][channel] of an output plane
+    constexpr int OC = 16 * NT;  // output channels of the slice
+    // [slot][group][voxel]; tap-major steps read up to 4 groups at one voxel
+    // offset, 256 bytes apart modulo the banks where the groups' stride is padded
+    // (60^3 32 -> 32 21.4 us unpadded, 20.0 padded, 48 -> 32 36.7 and 32.8; from 7
+    // groups on the staging writes conflict instead and it lost 5 %)
+    constexpr int PS = SPLIT && G <= 6 ? (PV + 15) / 16 * 16 : PV;
+    __shared__ uint4 ring[4][PS * G];
+    unsigned b = lgdhip::xcd_tile(blockIdx.x, per, true);
+    if (b >= groups) return;  // whole work-group, before any barrier
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int i = lane & 15, q = lane >> 4;
-    int b = blockIdx.x;
-    const int x0 = (b % bx) * 16;
+    const int slice = (int)(b % slices);
+    b /= slices;
+    const int x0 = (int)(b % bx) * 16;
     b /= bx;
-    const int y0 = (b % by) * 8;
-    const int z0 = (b / by) * kZmChunk;
-    const int zend = min(z0 + kZmChunk, n);
+    const int y0 = (int)(b % by) * 8;
+    const int z0 = (int)(b / by) * zchunk;
+    const int zend = min(z0 + zchunk, n);
+    W += (int64_t)slice * OC * Kp;
+    offy += slice * OC;
 
     const gh_ptr zero = (gh_ptr)(const void *)kZero16;
     const gh_ptr xg = (gh_ptr)X + offx;
@@ -493,8 +536,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         pok[p] = k < CHUNKS && (unsigned)xx < (unsigned)n && (unsigned)yy < (unsigned)n;
         pofs[p] = pok[p] ? (yy * n + xx) * ldx + 8 * g : 0;
     }
-    uint4 stage[PER];
-    auto plane_load = [&](int z) {
+    constexpr int PF = zm_ahead(G, NT);
+    uint4 stage[PF][PER];
+    auto plane_load = [&](int set, int z) {
         const bool zok = (unsigned)z < (unsigned)n;
         const gh_ptr base = xg + (int64_t)(zok ? z : 0) * n * n * ldx;
 #pragma unroll
@@ -506,102 +550,179 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
                 for (int e = 0; e < 8; ++e)
                     if (e >= cin) f.h[e] = 0;
             }
-            stage[p] = f.q;
+            stage[set][p] = f.q;
         }
     };
-    auto plane_store = [&](int slot) {
+    auto plane_store = [&](int set, int slot) {
 #pragma unroll
         for (int p = 0; p < PER; ++p) {
             const int k = tid + 256 * p;
-            if (k < CHUNKS) ring[slot][(k % G) * PV + k / G] = stage[p];
+            if (k < CHUNKS) ring[slot][(k % G) * PS + k / G] = stage[set][p];
         }
     };
 
-    // weights: group g, k step j -> tap 4j + q, channels 8g..8g+7 of output
-    // channel i (zero for the 28th tap and past cout / cin)
-    Frag bf[G][7];
+    // A step's fragment reads and weights: lane group q takes tap and group of
+    // the step's chunk q (zero weights past the last tap and past cin).  Chunks
+    // 4 s .. 4 s + 3 of a tap-major row lie in at most two taps (G >= 2).
+    constexpr int STEPS = zm_steps(G, SPLIT);
+    auto chunk_of = [&](int st, int &tap, int &g) __attribute__((always_inline)) {
+        if (SPLIT) {
+            const int t0 = 4 * st / G, t1 = (4 * st + 3) / G;
+            tap = t0 == t1 || 4 * st + q < G * t1 ? t0 : t1;
+            g = 4 * st + q - G * tap;
+        } else {
+            tap = 4 * (st % 7) + q;
+            g = st / 7;
+        }
+        const bool ok = tap < 27;
+        if (!ok) tap = 13, g = 0;
+        return ok;
+    };
+    Frag bf[STEPS][NT];
 #pragma unroll
-    for (int g = 0; g < G; ++g)
+    for (int j = 0; j < STEPS; ++j)
 #pragma unroll
-        for (int j = 0; j < 7; ++j) {
-            const bool ok = 4 * j + q < 27 && i < cout;
-            const gh_ptr src = (gh_ptr)W + (int64_t)i * Kp + (4 * j + q) * cin + 8 * g;
+        for (int t = 0; t < NT; ++t) {
+            int tap, g;
+            const bool ok = chunk_of(j, tap, g);
+            const gh_ptr src = (gh_ptr)W + (int64_t)(16 * t + i) * Kp + tap * cin + 8 * g;
             if (IN == kInVec) {
-                bf[g][j].q = load_global16(ok ? src : zero);
+                bf[j][t].q = load_global16(ok ? src : zero);
             } else {
 #pragma unroll
-                for (int e = 0; e < 8; ++e) bf[g][j].h[e] = *(ok && e < cin ? src + e : zero);
+                for (int e = 0; e < 8; ++e) bf[j][t].h[e] = *(ok && e < cin ? src + e : zero);
             }
         }
-    // this lane group's taps: ring slot offset (dz + 1), row / column offset
+    // ring offset of row 2 wave, voxel i; group-major steps: this lane group's
+    // taps' slot (dz + 1) and voxel offset
+    const int vox = 2 * wave * SX + i;
     int tslot[7], toff[7];
 #pragma unroll
     for (int j = 0; j < 7; ++j) {
-        const int tap = 4 * j + q;
-        int dz, dy, dx;
-        tap_offset(tap < 27 ? tap : 13, 3, dz, dy, dx);
-        tslot[j] = dz + 1;
-        toff[j] = (dy + 1) * SX + (dx + 1) + i;
+        const int tap = 4 * j + q < 27 ? 4 * j + q : 13;
+        tslot[j] = tap / 9;
+        toff[j] = tap / 3 % 3 * SX + tap % 3 + vox;
     }
-    const float bv = bias && i < cout ? bias[i] : 0.0f;
+    // The products are taken as W X^T, so a lane holds 4 consecutive output
+    // channels, 16 t + 4 q .. + 3, of voxel i of its row: 8-byte stores, the 64
+    // lanes of a tile 512 contiguous bytes (at 16 channels).
+    float bv[NT][4];
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) bv[t][e] = bias ? bias[slice * OC + 16 * t + 4 * q + e] : 0.0f;
+    const bool xin = x0 + i < n;
+    bool rin[2];  // the lane's output voxel of each row is inside
+    int vofs[2];  // its index within a plane
+#pragma unroll
+    for (int r = 0; r < 2; ++r) {
+        rin[r] = xin && y0 + 2 * wave + r < n;
+        vofs[r] = (y0 + 2 * wave + r) * n + x0 + i;
+    }
 
-    // prologue: planes z0-1, z0, z0+1 in slots 0..2, z0+2 in flight
-    plane_load(z0 - 1);
-    plane_store(0);
-    plane_load(z0);
-    plane_store(1);
-    plane_load(z0 + 1);
-    plane_store(2);
-    plane_load(z0 + 2);
+    // prologue: planes z0-1, z0, z0+1 in slots 0..2, the next PF in flight
+    plane_load(0, z0 - 1);
+    plane_store(0, 0);
+    plane_load(0, z0);
+    plane_store(0, 1);
+    plane_load(0, z0 + 1);
+    plane_store(0, 2);
+    plane_load(0, z0 + 2);
+    if (PF == 2) plane_load(PF - 1, z0 + 3);
     __syncthreads();
-    for (int z = z0, st = 0; z < zend; ++z, ++st) {
-        // the previous plane's output tile goes out (written before the barrier)
-        if (st > 0) {
-            const int ob = (st - 1) & 1;
-            const int vt = tid >> 1, part = tid & 1;  // 128 voxels x 2 halves of 16 channels
-            const int x = x0 + vt % 16, y = y0 + vt / 16;
-            if (x < n && y < n)
-                *reinterpret_cast<uint4 *>(Y + (((int64_t)(z - 1) * n + y) * n + x) * ldy + offy + 8 * part) =
-                    *reinterpret_cast<const uint4 *>(&oplane[ob][vt * 16 + 8 * part]);
-        }
-        f32x4 acc[2];
-        acc[0] = acc[1] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int g = 0; g < G; ++g)
-#pragma unroll
-            for (int j = 0; j < 7; ++j) {
-                const uint4 *pl = &ring[(st + tslot[j]) & 3][g * PV];
-#pragma unroll
-                for (int r = 0; r < 2; ++r) {
-                    Frag a;
-                    a.q = pl[(2 * wave + r) * SX + toff[j]];
-                    acc[r] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.v, bf[g][j].v, acc[r], 0, 0, 0);
-                }
-            }
-        // output plane z into LDS: row 2w + r, voxels 4q + e, channel i
+    auto step = [&](auto ph_c, int z) __attribute__((always_inline)) {
+        constexpr int PH = decltype(ph_c)::value;  // (z - z0) & 1
+        const int st = z - z0;
+        const int64_t plane = (int64_t)z * n * n;
+        // plane z+2 into the free slot, the next PF in flight
+        plane_store(PH % PF, (st + 3) & 3);
+        plane_load(PH % PF, z + 2 + PF);
+        f32x4 acc[2][NT];
 #pragma unroll
         for (int r = 0; r < 2; ++r)
 #pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                float o = acc[r][e] + bv;
-                if (relu) o = o > 0.0f ? o : 0.0f;
-                oplane[st & 1][((2 * wave + r) * 16 + 4 * q + e) * 16 + i] = f2bf(o);
+            for (int t = 0; t < NT; ++t) acc[r][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+        f32x4 first[2][NT];  // SPLIT = 2: the first slice's sums
+        const uint4 *const slots[3] = {ring[st & 3], ring[(st + 1) & 3], ring[(st + 2) & 3]};
+#pragma unroll
+        for (int j = 0; j < STEPS; ++j) {
+            const uint4 *pl;
+            if (SPLIT) {
+                // one tap: the lanes differ by their group only; two: by a select
+                const int t0 = 4 * j / G, t1 = (4 * j + 3) / G < 27 ? (4 * j + 3) / G : t0;
+                const uint4 *p0 = slots[t0 / 9] + (4 * j - G * t0) * PS + t0 / 3 % 3 * SX + t0 % 3;
+                const uint4 *p1 = slots[t1 / 9] + (4 * j - G * t1) * PS + t1 / 3 % 3 * SX + t1 % 3;
+                // (past the last chunk, zero weights: any group of the tap)
+                const int gq = 4 * j + 3 < 27 * G || q < 27 * G - 4 * j ? q : 0;
+                pl = (t0 == t1 || 4 * j + q < G * t1 ? p0 : p1) + gq * PS + vox;
+            } else {
+                pl = &ring[(st + tslot[j % 7]) & 3][j / 7 * PS + toff[j % 7]];
             }
-        // plane z+2 into the free slot, plane z+3 in flight
-        plane_store((st + 3) & 3);
-        plane_load(z + 3);
+            if (SPLIT == 2 && j == zm_second(G)) {
+#pragma unroll
+                for (int r = 0; r < 2; ++r)
+#pragma unroll
+                    for (int t = 0; t < NT; ++t) {
+                        first[r][t] = acc[r][t];
+                        acc[r][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+                    }
+            }
+#pragma unroll
+            for (int r = 0; r < 2; ++r) {
+                Frag a;
+                a.q = pl[r * SX];
+#pragma unroll
+                for (int t = 0; t < NT; ++t)
+                    acc[r][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bf[j][t].v, a.v, acc[r][t], 0, 0, 0);
+            }
+        }
+        // schedule: kReads fragment reads in flight ahead of the products that
+        // consume them (the compiler alone keeps about two, and the step then
+        // waits out an LDS latency per k step)
+        constexpr int kReads = zm_reads(G);
+        __builtin_amdgcn_sched_group_barrier(0x100, kReads, 0);
+        lgdhip::static_for<0, 2 * STEPS - kReads>([&](auto) {
+            __builtin_amdgcn_sched_group_barrier(0x008, NT, 0);
+            __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+        });
+        __builtin_amdgcn_sched_group_barrier(0x008, NT * kReads, 0);
+        if (SPLIT == 2) {
+#pragma unroll
+            for (int r = 0; r < 2; ++r)
+#pragma unroll
+                for (int t = 0; t < NT; ++t)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) acc[r][t][e] = first[r][t][e] + acc[r][t][e];
+        }
+#pragma unroll
+        for (int r = 0; r < 2; ++r) {
+            const int64_t v = plane + vofs[r];
+            u16 *out = Y + v * ldy + offy + 4 * q;
+#pragma unroll
+            for (int t = 0; t < NT; ++t) {
+                float o[4];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    o[e] = acc[r][t][e] + bv[t][e];
+                    if (relu) o[e] = o[e] > 0.0f ? o[e] : 0.0f;
+                }
+                if (Y && rin[r])
+                    *reinterpret_cast<uint2 *>(out + 16 * t) = make_uint2(f2bf(o[0]) | (uint32_t)f2bf(o[1]) << 16,
+                                                                          f2bf(o[2]) | (uint32_t)f2bf(o[3]) << 16);
+                if (Y32 && rin[r]) {
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) Y32[v * ld32 + slice * OC + 16 * t + 4 * q + e] = o[e];
+                }
+            }
+        }
         __syncthreads();
+    };
+    int z = z0;
+    for (; z + 1 < zend; z += 2) {
+        step(lgdhip::ic<0>{}, z);
+        step(lgdhip::ic<1>{}, z + 1);
     }
-    // the last plane's output
-    {
-        const int st = zend - z0;
-        const int ob = (st - 1) & 1;
-        const int vt = tid >> 1, part = tid & 1;
-        const int x = x0 + vt % 16, y = y0 + vt / 16;
-        if (x < n && y < n)
-            *reinterpret_cast<uint4 *>(Y + (((int64_t)(zend - 1) * n + y) * n + x) * ldy + offy + 8 * part) =
-                *reinterpret_cast<const uint4 *>(&oplane[ob][vt * 16 + 8 * part]);
-    }
+    if (z < zend) step(lgdhip::ic<0>{}, z);
 }
 
 // GEMM-tiled implicit convolution for 3x3x3 layers with cin % 8 == 0 on the
@@ -871,9 +992,10 @@ __global__ __launch_bounds__(256) void conv1x1_to1_wgrad(const u16 *__restrict__
 // the LDS-staged kernel takes 3x3x3 layers with up to 32 output channels on
 // volumes of at least 16^3
 constexpr int kLdsMinN = 16;
-// z-marching in 16-channel slices for wider outputs from this edge on (96^3:
-// 432 work-groups per slice launch; 64^3 would leave half the CUs idle)
-constexpr int kZmSliceMinN = 96;
+// layers of up to 48 input and more than 32 output channels: in the LDS-tile
+// kernel's k order from this edge on where the z-marching kernel takes them,
+// below it in the GEMM-tiled kernel's
+constexpr int kZmGroupOrderN = 96;
 
 // The GEMM-tiled kernel's launch: 64 x 64 blocks, stages of 64 k, and the
 // number of slices the stage range is split into when a workspace for the
@@ -908,6 +1030,41 @@ size_t gemm_workspace_bytes(int n, const GemmPlan &p) {
 // does not take, the LDS-tile kernel, which sums in the same k order)
 bool gemm_applies(int n, int cin, int ksize, int cout) {
     return ksize == 3 && (cin & 7) == 0 && cout > 16 && (n < 64 || cout > 32);
+}
+
+// conv3d_fwd_zm's launch: output tiles per slice (as many as the weight
+// fragments' registers allow), columns and z planes per chunk
+struct ZmPlan {
+    int nt, slices, bx, by, bz, zchunk;
+};
+ZmPlan zm_plan(int n, int groups, int cout) {
+    ZmPlan z;
+    const int tiles = cout / 16;
+    z.nt = std::max(1, std::min(3, 4 / groups));
+    const int resident = zm_waves(groups, z.nt) >= 2 ? 2 : 1;
+    while (tiles % z.nt) --z.nt;
+    z.slices = tiles / z.nt;
+    z.bx = (n + 15) / 16;
+    z.by = (n + 7) / 8;
+    // Chunks of equal length, by the plane steps of the longest work-group:
+    // where two work-groups share a CU, a step of one that has the CU alone
+    // takes 0.6 of a step of two (0.8 from 5 input groups on); a chunk reads
+    // two planes beyond its own and starts in about one step more.
+    double best = 1e300;
+    for (int chunks = 1; chunks <= n; ++chunks) {
+        const int zc = (n + chunks - 1) / chunks;
+        if ((n + zc - 1) / zc != chunks) continue;
+        const int64_t on_cu = ((int64_t)z.bx * z.by * z.slices * chunks + lgdhip::kCUs - 1) / lgdhip::kCUs;
+        double rounds = resident == 1 ? (double)on_cu : (double)((on_cu + 1) / 2);
+        if (resident == 2 && on_cu == 1) rounds = groups <= 4 ? 0.6 : 0.8;
+        const double steps = rounds * (zc + 3);
+        if (steps < best) {
+            best = steps;
+            z.zchunk = zc;
+            z.bz = chunks;
+        }
+    }
+    return z;
 }
 
 // voxel tiles per wave of the forward kernel: weight-fragment reuse bounded
@@ -1776,35 +1933,39 @@ int lgdhip_conv3d_bf16_forward_ws(const void *x, int n, int ldx, int offx, int c
         LGD_LAUNCHED("conv1x1_from1");
         return 0;
     }
-    // z-marching kernel: 16 output channels written as plain BF16 into an
-    // aligned slice, input of at most 6 groups of 8 channels (or a masked
-    // row of fewer than 8).  Wider outputs on volumes of at least
-    // kZmSliceMinN^3 run one launch per 16-channel slice (weights rows 16 j
-    // .. 16 j + 15, output channels offy + 16 j ..): each launch still has
-    // hundreds of work-groups, each input plane is staged once per slice,
-    // and the slices together beat one GEMM-tiled launch (the input
-    // gradient of a 16 -> 48 layer at 128^3: 412 us there)
-    const bool zm_width = cout == 16 || (cout % 16 == 0 && cout <= 16 * kMaxNTiles && n >= kZmSliceMinN);
-    if (ksize == 3 && zm_width && n >= kLdsMinN && y && !y32 && !accumulate && (ldy & 7) == 0 &&
-        (offy & 7) == 0 && ((uintptr_t)y & 15) == 0) {
+    // z-marching kernel: output channels a multiple of 16, the BF16 output (if
+    // any) into an 8-byte aligned range, input of 1 to 8 groups of 8 channels (or
+    // a masked row of fewer than 8).  It was the fastest at every such shape
+    // measured (figures at the kernel), except that one work-group per CU (7
+    // groups on) and two slices lose to the LDS-tile kernel's one pass over 32
+    // channels (64^3 64 -> 32: 71 us, there 63).  It keeps the k order of the
+    // kernel the layer would go to, so it leaves out the layers that the
+    // GEMM-tiled kernel splits more than two ways.
+    if (ksize == 3 && cout % 16 == 0 && n >= kLdsMinN && !accumulate &&
+        (!y || ((ldy & 3) == 0 && (offy & 3) == 0 && ((uintptr_t)y & 7) == 0))) {
         const bool masked = cin < 8 && (ldx & 7) == 0 && (offx & 7) == 0 && offx + 8 <= ldx &&
                             ((uintptr_t)x & 15) == 0;
         const int groups = (cin & 7) == 0 ? cin / 8 : (masked ? 1 : 0);
-        if (groups >= 1 && groups <= 6) {
-            const int bx = (n + 15) / 16, by = (n + 7) / 8, bz = (n + kZmChunk - 1) / kZmChunk;
-            const unsigned blocks = (unsigned)((int64_t)bx * by * bz);
-            for (int j = 0; j < cout / 16; ++j) {
-                const u16 *Wj = Wb + (size_t)16 * j * Kp;  // Kp % 32 == 0: 16-byte aligned
-                const float *bj = bias ? bias + 16 * j : nullptr;
-                const int offj = offy + 16 * j;
-#define LGD_ZM_CASE(G, I)                                                                                    \
-    if (groups == G && (I == kInMasked) == masked)                                                           \
-        conv3d_fwd_zm<G, I><<<blocks, 256, 0, s>>>(X, n, ldx, offx, cin, Wj, Kp, bj, 16, Y, ldy, offj, relu, bx, by);
-                LGD_ZM_CASE(1, kInMasked) LGD_ZM_CASE(1, kInVec) LGD_ZM_CASE(2, kInVec) LGD_ZM_CASE(3, kInVec)
-                LGD_ZM_CASE(4, kInVec) LGD_ZM_CASE(5, kInVec) LGD_ZM_CASE(6, kInVec)
+        // (with one group the two orders are the same)
+        const bool gemm_order =
+            groups > 1 && (n < kZmGroupOrderN || groups > 6) && gemm_applies(n, cin, ksize, cout);
+        const int split = gemm_order ? gemm_plan(n, cin, cout, workspace != nullptr).slices : 0;
+        if (groups >= 1 && (groups <= 6 || (groups <= 8 && (split || cout == 16))) && split <= 2) {
+            const ZmPlan z = zm_plan(n, groups, cout);
+            const unsigned wgs = (unsigned)((int64_t)z.bx * z.by * z.bz * z.slices), per = lgdhip::xcd_per(wgs);
+#define LGD_ZM_CASE(G, I, NT, S)                                                                            \
+    if (groups == G && (I == kInMasked) == masked && z.nt == NT && split == S)                              \
+        conv3d_fwd_zm<G, I, NT, S><<<lgdhip::xcd_groups(wgs), 256, 0, s>>>(                                 \
+            X, n, ldx, offx, cin, Wb, Kp, bias, Y, ldy, offy, y32, ld32, relu, z.bx, z.by, z.slices, z.zchunk, \
+            wgs, per);
+#define LGD_ZM_CASES(G, NT) LGD_ZM_CASE(G, kInVec, NT, 0) LGD_ZM_CASE(G, kInVec, NT, 1) LGD_ZM_CASE(G, kInVec, NT, 2)
+            LGD_ZM_CASE(1, kInMasked, 1, 0) LGD_ZM_CASE(1, kInMasked, 2, 0) LGD_ZM_CASE(1, kInMasked, 3, 0)
+            LGD_ZM_CASE(1, kInVec, 1, 0) LGD_ZM_CASE(1, kInVec, 2, 0) LGD_ZM_CASE(1, kInVec, 3, 0)
+            LGD_ZM_CASES(2, 1) LGD_ZM_CASES(2, 2) LGD_ZM_CASES(3, 1) LGD_ZM_CASES(4, 1) LGD_ZM_CASES(5, 1)
+            LGD_ZM_CASES(6, 1) LGD_ZM_CASES(7, 1) LGD_ZM_CASES(8, 1)
+#undef LGD_ZM_CASES
 #undef LGD_ZM_CASE
-                LGD_LAUNCHED("conv3d_fwd_zm");
-            }
+            LGD_LAUNCHED("conv3d_fwd_zm");
             return 0;
         }
     }

@@ -230,6 +230,59 @@ def test_conv_zm_slices(hip, oracle, cout, ld, off):
             assert np.all(np.abs(got.astype(np.float64) - ref) <= 2.0 ** -8 * np.abs(ref) + 1e-3)
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,cin,cout,ld,off", [
+    (64, 8, 48, 48, 0), (65, 16, 32, 36, 4), (64, 24, 32, 32, 0), (18, 32, 16, 16, 0), (19, 40, 16, 16, 0),
+    (17, 48, 16, 16, 0), (65, 5, 32, 32, 0), (19, 56, 16, 16, 0), (16, 64, 16, 16, 0), (64, 64, 32, 32, 0),
+    (42, 16, 32, 32, 0), (43, 24, 48, 52, 4), (41, 32, 32, 32, 0), (42, 40, 32, 32, 0), (41, 48, 64, 64, 0),
+    (41, 56, 32, 32, 0), (42, 64, 32, 32, 0), (33, 24, 32, 32, 0), (32, 32, 64, 64, 0), (36, 16, 48, 48, 0),
+    (37, 40, 48, 48, 0), (35, 48, 32, 32, 0), (33, 56, 48, 48, 0), (32, 64, 64, 64, 0)])
+def test_conv_zm_same_bits(hip, oracle, n, cin, cout, ld, off):
+    """The z-marching kernel over its input groups, output tiles per slice and
+    the three k orders, on edges that leave part of a column and a chunk of
+    planes outside: byte-equal to the kernel that takes the layer when the
+    launch accumulates (here into zeros), BF16 rows at 8-byte offsets, other
+    channels untouched, the FP32 output rounding to the BF16 one; and the FP32
+    output of the volume's first and last 10 planes (9 of them whole in the
+    oracle's cube) within K accumulated roundings of the FP64 oracle."""
+    rng = np.random.default_rng(n + 100 * cin + cout)
+    row = 8 if cin < 8 else cin
+    x = bf16_round(rng.standard_normal((n, n, n, row)).astype(np.float32))
+    w = bf16_round((rng.standard_normal((cout, 27, cin)) / np.sqrt(27 * cin)).astype(np.float32))
+    b = rng.standard_normal(cout).astype(np.float32)
+    lib = hip.load()
+    kp = lib.lgdhip_conv3d_kpad(cin, 3)
+    xb, wb, bb = dev(hip, to_bf16_bits(x)), dev(hip, to_bf16_bits(conv_weights_layout(w, kp))), dev(hip, b)
+    wsb = lib.lgdhip_conv3d_forward_workspace_bytes(n, cin, 3, cout)
+    ws = hip.DeviceBuffer(max(wsb, 16))
+    init = to_bf16_bits(rng.standard_normal((n, n, n, ld)).astype(np.float32)).reshape(n, n, n, ld).copy()
+    init[..., off:off + cout] = 0
+    y32 = hip.DeviceBuffer(n ** 3 * cout * 4)
+    print("[case] conv z-march orders", n, cin, cout, ld, off, flush=True)
+    hosts = []
+    for accumulate in (0, 1):
+        y = dev(hip, init)
+        hip.call("lgdhip_conv3d_bf16_forward_ws", xb.ptr, n, row, 0, cin, 3, wb.ptr, bb.ptr, cout, y.ptr, ld, off, None,
+                 0, 0, accumulate, ws.ptr, wsb, None)
+        host = np.empty(n ** 3 * ld, np.uint16)
+        y.download(host)
+        hosts.append(host.reshape(n, n, n, ld))
+    hip.call("lgdhip_conv3d_bf16_forward_ws", xb.ptr, n, row, 0, cin, 3, wb.ptr, bb.ptr, cout, None, 0, 0, y32.ptr,
+             cout, 0, 0, ws.ptr, wsb, None)
+    out = np.empty(n ** 3 * cout, np.float32)
+    y32.download(out)
+    out = out.reshape(n, n, n, cout)
+    assert np.array_equal(hosts[0], hosts[1])
+    assert np.array_equal(hosts[0][..., off:off + cout], to_bf16_bits(out))
+    for lo in (0, n - 10):
+        keep = slice(0, 9) if lo == 0 else slice(1, 10)
+        cube, inner = (slice(lo, lo + 10),) * 3, (keep,) * 3
+        c = x[cube][..., :cin].astype(np.float64)
+        ref = oracle.conv3d_forward(c, w.astype(np.float64), b.astype(np.float64), 3)[inner]
+        mag = oracle.conv3d_forward(np.abs(c), np.abs(w).astype(np.float64), np.abs(b).astype(np.float64), 3)[inner]
+        assert np.all(np.abs(out[cube][inner] - ref) <= (27 * cin + 2) * 2.0 ** -24 * mag + 1e-30)
+
+
 def run_conv_split(hip, x, w, bias, ld_out=None, off_out=0, relu=False, y_init=None):
     """run_conv through lgdhip_conv3d_bf16_forward_ws with the workspace the
     layer asks for; returns (y32, y_bf16, workspace bytes)."""
