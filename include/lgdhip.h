@@ -494,6 +494,14 @@ int lgdhip_conv3d_bf16_forward_ws(const void *x, int n, int ldx, int offx, int c
 /* weights of the input-gradient convolution: wt[ci][k'] (Kp' = kpad(cout)),
  * flipped taps, so dx = conv(dy, wt) with cin' = cout, cout' = cin */
 int lgdhip_conv3d_dgrad_weights(const void *w, int cin, int cout, int ksize, void *wt, lgdhip_stream_t stream);
+/* lgdhip_conv3d_bf16_forward_ws without bias, clamp or accumulation, its BF16
+ * outputs zeroed where act (cout channels, stride lda, offset offa) is not
+ * positive: the input gradient of a layer and the ReLU backward of the layer
+ * before it, in one launch where the shape allows.  The same bits as
+ * lgdhip_conv3d_bf16_forward_ws followed by lgdhip_relu_backward_bf16. */
+int lgdhip_conv3d_bf16_dgrad_relu(const void *x, int n, int ldx, int offx, int cin, int ksize, const void *w, int cout,
+                                  void *y, int ldy, int offy, const void *act, int lda, int offa, void *workspace,
+                                  size_t workspace_bytes, lgdhip_stream_t stream);
 /* dw[co][k] (+)= sum_v dy[v][co] x[v+tap(k)][ci(k)] (FP32, fixed-order
  * reduction over voxel chunks), db[co] = sum_v dy[v][co] (if non-NULL).
  * 3x3x3 layers of aligned 8-channel rows are reduced over column chunks of
@@ -512,11 +520,17 @@ int lgdhip_avgpool2_bf16(const void *x, int n, int ldx, int offx, void *y, int l
                          lgdhip_stream_t stream);
 int lgdhip_avgpool2_backward_bf16(const void *dy, int n, int ldy, int offy, void *dx, int ldx, int offx, int c,
                                   int accumulate, lgdhip_stream_t stream);
+/* the same gradient, zeroed where act (as dx, stride lda, offset offa) is not
+ * positive: with the ReLU backward of the layer that made x (act NULL: none) */
+int lgdhip_avgpool2_backward_relu_bf16(const void *dy, int n, int ldy, int offy, void *dx, int ldx, int offx, int c,
+                                       int accumulate, const void *act, int lda, int offa, lgdhip_stream_t stream);
 /* nearest 2x upsample m^3 -> (2m)^3, its gradient (sum of the 8 children) */
 int lgdhip_upsample2_bf16(const void *x, int m, int ldx, int offx, void *y, int ldy, int offy, int c,
                           lgdhip_stream_t stream);
 int lgdhip_upsample2_backward_bf16(const void *dy, int m, int ldy, int offy, void *dx, int ldx, int offx, int c,
                                    int accumulate, lgdhip_stream_t stream);
+int lgdhip_upsample2_backward_relu_bf16(const void *dy, int m, int ldy, int offy, void *dx, int ldx, int offx, int c,
+                                        int accumulate, const void *act, int lda, int offa, lgdhip_stream_t stream);
 /* nearest 2x upsample of x (m^3, cu channels) and a skip tensor ((2m)^3, cs
  * channels) written as whole concatenation rows y[v][offy .. offy+cu+cs)
  * (the upsampled channels first); no reference counterpart: the U-Net of

@@ -453,6 +453,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     }
 }
 
+// all ones in the halves of a word of two BF16 values that are positive
+__device__ __forceinline__ uint32_t positive_halves(uint32_t w) {
+    return (__uint_as_float(w << 16) > 0.0f ? 0xFFFFu : 0u) |
+           (__uint_as_float(w & 0xFFFF0000u) > 0.0f ? 0xFFFF0000u : 0u);
+}
+
 // Z-marching LDS convolution for 3x3x3 layers with cin = 8 G input channels (G
 // <= 6; G = 1 also takes cin < 8 rows, see IN) and slices of NT x 16 output
 // channels.  A work-group owns a 16 x 8 column of output voxels and one slice and
@@ -475,6 +481,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 // tap or two) per step.  SPLIT = 2: the same in conv3d_fwd_gemm's two slices of
 // its stages, each summed from zero and then added.
 //
+// MASK: outputs whose activation A (rows of lda elements) is not positive are
+// zeroed: the ReLU backward of the layer that made the tensor this one is the
+// gradient of, without a pass of its own (a training step at 128^3 took 2108 us
+// with these passes, 1997 us with the masks taken along here, in conv1x1_from1
+// and in the resampling gradients).
+//
 // Measured (us; the launch this one replaces in brackets: one 16-channel slice
 // per launch with the outputs re-tiled in LDS; the GEMM-tiled kernel and its
 // reduction; the LDS-tile kernel): 128^3 16 -> 16 41 [48], 3 -> 16 36 [47], 48 ->
@@ -493,11 +505,12 @@ constexpr int zm_second(int g) { return (zm_steps(g, 2) + 1) / 2 / 2 * 2; }
 // 16 at 128^3 133 us with six, 115 with three)
 constexpr int zm_reads(int g) { return g == 6 ? 3 : 6; }
 
-template <int G, int IN, int NT, int SPLIT>
+template <int G, int IN, int NT, int SPLIT, bool MASK>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(zm_waves(G, NT), zm_waves(G, NT)))) void
 conv3d_fwd_zm(const u16 *__restrict__ X, int n, int ldx, int offx, int cin, const u16 *__restrict__ W, int Kp,
               const float *__restrict__ bias, u16 *Y, int ldy, int offy, float *Y32, int ld32, int relu,
-              int bx, int by, int slices, int zchunk, unsigned groups, unsigned per) {
+              const u16 *__restrict__ A, int lda, int offa, int bx, int by, int slices, int zchunk, unsigned groups,
+              unsigned per) {
     constexpr int SX = 18, SY = 10, PV = SX * SY;  // staged voxels per plane
     constexpr int CHUNKS = PV * G;                 // 16-byte pieces per plane
     constexpr int PER = (CHUNKS + 255) / 256;
@@ -521,6 +534,7 @@ conv3d_fwd_zm(const u16 *__restrict__ X, int n, int ldx, int offx, int cin, cons
     const int zend = min(z0 + zchunk, n);
     W += (int64_t)slice * OC * Kp;
     offy += slice * OC;
+    offa += slice * OC;
 
     const gh_ptr zero = (gh_ptr)(const void *)kZero16;
     const gh_ptr xg = (gh_ptr)X + offx;
@@ -642,6 +656,15 @@ conv3d_fwd_zm(const u16 *__restrict__ X, int n, int ldx, int offx, int cin, cons
         for (int r = 0; r < 2; ++r)
 #pragma unroll
             for (int t = 0; t < NT; ++t) acc[r][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+        uint2 act[2][NT];  // MASK: the outputs' activations
+        if (MASK) {
+#pragma unroll
+            for (int r = 0; r < 2; ++r)
+#pragma unroll
+                for (int t = 0; t < NT; ++t)
+                    act[r][t] = load_global8(
+                        (gh_ptr)A + (rin[r] ? (plane + vofs[r]) * lda : 0) + offa + 16 * t + 4 * q);
+        }
         f32x4 first[2][NT];  // SPLIT = 2: the first slice's sums
         const uint4 *const slots[3] = {ring[st & 3], ring[(st + 1) & 3], ring[(st + 2) & 3]};
 #pragma unroll
@@ -706,9 +729,12 @@ conv3d_fwd_zm(const u16 *__restrict__ X, int n, int ldx, int offx, int cin, cons
                     o[e] = acc[r][t][e] + bv[t][e];
                     if (relu) o[e] = o[e] > 0.0f ? o[e] : 0.0f;
                 }
-                if (Y && rin[r])
-                    *reinterpret_cast<uint2 *>(out + 16 * t) = make_uint2(f2bf(o[0]) | (uint32_t)f2bf(o[1]) << 16,
-                                                                          f2bf(o[2]) | (uint32_t)f2bf(o[3]) << 16);
+                uint2 h = make_uint2(f2bf(o[0]) | (uint32_t)f2bf(o[1]) << 16, f2bf(o[2]) | (uint32_t)f2bf(o[3]) << 16);
+                if (MASK) {
+                    h.x &= positive_halves(act[r][t].x);
+                    h.y &= positive_halves(act[r][t].y);
+                }
+                if (Y && rin[r]) *reinterpret_cast<uint2 *>(out + 16 * t) = h;
                 if (Y32 && rin[r]) {
 #pragma unroll
                     for (int e = 0; e < 4; ++e) Y32[v * ld32 + slice * OC + 16 * t + 4 * q + e] = o[e];
@@ -938,7 +964,8 @@ __global__ __launch_bounds__(256) void conv1x1_to1(const u16 *__restrict__ X, in
 __global__ __launch_bounds__(256) void conv1x1_from1(const u16 *__restrict__ X, uint32_t items, int ldx, int offx,
                                                      const u16 *__restrict__ W, int Kp,
                                                      const float *__restrict__ bias, int c8, u16 *__restrict__ Y,
-                                                     int ldy, int offy, int relu) {
+                                                     int ldy, int offy, int relu, const u16 *__restrict__ A, int lda,
+                                                     int offa) {
     const uint32_t i = blockIdx.x * 256u + threadIdx.x;
     if (i >= items) return;
     const uint32_t v = i / (uint32_t)c8;
@@ -950,6 +977,13 @@ __global__ __launch_bounds__(256) void conv1x1_from1(const u16 *__restrict__ X, 
         float o = xv * bf2f(W[(int64_t)(co + e) * Kp]) + (bias ? bias[co + e] : 0.0f);
         if (relu) o = o > 0.0f ? o : 0.0f;
         f.h[e] = f2bf(o);
+    }
+    if (A) {  // ReLU backward of the layer that made Y's values, as conv3d_fwd_zm's
+        const uint4 a = *reinterpret_cast<const uint4 *>(A + (int64_t)v * lda + offa + co);
+        f.q.x &= positive_halves(a.x);
+        f.q.y &= positive_halves(a.y);
+        f.q.z &= positive_halves(a.z);
+        f.q.w &= positive_halves(a.w);
     }
     *reinterpret_cast<uint4 *>(Y + (int64_t)v * ldy + offy + co) = f.q;
 }
@@ -1631,7 +1665,7 @@ __global__ void avgpool2_v8(const u16 *__restrict__ X, int n, int ldx, int offx,
 }
 
 __global__ void avgpool2_backward_v8(const u16 *__restrict__ dY, int n, int ldy, int offy, u16 *dX, int ldx, int offx,
-                                     int c8, int accumulate) {
+                                     int c8, int accumulate, const u16 *__restrict__ A, int lda, int offa) {
     const int m = n / 2;
     int x, ch;
     if (!row_thread(n, c8, x, ch)) return;
@@ -1648,6 +1682,12 @@ __global__ void avgpool2_backward_v8(const u16 *__restrict__ dY, int n, int ldy,
         float g = bf2f(a.h[k]) * 0.125f;
         if (accumulate) g += bf2f(old.h[k]);
         o.h[k] = f2bf(g);
+    }
+    if (A) {  // ReLU backward of the layer that made X
+        const Bf8 act = ld8(A + v * lda + offa + ch);
+#pragma unroll
+        for (int k = 0; k < 8; ++k)
+            if (!(bf2f(act.h[k]) > 0.0f)) o.h[k] = 0;
     }
     st8(q, o);
 }
@@ -1707,7 +1747,7 @@ __global__ void upsample2_concat(const u16 *__restrict__ X, int m, int ldx, int 
 }
 
 __global__ void upsample2_backward_v8(const u16 *__restrict__ dY, int m, int ldy, int offy, u16 *dX, int ldx, int offx,
-                                      int c8, int accumulate) {
+                                      int c8, int accumulate, const u16 *__restrict__ A, int lda, int offa) {
     const int n = 2 * m;
     int x, ch;
     if (!row_thread(m, c8, x, ch)) return;
@@ -1726,6 +1766,12 @@ __global__ void upsample2_backward_v8(const u16 *__restrict__ dY, int m, int ldy
     Bf8 o;
 #pragma unroll
     for (int k = 0; k < 8; ++k) o.h[k] = f2bf(accumulate ? s[k] + bf2f(old.h[k]) : s[k]);
+    if (A) {  // ReLU backward of the layer that made X
+        const Bf8 act = ld8(A + v * lda + offa + ch);
+#pragma unroll
+        for (int k = 0; k < 8; ++k)
+            if (!(bf2f(act.h[k]) > 0.0f)) o.h[k] = 0;
+    }
     st8(q, o);
 }
 
@@ -1875,28 +1921,13 @@ int check_tensor(int n, int ld, int off, int c) {
     return 0;
 }
 
-} // namespace
-
-extern "C" {
-
-int lgdhip_conv3d_kpad(int cin, int ksize) { return (((ksize == 1 ? 1 : 27) * cin + 31) / 32) * 32; }
-
-size_t lgdhip_conv3d_forward_workspace_bytes(int n, int cin, int ksize, int cout) {
-    if (n < 1 || cin < 1 || cout < 1 || !gemm_applies(n, cin, ksize, cout)) return 0;
-    return gemm_workspace_bytes(n, gemm_plan(n, cin, cout, true));
-}
-
-int lgdhip_conv3d_bf16_forward(const void *x, int n, int ldx, int offx, int cin, int ksize, const void *w,
-                               const float *bias, int cout, void *y, int ldy, int offy, float *y32, int ld32,
-                               int relu, int accumulate, lgdhip_stream_t stream) {
-    return lgdhip_conv3d_bf16_forward_ws(x, n, ldx, offx, cin, ksize, w, bias, cout, y, ldy, offy, y32, ld32, relu,
-                                         accumulate, nullptr, 0, stream);
-}
-
-int lgdhip_conv3d_bf16_forward_ws(const void *x, int n, int ldx, int offx, int cin, int ksize, const void *w,
-                                  const float *bias, int cout, void *y, int ldy, int offy, float *y32, int ld32,
-                                  int relu, int accumulate, void *workspace, size_t workspace_bytes,
-                                  lgdhip_stream_t stream) {
+// lgdhip_conv3d_bf16_forward_ws, with the ReLU mask of an activation where the
+// launch takes one along (masked_out; lda, offa its row stride and offset)
+int conv3d_forward(const void *x, int n, int ldx, int offx, int cin, int ksize, const void *w, const float *bias,
+                   int cout, void *y, int ldy, int offy, float *y32, int ld32, int relu, int accumulate,
+                   void *workspace, size_t workspace_bytes, const u16 *act, int lda, int offa, bool &masked_out,
+                   lgdhip_stream_t stream) {
+    masked_out = false;
     LGD_REQUIRE(x && w && (y || y32), "NULL pointer");
     LGD_REQUIRE(ksize == 1 || ksize == 3, "ksize must be 1 or 3");
     LGD_REQUIRE(cout >= 1 && cout <= 16 * kMaxNTiles, "cout must be in [1, 192]");
@@ -1928,8 +1959,10 @@ int lgdhip_conv3d_bf16_forward_ws(const void *x, int n, int ldx, int offx, int c
     if (ksize == 1 && cin == 1 && cout % 8 == 0 && y && !y32 && !accumulate && (ldy & 7) == 0 && (offy & 7) == 0 &&
         ((uintptr_t)y & 15) == 0 && nvox * (cout / 8) < INT32_MAX) {
         const uint32_t items = (uint32_t)(nvox * (cout / 8));
+        masked_out = act && vec8(act, y, cout, lda, offa, ldy, offy);
         conv1x1_from1<<<(unsigned)((items + 255u) / 256u), 256, 0, s>>>(X, items, ldx, offx, Wb, Kp, bias, cout / 8, Y,
-                                                                      ldy, offy, relu);
+                                                                      ldy, offy, relu, masked_out ? act : nullptr, lda,
+                                                                      offa);
         LGD_LAUNCHED("conv1x1_from1");
         return 0;
     }
@@ -1953,16 +1986,23 @@ int lgdhip_conv3d_bf16_forward_ws(const void *x, int n, int ldx, int offx, int c
         if (groups >= 1 && (groups <= 6 || (groups <= 8 && (split || cout == 16))) && split <= 2) {
             const ZmPlan z = zm_plan(n, groups, cout);
             const unsigned wgs = (unsigned)((int64_t)z.bx * z.by * z.bz * z.slices), per = lgdhip::xcd_per(wgs);
-#define LGD_ZM_CASE(G, I, NT, S)                                                                            \
-    if (groups == G && (I == kInMasked) == masked && z.nt == NT && split == S)                              \
-        conv3d_fwd_zm<G, I, NT, S><<<lgdhip::xcd_groups(wgs), 256, 0, s>>>(                                 \
-            X, n, ldx, offx, cin, Wb, Kp, bias, Y, ldy, offy, y32, ld32, relu, z.bx, z.by, z.slices, z.zchunk, \
-            wgs, per);
-#define LGD_ZM_CASES(G, NT) LGD_ZM_CASE(G, kInVec, NT, 0) LGD_ZM_CASE(G, kInVec, NT, 1) LGD_ZM_CASE(G, kInVec, NT, 2)
-            LGD_ZM_CASE(1, kInMasked, 1, 0) LGD_ZM_CASE(1, kInMasked, 2, 0) LGD_ZM_CASE(1, kInMasked, 3, 0)
-            LGD_ZM_CASE(1, kInVec, 1, 0) LGD_ZM_CASE(1, kInVec, 2, 0) LGD_ZM_CASE(1, kInVec, 3, 0)
-            LGD_ZM_CASES(2, 1) LGD_ZM_CASES(2, 2) LGD_ZM_CASES(3, 1) LGD_ZM_CASES(4, 1) LGD_ZM_CASES(5, 1)
-            LGD_ZM_CASES(6, 1) LGD_ZM_CASES(7, 1) LGD_ZM_CASES(8, 1)
+            // the mask is compiled for square layers of 16, 32 and 64 channels,
+            // those with a ReLU on both sides in a network
+            masked_out = act && !y32 && z.nt == 1 && (groups == 2 || groups == 4 || groups == 8) && (lda & 3) == 0 &&
+                         (offa & 3) == 0 && ((uintptr_t)act & 7) == 0;
+#define LGD_ZM_CASE(G, I, NT, S, M)                                                                         \
+    if (groups == G && (I == kInMasked) == masked && z.nt == NT && split == S && M == masked_out)           \
+        conv3d_fwd_zm<G, I, NT, S, M><<<lgdhip::xcd_groups(wgs), 256, 0, s>>>(                              \
+            X, n, ldx, offx, cin, Wb, Kp, bias, Y, ldy, offy, y32, ld32, relu, act, lda, offa, z.bx, z.by,  \
+            z.slices, z.zchunk, wgs, per);
+#define LGD_ZM_CASES(G, NT, M)                                                          \
+    LGD_ZM_CASE(G, kInVec, NT, 0, M) LGD_ZM_CASE(G, kInVec, NT, 1, M) LGD_ZM_CASE(G, kInVec, NT, 2, M)
+            LGD_ZM_CASE(1, kInMasked, 1, 0, false) LGD_ZM_CASE(1, kInMasked, 2, 0, false)
+            LGD_ZM_CASE(1, kInMasked, 3, 0, false) LGD_ZM_CASE(1, kInVec, 1, 0, false)
+            LGD_ZM_CASE(1, kInVec, 2, 0, false) LGD_ZM_CASE(1, kInVec, 3, 0, false)
+            LGD_ZM_CASES(2, 1, false) LGD_ZM_CASES(2, 2, false) LGD_ZM_CASES(3, 1, false) LGD_ZM_CASES(4, 1, false)
+            LGD_ZM_CASES(5, 1, false) LGD_ZM_CASES(6, 1, false) LGD_ZM_CASES(7, 1, false) LGD_ZM_CASES(8, 1, false)
+            LGD_ZM_CASES(2, 1, true) LGD_ZM_CASES(4, 1, true) LGD_ZM_CASES(8, 1, true)
 #undef LGD_ZM_CASES
 #undef LGD_ZM_CASE
             LGD_LAUNCHED("conv3d_fwd_zm");
@@ -2042,6 +2082,46 @@ int lgdhip_conv3d_bf16_forward_ws(const void *x, int n, int ldx, int offx, int c
 #undef LGD_CONV_CASE
     LGD_LAUNCHED("conv3d_fwd_mfma");
     return 0;
+}
+
+} // namespace
+
+extern "C" {
+
+int lgdhip_conv3d_kpad(int cin, int ksize) { return (((ksize == 1 ? 1 : 27) * cin + 31) / 32) * 32; }
+
+size_t lgdhip_conv3d_forward_workspace_bytes(int n, int cin, int ksize, int cout) {
+    if (n < 1 || cin < 1 || cout < 1 || !gemm_applies(n, cin, ksize, cout)) return 0;
+    return gemm_workspace_bytes(n, gemm_plan(n, cin, cout, true));
+}
+
+int lgdhip_conv3d_bf16_forward(const void *x, int n, int ldx, int offx, int cin, int ksize, const void *w,
+                               const float *bias, int cout, void *y, int ldy, int offy, float *y32, int ld32,
+                               int relu, int accumulate, lgdhip_stream_t stream) {
+    return lgdhip_conv3d_bf16_forward_ws(x, n, ldx, offx, cin, ksize, w, bias, cout, y, ldy, offy, y32, ld32, relu,
+                                         accumulate, nullptr, 0, stream);
+}
+
+int lgdhip_conv3d_bf16_forward_ws(const void *x, int n, int ldx, int offx, int cin, int ksize, const void *w,
+                                  const float *bias, int cout, void *y, int ldy, int offy, float *y32, int ld32,
+                                  int relu, int accumulate, void *workspace, size_t workspace_bytes,
+                                  lgdhip_stream_t stream) {
+    bool masked;
+    return conv3d_forward(x, n, ldx, offx, cin, ksize, w, bias, cout, y, ldy, offy, y32, ld32, relu, accumulate,
+                          workspace, workspace_bytes, nullptr, 0, 0, masked, stream);
+}
+
+int lgdhip_conv3d_bf16_dgrad_relu(const void *x, int n, int ldx, int offx, int cin, int ksize, const void *w, int cout,
+                                  void *y, int ldy, int offy, const void *act, int lda, int offa, void *workspace,
+                                  size_t workspace_bytes, lgdhip_stream_t stream) {
+    LGD_REQUIRE(y && act, "NULL pointer");
+    int rc = check_tensor(n, lda, offa, cout);
+    if (rc) return rc;
+    bool masked;
+    rc = conv3d_forward(x, n, ldx, offx, cin, ksize, w, nullptr, cout, y, ldy, offy, nullptr, 0, 0, 0, workspace,
+                        workspace_bytes, (const u16 *)act, lda, offa, masked, stream);
+    if (rc || masked) return rc;
+    return lgdhip_relu_backward_bf16(y, ldy, offy, act, lda, offa, cout, (int64_t)n * n * n, stream);
 }
 
 size_t lgdhip_conv3d_wgrad_workspace_bytes(int n, int cin, int ksize, int cout, int chunk_vox) {
@@ -2187,17 +2267,22 @@ int lgdhip_avgpool2_bf16(const void *x, int n, int ldx, int offx, void *y, int l
 
 int lgdhip_avgpool2_backward_bf16(const void *dy, int n, int ldy, int offy, void *dx, int ldx, int offx, int c,
                                   int accumulate, lgdhip_stream_t stream) {
+    return lgdhip_avgpool2_backward_relu_bf16(dy, n, ldy, offy, dx, ldx, offx, c, accumulate, nullptr, 0, 0, stream);
+}
+
+int lgdhip_avgpool2_backward_relu_bf16(const void *dy, int n, int ldy, int offy, void *dx, int ldx, int offx, int c,
+                                       int accumulate, const void *act, int lda, int offa, lgdhip_stream_t stream) {
     LGD_REQUIRE(dy && dx && n % 2 == 0, "bad arguments");
-    if (vec8(dy, dx, c, ldy, offy, ldx, offx) && n <= kMaxRowGrid) {
+    if (vec8(dy, dx, c, ldy, offy, ldx, offx) && (!act || vec8(act, dx, c, lda, offa, ldx, offx)) && n <= kMaxRowGrid) {
         avgpool2_backward_v8<<<row_grid(n, c / 8), 256, 0, lgdhip::as_stream(stream)>>>(
-            (const u16 *)dy, n, ldy, offy, (u16 *)dx, ldx, offx, c / 8, accumulate);
+            (const u16 *)dy, n, ldy, offy, (u16 *)dx, ldx, offx, c / 8, accumulate, (const u16 *)act, lda, offa);
         LGD_LAUNCHED("avgpool2_backward_v8");
         return 0;
     }
     avgpool2_backward<<<blocks_for((int64_t)n * n * n * c), 256, 0, lgdhip::as_stream(stream)>>>(
         (const u16 *)dy, n, ldy, offy, (u16 *)dx, ldx, offx, c, accumulate);
     LGD_LAUNCHED("avgpool2_backward");
-    return 0;
+    return act ? lgdhip_relu_backward_bf16(dx, ldx, offx, act, lda, offa, c, (int64_t)n * n * n, stream) : 0;
 }
 
 int lgdhip_upsample2_bf16(const void *x, int m, int ldx, int offx, void *y, int ldy, int offy, int c,
@@ -2233,18 +2318,23 @@ int lgdhip_upsample2_concat_bf16(const void *x, int m, int ldx, int offx, int cu
 }
 
 int lgdhip_upsample2_backward_bf16(const void *dy, int m, int ldy, int offy, void *dx, int ldx, int offx, int c,
-                                   int accumulate, lgdhip_stream_t stream) {
+                                  int accumulate, lgdhip_stream_t stream) {
+    return lgdhip_upsample2_backward_relu_bf16(dy, m, ldy, offy, dx, ldx, offx, c, accumulate, nullptr, 0, 0, stream);
+}
+
+int lgdhip_upsample2_backward_relu_bf16(const void *dy, int m, int ldy, int offy, void *dx, int ldx, int offx, int c,
+                                       int accumulate, const void *act, int lda, int offa, lgdhip_stream_t stream) {
     LGD_REQUIRE(dy && dx && m >= 1, "bad arguments");
-    if (vec8(dy, dx, c, ldy, offy, ldx, offx) && 2 * (int64_t)m <= kMaxRowGrid) {
+    if (vec8(dy, dx, c, ldy, offy, ldx, offx) && (!act || vec8(act, dx, c, lda, offa, ldx, offx)) && 2 * (int64_t)m <= kMaxRowGrid) {
         upsample2_backward_v8<<<row_grid(m, c / 8), 256, 0, lgdhip::as_stream(stream)>>>(
-            (const u16 *)dy, m, ldy, offy, (u16 *)dx, ldx, offx, c / 8, accumulate);
+            (const u16 *)dy, m, ldy, offy, (u16 *)dx, ldx, offx, c / 8, accumulate, (const u16 *)act, lda, offa);
         LGD_LAUNCHED("upsample2_backward_v8");
         return 0;
     }
     upsample2_backward<<<blocks_for((int64_t)m * m * m * c), 256, 0, lgdhip::as_stream(stream)>>>(
         (const u16 *)dy, m, ldy, offy, (u16 *)dx, ldx, offx, c, accumulate);
     LGD_LAUNCHED("upsample2_backward");
-    return 0;
+    return act ? lgdhip_relu_backward_bf16(dx, ldx, offx, act, lda, offa, c, (int64_t)m * m * m, stream) : 0;
 }
 
 int lgdhip_pack_bf16(const float *src, int64_t nvox, void *y, int ldy, int offy, lgdhip_stream_t stream) {

@@ -178,6 +178,9 @@ SIGNATURES = {
     "lgdhip_relu_backward_bf16": (_I, [_P, _I, _I, _P, _I, _I, _I, _I64, _P]),
     "lgdhip_avgpool2_bf16": (_I, [_P, _I, _I, _I, _P, _I, _I, _I, _P]),
     "lgdhip_avgpool2_backward_bf16": (_I, [_P, _I, _I, _I, _P, _I, _I, _I, _I, _P]),
+    "lgdhip_avgpool2_backward_relu_bf16": (_I, [_P, _I, _I, _I, _P, _I, _I, _I, _I, _P, _I, _I, _P]),
+    "lgdhip_upsample2_backward_relu_bf16": (_I, [_P, _I, _I, _I, _P, _I, _I, _I, _I, _P, _I, _I, _P]),
+    "lgdhip_conv3d_bf16_dgrad_relu": (_I, [_P, _I, _I, _I, _I, _I, _P, _I, _P, _I, _I, _P, _I, _I, _P, _SZ, _P]),
     "lgdhip_upsample2_bf16": (_I, [_P, _I, _I, _I, _P, _I, _I, _I, _P]),
     "lgdhip_upsample2_backward_bf16": (_I, [_P, _I, _I, _I, _P, _I, _I, _I, _I, _P]),
     "lgdhip_upsample2_concat_bf16": (_I, [_P, _I, _I, _I, _I, _P, _I, _I, _I, _P, _I, _I, _P]),

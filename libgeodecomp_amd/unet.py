@@ -263,57 +263,60 @@ class UNet3D:
         self.loss_partial.download(parts, self.stream)
         return float(parts.astype(np.float64).sum() / nv)
 
-    def _back(self, name, x: Tensor, xoff, g_out: Tensor, goff, y_act: Tensor | None, yoff, g_in: Tensor | None,
-              ginoff, accumulate_w: int, accumulate_in: int = 0):
-        """Backward of one conv: ReLU mask on g_out (if relu), weight/bias
-        gradient, and the input gradient into g_in (accumulated if asked)."""
+    def _back(self, name, x: Tensor, xoff, g_out: Tensor, goff, g_in: Tensor | None, accumulate_w: int,
+              act: Tensor | None = None):
+        """Backward of one conv, whose ReLU (if any) g_out has been through:
+        weight/bias gradient, and the input gradient into g_in, through the
+        ReLU of the layer whose output act is (if given)."""
         l = self.layers[name]
         S = self.stream
-        if l.relu:
-            lgdhip.call("lgdhip_relu_backward_bf16", g_out.ptr, g_out.ld, goff, y_act.ptr, y_act.ld, yoff, l.cout,
-                        l.n ** 3, S)
         lgdhip.call("lgdhip_conv3d_bf16_wgrad", x.ptr, l.n, x.ld, xoff, l.cin, l.ksize, g_out.ptr, g_out.ld, goff,
                     l.cout, l.gw.ptr, l.gb.ptr if self.use_bias else None, accumulate_w, 0, self.ws.ptr,
                     self.ws_bytes, S)
-        if g_in is not None:
+        if act is not None:
+            lgdhip.call("lgdhip_conv3d_bf16_dgrad_relu", g_out.ptr, l.n, g_out.ld, goff, l.cout, l.ksize, l.wt.ptr,
+                        l.cin, g_in.ptr, g_in.ld, 0, act.ptr, act.ld, 0, self.ws.ptr, self.ws_bytes, S)
+        elif g_in is not None:
             lgdhip.call("lgdhip_conv3d_bf16_forward_ws", g_out.ptr, l.n, g_out.ld, goff, l.cout, l.ksize,
-                        l.wt.ptr, None, l.cin, g_in.ptr, g_in.ld, ginoff, None, 1, 0, accumulate_in, self.ws.ptr,
-                        self.ws_bytes, S)
+                        l.wt.ptr, None, l.cin, g_in.ptr, g_in.ld, 0, None, 1, 0, 0, self.ws.ptr, self.ws_bytes, S)
 
     def backward(self, accumulate: int = 0):
         """Gradients of the last loss() w.r.t. every weight (accumulate adds
-        to the previous sample's gradients, for mini-batches)."""
+        to the previous sample's gradients, for mini-batches).  Every gradient
+        goes through its layer's ReLU where it is made."""
         c0, c1, c2, c3 = self.ch
-        S = self.stream
         G = self.g
         acc = accumulate
-        self._back("out", self.b0d, 0, self.gpred, 0, None, 0, G["b0d"], 0, acc)
-        self._back("d0b", self.a0d, 0, G["b0d"], 0, self.b0d, 0, G["a0d"], 0, acc)
-        self._back("d0a", self.cat0, 0, G["a0d"], 0, self.a0d, 0, G["cat0"], 0, acc)
-        lgdhip.call("lgdhip_upsample2_backward_bf16", G["cat0"].ptr, self.n // 2, G["cat0"].ld, 0, G["b1d"].ptr,
-                    c1, 0, c1, 0, S)
-        self._back("d1b", self.a1d, 0, G["b1d"], 0, self.b1d, 0, G["a1d"], 0, acc)
-        self._back("d1a", self.cat1, 0, G["a1d"], 0, self.a1d, 0, G["cat1"], 0, acc)
-        lgdhip.call("lgdhip_upsample2_backward_bf16", G["cat1"].ptr, self.n // 4, G["cat1"].ld, 0, G["b2d"].ptr,
-                    c2, 0, c2, 0, S)
-        self._back("d2b", self.a2d, 0, G["b2d"], 0, self.b2d, 0, G["a2d"], 0, acc)
-        self._back("d2a", self.cat2, 0, G["a2d"], 0, self.a2d, 0, G["cat2"], 0, acc)
-        lgdhip.call("lgdhip_upsample2_backward_bf16", G["cat2"].ptr, self.n // 8, G["cat2"].ld, 0, G["b3"].ptr,
-                    c3, 0, c3, 0, S)
-        self._back("e3b", self.a3, 0, G["b3"], 0, self.b3, 0, G["a3"], 0, acc)
-        self._back("e3a", self.p3, 0, G["a3"], 0, self.a3, 0, G["p3"], 0, acc)
-        lgdhip.call("lgdhip_avgpool2_backward_bf16", G["p3"].ptr, self.n // 4, c2, 0, G["cat2"].ptr,
-                    G["cat2"].ld, c3, c2, 1, S)
-        self._back("e2b", self.a2, 0, G["cat2"], c3, self.s2, 0, G["a2"], 0, acc)
-        self._back("e2a", self.p2, 0, G["a2"], 0, self.a2, 0, G["p2"], 0, acc)
-        lgdhip.call("lgdhip_avgpool2_backward_bf16", G["p2"].ptr, self.n // 2, c1, 0, G["cat1"].ptr,
-                    G["cat1"].ld, c2, c1, 1, S)
-        self._back("e1b", self.a1, 0, G["cat1"], c2, self.s1, 0, G["a1"], 0, acc)
-        self._back("e1a", self.p1, 0, G["a1"], 0, self.a1, 0, G["p1"], 0, acc)
-        lgdhip.call("lgdhip_avgpool2_backward_bf16", G["p1"].ptr, self.n, c0, 0, G["cat0"].ptr, G["cat0"].ld, c1,
-                    c0, 1, S)
-        self._back("e0b", self.a0, 0, G["cat0"], c1, self.s0, 0, G["a0"], 0, acc)
-        self._back("e0a", self.x, 0, G["a0"], 0, self.a0, 0, None, 0, acc)
+
+        def up(cat, m, g, act, c):
+            lgdhip.call("lgdhip_upsample2_backward_relu_bf16", G[cat].ptr, m, G[cat].ld, 0, G[g].ptr, c, 0, c, 0,
+                        act.ptr, act.ld, 0, self.stream)
+
+        def pool(p, n, cat, off, act, c):
+            lgdhip.call("lgdhip_avgpool2_backward_relu_bf16", G[p].ptr, n, c, 0, G[cat].ptr, G[cat].ld, off, c, 1,
+                        act.ptr, act.ld, 0, self.stream)
+
+        self._back("out", self.b0d, 0, self.gpred, 0, G["b0d"], acc, self.b0d)
+        self._back("d0b", self.a0d, 0, G["b0d"], 0, G["a0d"], acc, self.a0d)
+        self._back("d0a", self.cat0, 0, G["a0d"], 0, G["cat0"], acc)
+        up("cat0", self.n // 2, "b1d", self.b1d, c1)
+        self._back("d1b", self.a1d, 0, G["b1d"], 0, G["a1d"], acc, self.a1d)
+        self._back("d1a", self.cat1, 0, G["a1d"], 0, G["cat1"], acc)
+        up("cat1", self.n // 4, "b2d", self.b2d, c2)
+        self._back("d2b", self.a2d, 0, G["b2d"], 0, G["a2d"], acc, self.a2d)
+        self._back("d2a", self.cat2, 0, G["a2d"], 0, G["cat2"], acc)
+        up("cat2", self.n // 8, "b3", self.b3, c3)
+        self._back("e3b", self.a3, 0, G["b3"], 0, G["a3"], acc, self.a3)
+        self._back("e3a", self.p3, 0, G["a3"], 0, G["p3"], acc)
+        pool("p3", self.n // 4, "cat2", c3, self.s2, c2)
+        self._back("e2b", self.a2, 0, G["cat2"], c3, G["a2"], acc, self.a2)
+        self._back("e2a", self.p2, 0, G["a2"], 0, G["p2"], acc)
+        pool("p2", self.n // 2, "cat1", c2, self.s1, c1)
+        self._back("e1b", self.a1, 0, G["cat1"], c2, G["a1"], acc, self.a1)
+        self._back("e1a", self.p1, 0, G["a1"], 0, G["p1"], acc)
+        pool("p1", self.n, "cat0", c1, self.s0, c0)
+        self._back("e0b", self.a0, 0, G["cat0"], c1, G["a0"], acc, self.a0)
+        self._back("e0a", self.x, 0, G["a0"], 0, None, acc)
 
     def adam(self, lr: float = 1e-3, b1: float = 0.9, b2: float = 0.999, eps: float = 1e-8):
         """One Adam step on every layer (Adam is invariant to the gradient's

@@ -645,6 +645,75 @@ def test_relu_backward_rows(hip, c, ldg, offg, ldy, offy):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("n,cin,cout,ksize,lda,offa", [
+    (9, 1, 16, 1, 16, 0), (9, 1, 16, 1, 20, 4), (17, 16, 16, 3, 16, 0), (65, 32, 32, 3, 32, 0), (42, 32, 32, 3, 36, 4),
+    (33, 32, 32, 3, 32, 0), (32, 64, 64, 3, 64, 0), (42, 64, 64, 3, 72, 8), (19, 64, 16, 3, 18, 2), (16, 64, 64, 3, 64, 0),
+    (12, 128, 128, 3, 128, 0), (20, 24, 16, 3, 16, 0)])
+def test_conv_dgrad_relu(hip, n, cin, cout, ksize, lda, offa):
+    """The input gradient with the ReLU mask taken along (or, where the launch
+    does not take one, in a pass of its own) has the bits of the convolution
+    followed by the mask."""
+    rng = np.random.default_rng(n + cin + cout)
+    lib = hip.load()
+    kp = lib.lgdhip_conv3d_kpad(cin, ksize)
+    taps = 27 if ksize == 3 else 1
+    xb = dev(hip, to_bf16_bits(rng.standard_normal((n, n, n, cin)).astype(np.float32)))
+    w = bf16_round((rng.standard_normal((cout, taps, cin)) / 9).astype(np.float32))
+    wb = dev(hip, to_bf16_bits(conv_weights_layout(w, kp)))
+    a = rng.standard_normal((n, n, n, lda)).astype(np.float32)
+    a[rng.random(a.shape) < 0.2] = 0.0
+    a[rng.random(a.shape) < 0.02] = -0.0
+    ab = dev(hip, to_bf16_bits(a))
+    wsb = lib.lgdhip_conv3d_forward_workspace_bytes(n, cin, ksize, cout)
+    ws = hip.DeviceBuffer(max(wsb, 16))
+    print("[case] dgrad relu", n, cin, cout, ksize, lda, offa, flush=True)
+    out = []
+    for fused in (True, False):
+        y = dev(hip, np.full(n ** 3 * cout, 0x7FC0, np.uint16))
+        if fused:
+            hip.call("lgdhip_conv3d_bf16_dgrad_relu", xb.ptr, n, cin, 0, cin, ksize, wb.ptr, cout, y.ptr, cout, 0,
+                     ab.ptr, lda, offa, ws.ptr, wsb, None)
+        else:
+            hip.call("lgdhip_conv3d_bf16_forward_ws", xb.ptr, n, cin, 0, cin, ksize, wb.ptr, None, cout, y.ptr, cout, 0,
+                     None, 0, 0, 0, ws.ptr, wsb, None)
+            hip.call("lgdhip_relu_backward_bf16", y.ptr, cout, 0, ab.ptr, lda, offa, cout, n ** 3, None)
+        host = np.empty(n ** 3 * cout, np.uint16)
+        y.download(host)
+        out.append(host)
+    assert np.array_equal(out[0], out[1])
+    assert np.count_nonzero(out[0]) > 0.2 * out[0].size
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("c,ld,off,lda,offa", [(16, 16, 0, 16, 0), (16, 40, 8, 24, 8), (3, 5, 1, 4, 0)])
+@pytest.mark.parametrize("pool", [True, False])
+def test_resampling_gradient_relu(hip, pool, c, ld, off, lda, offa):
+    """The pooling and upsampling gradients through a ReLU: the bits of the
+    gradient followed by the mask, accumulating or not."""
+    rng = np.random.default_rng(c + ld)
+    n = 6  # dx's edge
+    m = n // 2 if pool else 2 * n
+    dyb = dev(hip, to_bf16_bits(rng.standard_normal((m, m, m, c)).astype(np.float32)))
+    ab = dev(hip, to_bf16_bits(rng.standard_normal((n, n, n, lda)).astype(np.float32)))
+    init = to_bf16_bits(rng.standard_normal((n, n, n, ld)).astype(np.float32))
+    name = "lgdhip_avgpool2_backward" if pool else "lgdhip_upsample2_backward"
+    for accumulate in (0, 1):
+        out = []
+        for fused in (True, False):
+            g = dev(hip, init)
+            args = (dyb.ptr, n, c, 0, g.ptr, ld, off, c, accumulate)
+            if fused:
+                hip.call(name + "_relu_bf16", *args, ab.ptr, lda, offa, None)
+            else:
+                hip.call(name + "_bf16", *args, None)
+                hip.call("lgdhip_relu_backward_bf16", g.ptr, ld, off, ab.ptr, lda, offa, c, n ** 3, None)
+            host = np.empty(n ** 3 * ld, np.uint16)
+            g.download(host)
+            out.append(host)
+        assert np.array_equal(out[0], out[1])
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("count,ld", [(1, 8), (3, 8), (8, 16)])
 def test_pack_rows(hip, count, ld):
     """Whole rows from separate fields: BF16 values, zeros past them, nothing
