@@ -1921,6 +1921,11 @@ int check_tensor(int n, int ld, int off, int c) {
     return 0;
 }
 
+int small_workspace() {
+    return lgdhip::set_error(LGDHIP_ERR_WORKSPACE,
+                             "forward workspace too small (lgdhip_conv3d_forward_workspace_bytes)");
+}
+
 // lgdhip_conv3d_bf16_forward_ws, with the ReLU mask of an activation where the
 // launch takes one along (masked_out; lda, offa its row stride and offset)
 int conv3d_forward(const void *x, int n, int ldx, int offx, int cin, int ksize, const void *w, const float *bias,
@@ -1982,7 +1987,12 @@ int conv3d_forward(const void *x, int n, int ldx, int offx, int cin, int ksize, 
         // (with one group the two orders are the same)
         const bool gemm_order =
             groups > 1 && (n < kZmGroupOrderN || groups > 6) && gemm_applies(n, cin, ksize, cout);
-        const int split = gemm_order ? gemm_plan(n, cin, cout, workspace != nullptr).slices : 0;
+        int split = 0;
+        if (gemm_order) {
+            const GemmPlan p = gemm_plan(n, cin, cout, workspace != nullptr);
+            if (workspace && workspace_bytes < gemm_workspace_bytes(n, p)) return small_workspace();
+            split = p.slices;
+        }
         if (groups >= 1 && (groups <= 6 || (groups <= 8 && (split || cout == 16))) && split <= 2) {
             const ZmPlan z = zm_plan(n, groups, cout);
             const unsigned wgs = (unsigned)((int64_t)z.bx * z.by * z.bz * z.slices), per = lgdhip::xcd_per(wgs);
@@ -2011,9 +2021,7 @@ int conv3d_forward(const void *x, int n, int ldx, int offx, int cin, int ksize, 
     }
     if (gemm_applies(n, cin, ksize, cout)) {
         const GemmPlan p = gemm_plan(n, cin, cout, workspace != nullptr);
-        if (workspace && workspace_bytes < gemm_workspace_bytes(n, p))
-            return lgdhip::set_error(LGDHIP_ERR_WORKSPACE,
-                                     "forward workspace too small (lgdhip_conv3d_forward_workspace_bytes)");
+        if (workspace && workspace_bytes < gemm_workspace_bytes(n, p)) return small_workspace();
         const unsigned blocks = (unsigned)((int64_t)p.mblocks * p.nblocks * p.slices);
         if (p.slices > 1) {
             // (gemm_plan splits only launches of fewer than 4 x 256 blocks)

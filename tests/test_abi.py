@@ -115,6 +115,18 @@ def test_conv_forward_workspace_without_gpu():
     assert rc == -3 and "workspace" in lib.lgdhip_last_error().decode()
 
 
+def test_conv_forward_small_workspace_refused_without_gpu():
+    """A workspace smaller than a layer asks for is refused also where the
+    launch would not use it (the z-marching kernel in two k slices)."""
+    lib = lgdhip.load()
+    need = lib.lgdhip_conv3d_forward_workspace_bytes(32, 32, 3, 64)
+    assert need > 0
+    fake = C.c_void_p(0x1000)
+    rc = lib.lgdhip_conv3d_bf16_forward_ws(fake, 32, 32, 0, 32, 3, fake, None, 64, fake, 64, 0, None, 1, 0, 0,
+                                           fake, need - 1, None)
+    assert rc == -3 and "workspace" in lib.lgdhip_last_error().decode()
+
+
 def test_jacobi_zrange_rejects_bad_ranges_without_gpu():
     lib = lgdhip.load()
     g = lgdhip.make_grid(3, 16, 16, 12, halo=1, elem_bytes=8)
