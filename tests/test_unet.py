@@ -860,3 +860,43 @@ def test_unet_gradients_vs_fp64_oracle(hip, oracle):
             if not (ew < tol_w and cos > tol_cos and eb < tol_w):
                 failures.append((bf16, name))
     assert not failures, failures
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,cin,cout,ld,off", [(16, 128, 128, 128, 0), (32, 16, 64, 72, 8), (24, 16, 48, 48, 0),
+                                               (21, 3, 24, 32, 8), (5, 8, 8, 8, 0), (64, 16, 16, 16, 0)])
+def test_conv_bias_grad_order(hip, n, cin, cout, ld, off):
+    """db of aligned rows: per chunk of 8192 voxels 256 interleaved sums and a
+    tree, then the chunks in order, bit for bit (a chain of 32 + 8 + chunks
+    additions instead of one thread's 8192 / (256 / cout)), accumulating or not."""
+    nvox = n ** 3
+    rng = np.random.default_rng(n + cout)
+    g = bf16_round((rng.standard_normal((nvox, ld)) * np.exp(rng.standard_normal((nvox, ld)))).astype(np.float32))
+    row = 8 if cin < 8 else cin
+    xb, gb = dev(hip, np.zeros(nvox * row, np.uint16)), dev(hip, to_bf16_bits(g))
+    lib = hip.load()
+    wsb = lib.lgdhip_conv3d_wgrad_workspace_bytes(n, cin, 3, cout, 0)
+    ws, dw = hip.DeviceBuffer(wsb), hip.DeviceBuffer(cout * lib.lgdhip_conv3d_kpad(cin, 3) * 4)
+    db = hip.DeviceBuffer(cout * 4)
+    print("[case] bias gradient", n, cout, ld, off, flush=True)
+    exp = np.zeros(cout, np.float32)
+    for v0 in range(0, nvox, 8192):
+        c = g[v0:v0 + 8192, off:off + cout]
+        lanes = np.zeros((256, cout), np.float32)
+        for r in range(0, len(c), 256):
+            part = c[r:r + 256]
+            lanes[:len(part)] += part
+        w = 128
+        while w:
+            lanes[:w] += lanes[w:2 * w]
+            w //= 2
+        exp += lanes[0]
+    for accumulate in (0, 1):
+        hip.call("lgdhip_conv3d_bf16_wgrad", xb.ptr, n, row, 0, cin, 3, gb.ptr, ld, off, cout, dw.ptr, db.ptr, accumulate,
+                 0, ws.ptr, wsb, None)
+        out = np.empty(cout, np.float32)
+        db.download(out)
+        assert np.array_equal(out, exp * (1 + accumulate))
+    ref = g[:, off:off + cout].astype(np.float64)
+    chain = 32 + 8 + (nvox + 8191) // 8192
+    assert np.all(np.abs(exp - ref.sum(0)) <= chain * 2.0 ** -24 * np.abs(ref).sum(0))
