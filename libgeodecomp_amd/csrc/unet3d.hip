@@ -502,8 +502,9 @@ constexpr int zm_ahead(int g, int nt) { return g * nt == 5 || g * nt == 6 ? 1 : 
 constexpr int zm_steps(int g, int split) { return split ? (27 * g + 3) / 4 : 7 * g; }
 constexpr int zm_second(int g) { return (zm_steps(g, 2) + 1) / 2 / 2 * 2; }
 // fragment reads in flight (at 6 groups the weights leave room for three: 48 ->
-// 16 at 128^3 133 us with six, 115 with three)
-constexpr int zm_reads(int g) { return g == 6 ? 3 : 6; }
+// 16 at 128^3 133 us with six, 115 with three; in tap-major order for two: 48 ->
+// 32 at 60^3 38.6 us with three, 32.6 with two)
+constexpr int zm_reads(int g, int split) { return g == 6 ? (split ? 2 : 3) : 6; }
 
 template <int G, int IN, int NT, int SPLIT, bool MASK>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(zm_waves(G, NT), zm_waves(G, NT)))) void
@@ -520,7 +521,10 @@ conv3d_fwd_zm(const u16 *__restrict__ X, int n, int ldx, int offx, int cin, cons
     // (60^3 32 -> 32 21.4 us unpadded, 20.0 padded, 48 -> 32 36.7 and 32.8; from 7
     // groups on the staging writes conflict instead and it lost 5 %)
     constexpr int PS = SPLIT && G <= 6 ? (PV + 15) / 16 * 16 : PV;
-    __shared__ uint4 ring[4][PS * G];
+    // the last SX + 1 pieces of a slot stay zero: what a lane past the last tap
+    // reads (its weights are zero, but zero times an infinite activation is NaN)
+    constexpr int ZERO = PS * G;
+    __shared__ uint4 ring[4][ZERO + SX + 1];
     unsigned b = lgdhip::xcd_tile(blockIdx.x, per, true);
     if (b >= groups) return;  // whole work-group, before any barrier
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -634,6 +638,7 @@ conv3d_fwd_zm(const u16 *__restrict__ X, int n, int ldx, int offx, int cin, cons
         vofs[r] = (y0 + 2 * wave + r) * n + x0 + i;
     }
 
+    if (tid < 4 * (SX + 1)) ring[tid / (SX + 1)][ZERO + tid % (SX + 1)] = make_uint4(0u, 0u, 0u, 0u);
     // prologue: planes z0-1, z0, z0+1 in slots 0..2, the next PF in flight
     plane_load(0, z0 - 1);
     plane_store(0, 0);
@@ -675,11 +680,13 @@ conv3d_fwd_zm(const u16 *__restrict__ X, int n, int ldx, int offx, int cin, cons
                 const int t0 = 4 * j / G, t1 = (4 * j + 3) / G < 27 ? (4 * j + 3) / G : t0;
                 const uint4 *p0 = slots[t0 / 9] + (4 * j - G * t0) * PS + t0 / 3 % 3 * SX + t0 % 3;
                 const uint4 *p1 = slots[t1 / 9] + (4 * j - G * t1) * PS + t1 / 3 % 3 * SX + t1 % 3;
-                // (past the last chunk, zero weights: any group of the tap)
-                const int gq = 4 * j + 3 < 27 * G || q < 27 * G - 4 * j ? q : 0;
-                pl = (t0 == t1 || 4 * j + q < G * t1 ? p0 : p1) + gq * PS + vox;
+                if (4 * j + 3 < 27 * G)
+                    pl = (t0 == t1 || 4 * j + q < G * t1 ? p0 : p1) + q * PS + vox;
+                else  // the last step, all of its chunks of tap 26
+                    pl = slots[2] + (q < 27 * G - 4 * j ? (4 * j - 26 * G + q) * PS + 2 * SX + 2 + vox : ZERO);
             } else {
                 pl = &ring[(st + tslot[j % 7]) & 3][j / 7 * PS + toff[j % 7]];
+                if (j % 7 == 6 && q == 3) pl = &ring[0][ZERO];
             }
             if (SPLIT == 2 && j == zm_second(G)) {
 #pragma unroll
@@ -702,7 +709,7 @@ conv3d_fwd_zm(const u16 *__restrict__ X, int n, int ldx, int offx, int cin, cons
         // schedule: kReads fragment reads in flight ahead of the products that
         // consume them (the compiler alone keeps about two, and the step then
         // waits out an LDS latency per k step)
-        constexpr int kReads = zm_reads(G);
+        constexpr int kReads = zm_reads(G, SPLIT);
         __builtin_amdgcn_sched_group_barrier(0x100, kReads, 0);
         lgdhip::static_for<0, 2 * STEPS - kReads>([&](auto) {
             __builtin_amdgcn_sched_group_barrier(0x008, NT, 0);

@@ -900,3 +900,56 @@ def test_conv_bias_grad_order(hip, n, cin, cout, ld, off):
     ref = g[:, off:off + cout].astype(np.float64)
     chain = 32 + 8 + (nvox + 8191) // 8192
     assert np.all(np.abs(exp - ref.sum(0)) <= chain * 2.0 ** -24 * np.abs(ref).sum(0))
+
+
+def infinite_voxels(n, channels):
+    """Voxels 3 or more apart (corners, edges and faces among them), each with
+    one of the channels in turn."""
+    at = [*range(0, n - 3, 5), n - 1]
+    vox = [(z, y, x) for z in at for y in at for x in at if (z * 7 + y * 3 + x) % 4 != 1]
+    return [(v, channels[k % len(channels)]) for k, v in enumerate(vox)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,cin,cout", [(16, 8, 48), (20, 3, 48), (65, 16, 32), (42, 16, 32), (43, 24, 48), (33, 24, 32),
+                                        (41, 32, 32), (42, 40, 32), (37, 40, 48), (41, 48, 64), (41, 56, 32), (33, 56, 48),
+                                        (42, 64, 32), (32, 64, 64)])
+def test_conv_zm_infinite_activations(hip, n, cin, cout):
+    """An infinite activation makes the outputs within its 27 taps infinite (by
+    the sign of the weight), none of them NaN, and leaves every other bit alone:
+    k positions past the last tap add nothing.  All k orders and input groups."""
+    rng = np.random.default_rng(n + cin + cout)
+    row = 8 if cin < 8 else cin
+    x = bf16_round(rng.standard_normal((n, n, n, row)).astype(np.float32))
+    w = bf16_round((rng.standard_normal((cout, 27, cin)) / np.sqrt(27 * cin)).astype(np.float32))
+    w[w == 0] = 0.5
+    spots = infinite_voxels(n, list(range(cin)))
+    finite, xi = x.copy(), x.copy()
+    for k, (v, c) in enumerate(spots):
+        finite[v + (c,)] = 0.0
+        xi[v + (c,)] = np.inf if k % 3 else -np.inf
+    lib = hip.load()
+    kp = lib.lgdhip_conv3d_kpad(cin, 3)
+    wb = dev(hip, to_bf16_bits(conv_weights_layout(w, kp)))
+    wsb = lib.lgdhip_conv3d_forward_workspace_bytes(n, cin, 3, cout)
+    ws = hip.DeviceBuffer(max(wsb, 16))
+    print("[case] conv z-march infinities", n, cin, cout, flush=True)
+
+    def run(values, relu):
+        xb, y = dev(hip, to_bf16_bits(values)), hip.DeviceBuffer(n ** 3 * cout * 2)
+        hip.call("lgdhip_conv3d_bf16_forward_ws", xb.ptr, n, row, 0, cin, 3, wb.ptr, None, cout, y.ptr, cout, 0, None,
+                 0, relu, 0, ws.ptr, wsb, None)
+        out = np.empty(n ** 3 * cout, np.uint16)
+        y.download(out)
+        return from_bf16_bits(out).reshape(n, n, n, cout)
+
+    for relu in (0, 1):
+        exp, out = run(finite, relu), run(xi, relu)
+        for v, c in spots:
+            for tap in range(27):
+                u = (v[0] - (tap // 9 - 1), v[1] - (tap // 3 % 3 - 1), v[2] - (tap % 3 - 1))
+                if min(u) < 0 or max(u) >= n:
+                    continue
+                o = w[:, tap, c] * xi[v + (c,)]
+                exp[u] = np.where(o > 0, o, 0) if relu else o
+        assert np.array_equal(out, exp)
