@@ -1275,6 +1275,7 @@ __global__ __launch_bounds__(64 * TI * TO * KS, TI * TO * KS == 4 ? 3 : 1) void 
     constexpr int kStage = 2 * (PX + PY);                      // uint4: [X buffers][dY buffers]
     constexpr int kRed = KS > 1 ? KS / 2 * TI * TO * 9 * 64 : 0;  // uint4 (4 floats): a dz's accumulators of half the waves
     __shared__ uint4 smem[kStage > kRed ? kStage : kRed];
+    __shared__ int overflow;
     uint4 *const xs = smem, *const ys = smem + 2 * PX;
     unsigned b = lgdhip::xcd_tile(blockIdx.x, per, true);
     if (b >= groups) return;  // whole work-group, before any barrier
@@ -1365,28 +1366,20 @@ __global__ __launch_bounds__(64 * TI * TO * KS, TI * TO * KS == 4 ? 3 : 1) void 
     };
 
     f32x4 acc[3][9];
-#pragma unroll
-    for (int d = 0; d < 3; ++d)
-#pragma unroll
-        for (int e = 0; e < 9; ++e) acc[d][e] = f32x4{0.f, 0.f, 0.f, 0.f};
     Frag a[3][NKS];  // dY of planes z + 1, z, z - 1
+    auto clear = [&]() __attribute__((always_inline)) {
 #pragma unroll
-    for (int d = 0; d < 3; ++d)
+        for (int d = 0; d < 3; ++d) {
 #pragma unroll
-        for (int s = 0; s < NKS; ++s) a[d][s].q = make_uint4(0u, 0u, 0u, 0u);
-
-    load_x(0, zs - 1);
-    load_y(0, zs);
-    load_x(1, zs);
-    load_y(1, zs + 1);
-    store_xy(0, 0);
-    __syncthreads();
-    // step at X plane z (dY plane z + 1) in buffer PH: the planes of step z + 2 go
-    // out, those of z + 1 (in flight for a whole step) are stored after the products
-    auto plane = [&](auto ph_c, int z) __attribute__((always_inline)) {
+            for (int e = 0; e < 9; ++e) acc[d][e] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int s = 0; s < NKS; ++s) a[d][s].q = make_uint4(0u, 0u, 0u, 0u);
+        }
+    };
+    // the products of X plane z, in buffer PH with dY plane z + 1
+    auto products = [&](auto ph_c, auto masked_c, int z) __attribute__((always_inline)) {
         constexpr int PH = decltype(ph_c)::value;
-        load_x(PH, z + 2);
-        load_y(PH, z + 3);
+        constexpr bool MASKED = decltype(masked_c)::value;
 #pragma unroll
         for (int s = 0; s < NKS; ++s) {
             const int step = ks + KS * s;  // rows 2 step, 2 step + 1
@@ -1394,23 +1387,81 @@ __global__ __launch_bounds__(64 * TI * TO * KS, TI * TO * KS == 4 ? 3 : 1) void 
             a[1][s] = a[0][s];
             a[0][s] = frag(ylane + PH * PY * 16 + step * 2 * 16 * 32);
             const lc_ptr xp = xlane + PH * PX * 16 + step * 2 * kWgX * 32;
+            uint32_t in[4];  // MASKED: the fragment's voxels whose dY is inside the volume
+            if (MASKED) {
+#pragma unroll
+                for (int w = 0; w < 4; ++w) {
+                    const int xx = x0 + 4 * (q & 1) + 8 * (w / 2) + 2 * (w % 2);
+                    const bool yin = y0 + 2 * step + row < n;
+                    in[w] = (yin && xx < n ? 0xFFFFu : 0u) | (yin && xx + 1 < n ? 0xFFFF0000u : 0u);
+                }
+            }
 #pragma unroll
             for (int e = 0; e < 9; ++e) {  // tap (dy, dx) = (e / 3 - 1, e % 3 - 1)
                 const Frag f = frag(xp + ((e / 3) * kWgX + e % 3) * 32);
 #pragma unroll
-                for (int d = 0; d < 3; ++d)
-                    acc[d][e] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[d][s].v, f.v, acc[d][e], 0, 0, 0);
+                for (int d = 0; d < 3; ++d) {
+                    Frag g = f;
+                    if (MASKED) {
+                        const uint32_t zin = z + 1 - d >= zs && z + 1 - d < ze ? ~0u : 0u;
+                        g.q = make_uint4(f.q.x & in[0] & zin, f.q.y & in[1] & zin, f.q.z & in[2] & zin,
+                                         f.q.w & in[3] & zin);
+                    }
+                    acc[d][e] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[d][s].v, g.v, acc[d][e], 0, 0, 0);
+                }
             }
         }
-        store_xy(PH ^ 1, PH ^ 1);
-        __syncthreads();
+    };
+
+    if (tid == 0) overflow = 0;
+    clear();
+    load_x(0, zs - 1);
+    load_y(0, zs);
+    load_x(1, zs);
+    load_y(1, zs + 1);
+    store_xy(0, 0);
+    __syncthreads();
+    // step at X plane z (dY plane z + 1) in buffer PH: the planes of step z + 2 go
+    // out, those of z + 1 (in flight for a whole step) are stored after the products;
+    // LAST: z may be (1) or is (2) the last plane, after which nothing is stored
+    auto plane = [&](auto ph_c, auto last_c, int z) __attribute__((always_inline)) {
+        constexpr int PH = decltype(ph_c)::value, LAST = decltype(last_c)::value;
+        load_x(PH, z + 2);
+        load_y(PH, z + 3);
+        products(ph_c, lgdhip::ic<0>{}, z);
+        if (LAST == 0 || (LAST == 1 && z < ze)) {
+            store_xy(PH ^ 1, PH ^ 1);
+            __syncthreads();
+        }
     };
     int z = zs - 1;
     for (; z + 1 <= ze; z += 2) {
-        plane(lgdhip::ic<0>{}, z);
-        plane(lgdhip::ic<1>{}, z + 1);
+        plane(lgdhip::ic<0>{}, lgdhip::ic<0>{}, z);
+        plane(lgdhip::ic<1>{}, lgdhip::ic<1>{}, z + 1);
     }
-    if (z <= ze) plane(lgdhip::ic<0>{}, z);
+    if (z <= ze) plane(lgdhip::ic<0>{}, lgdhip::ic<2>{}, z);
+    // Voxels outside the chunk or the volume add dY = 0 times a real X, which is
+    // NaN where that X is infinite.  If a sum is not finite, the chunk is summed
+    // again without those X, one plane at a time; on finite tensors the test costs
+    // up to 1.4 us a launch (128^3 16 -> 16 40.9 us without, 41.5 with, 64^3 32 ->
+    // 32 26.5 and 27.9).  Masks in the march itself spilled 20 to 290 registers.
+    f32x4 sum = acc[0][0];
+#pragma unroll
+    for (int k = 1; k < 27; ++k) sum += acc[k / 9][k % 9];
+    const float all = sum[0] + sum[1] + sum[2] + sum[3];
+    if (!(fabsf(all) < INFINITY)) overflow = 1;
+    __syncthreads();
+    if (__builtin_expect(overflow != 0, 0)) {
+        clear();
+        for (z = zs - 1; z <= ze; ++z) {
+            load_x(0, z);
+            load_y(0, z + 1);
+            store_xy(0, 0);
+            __syncthreads();
+            products(lgdhip::ic<0>{}, lgdhip::ic<1>{}, z);
+            __syncthreads();
+        }
+    }
     // sum the KS waves of each tile pair, one dz at a time: the upper half of the
     // waves writes, the lower half adds
     if (KS > 1) {

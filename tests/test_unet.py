@@ -953,3 +953,50 @@ def test_conv_zm_infinite_activations(hip, n, cin, cout):
                 o = w[:, tap, c] * xi[v + (c,)]
                 exp[u] = np.where(o > 0, o, 0) if relu else o
         assert np.array_equal(out, exp)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,cin,cout", [(16, 16, 16), (17, 16, 16), (13, 24, 40), (33, 3, 16), (20, 3, 48), (31, 64, 128),
+                                        (32, 64, 32), (30, 96, 128), (45, 48, 128), (64, 32, 16), (1, 16, 16)])
+def test_conv_wgrad_infinite_activations(hip, n, cin, cout):
+    """An infinite activation makes the weight gradients of its channel infinite
+    (by the sign of the output gradient) for the taps that reach it inside the
+    volume, and leaves the others' bits alone: no voxel outside a column, a
+    chunk of planes or the volume adds to a sum."""
+    rng = np.random.default_rng(n + cin + cout)
+    row = 8 if cin < 8 else cin
+    x = bf16_round(rng.standard_normal((n, n, n, row)).astype(np.float32))
+    g = bf16_round(rng.standard_normal((n, n, n, cout)).astype(np.float32))
+    g[g == 0] = 0.5
+    lib = hip.load()
+    kp = lib.lgdhip_conv3d_kpad(cin, 3)
+    wsb = lib.lgdhip_conv3d_wgrad_workspace_bytes(n, cin, 3, cout, 0)
+    ws, dw = hip.DeviceBuffer(wsb), hip.DeviceBuffer(cout * kp * 4)
+    gb = dev(hip, to_bf16_bits(g))
+    print("[case] conv wgrad infinities", n, cin, cout, flush=True)
+
+    def run(values):
+        xb = dev(hip, to_bf16_bits(values))
+        hip.call("lgdhip_conv3d_bf16_wgrad", xb.ptr, n, row, 0, cin, 3, gb.ptr, cout, 0, cout, dw.ptr, None, 0, 0,
+                 ws.ptr, wsb, None)
+        out = np.empty((cout, kp), np.float32)
+        dw.download(out)
+        return out[:, :27 * cin].reshape(cout, 27, cin).copy()
+
+    # one infinite voxel per channel and pass: faces, edges, corners, and around
+    # the borders of columns (16 x 8) and chunks (powers of two) of the volume
+    near = sorted({min(n - 1, max(0, b + d)) for b in (0, 8, 16, 32, n) for d in (-2, -1, 0, 1)})
+    for _ in range(3):
+        finite, xi, spots = x.copy(), x.copy(), []
+        for c in range(cin):
+            v = tuple(int(k) for k in rng.choice(near, 3))
+            finite[v + (c,)] = 0.0
+            xi[v + (c,)] = np.inf if c % 3 else -np.inf
+            spots.append(v)
+        exp, out = run(finite), run(xi)
+        for c, v in enumerate(spots):
+            for tap in range(27):
+                u = (v[0] - (tap // 9 - 1), v[1] - (tap // 3 % 3 - 1), v[2] - (tap % 3 - 1))
+                if min(u) >= 0 and max(u) < n:
+                    exp[:, tap, c] = g[u] * xi[v + (c,)]
+        assert np.array_equal(out, exp)
