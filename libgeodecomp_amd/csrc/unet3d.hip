@@ -476,7 +476,10 @@ __device__ __forceinline__ uint32_t positive_halves(uint32_t w) {
 //
 // The k order is that of the kernel that takes the layer when this one does not
 // (accumulation, unaligned rows), so a layer's result has the same bits either
-// way.  SPLIT = 0: conv3d_fwd_lds's, group-major, 4 taps of one group per step.
+// way, with two exceptions that differ by roundings of the FP32 sums: plain
+// launches of 2 to 6 groups and more than 32 output channels on 96^3 and larger
+// (kZmGroupOrderN), and masked rows with more than 32 output channels, which
+// conv3d_fwd_mfma takes otherwise.  SPLIT = 0: conv3d_fwd_lds's, group-major, 4 taps of one group per step.
 // SPLIT = 1: conv3d_fwd_gemm's, the weights' tap-major rows, 4 groups (of one
 // tap or two) per step.  SPLIT = 2: the same in conv3d_fwd_gemm's two slices of
 // its stages, each summed from zero and then added.
@@ -1033,9 +1036,9 @@ __global__ __launch_bounds__(256) void conv1x1_to1_wgrad(const u16 *__restrict__
 // the LDS-staged kernel takes 3x3x3 layers with up to 32 output channels on
 // volumes of at least 16^3
 constexpr int kLdsMinN = 16;
-// layers of up to 48 input and more than 32 output channels: in the LDS-tile
-// kernel's k order from this edge on where the z-marching kernel takes them,
-// below it in the GEMM-tiled kernel's
+// layers of 16 to 48 input and more than 32 output channels: a plain BF16 output
+// (16-byte aligned, no FP32 copy) is summed in the LDS-tile kernel's k order from
+// this edge on, below it, as all their other outputs, in the GEMM-tiled kernel's
 constexpr int kZmGroupOrderN = 96;
 
 // The GEMM-tiled kernel's launch: 64 x 64 blocks, stages of 64 k, and the
@@ -2080,8 +2083,9 @@ int conv3d_forward(const void *x, int n, int ldx, int offx, int cin, int ksize, 
                             ((uintptr_t)x & 15) == 0;
         const int groups = (cin & 7) == 0 ? cin / 8 : (masked ? 1 : 0);
         // (with one group the two orders are the same)
-        const bool gemm_order =
-            groups > 1 && (n < kZmGroupOrderN || groups > 6) && gemm_applies(n, cin, ksize, cout);
+        const bool plain = y && !y32 && (ldy & 7) == 0 && (offy & 7) == 0 && ((uintptr_t)y & 15) == 0;
+        const bool gemm_order = groups > 1 && (n < kZmGroupOrderN || groups > 6 || !plain) &&
+                                gemm_applies(n, cin, ksize, cout);
         int split = 0;
         if (gemm_order) {
             const GemmPlan p = gemm_plan(n, cin, cout, workspace != nullptr);

@@ -1000,3 +1000,42 @@ def test_conv_wgrad_infinite_activations(hip, n, cin, cout):
                 if min(u) >= 0 and max(u) < n:
                     exp[:, tap, c] = g[u] * xi[v + (c,)]
         assert np.array_equal(out, exp)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,cin,cout", [(97, 16, 48), (96, 40, 64), (20, 3, 48)])
+def test_conv_zm_other_orders(hip, n, cin, cout):
+    """Layers whose plain 16-byte-aligned launch sums in another k order than
+    the kernel of their accumulating launch: more than 32 output channels on
+    96^3 and larger (group-major against tap-major), and a masked row.  There
+    the two agree within K accumulated roundings, and the FP32 output and an
+    8-byte-aligned one of 96^3 and larger have the accumulating launch's bits."""
+    rng = np.random.default_rng(n + cin)
+    row = 8 if cin < 8 else cin
+    x = bf16_round(rng.standard_normal((n ** 3, row)).astype(np.float32))
+    w = bf16_round((rng.standard_normal((cout, 27, cin)) / np.sqrt(27 * cin)).astype(np.float32))
+    lib = hip.load()
+    kp = lib.lgdhip_conv3d_kpad(cin, 3)
+    wsb = lib.lgdhip_conv3d_forward_workspace_bytes(n, cin, 3, cout)
+    ws = hip.DeviceBuffer(max(wsb, 16))
+    print("[case] conv z-march other orders", n, cin, cout, flush=True)
+
+    def run(x, w, ld=None, off=0, accumulate=0):
+        xb, wb = dev(hip, to_bf16_bits(x)), dev(hip, to_bf16_bits(conv_weights_layout(w, kp)))
+        f32 = ld is None
+        y = dev(hip, np.zeros(n ** 3 * (cout if f32 else ld), np.float32 if f32 else np.uint16))
+        hip.call("lgdhip_conv3d_bf16_forward_ws", xb.ptr, n, row, 0, cin, 3, wb.ptr, None, cout, None if f32 else y.ptr,
+                 ld or 0, off, y.ptr if f32 else None, cout if f32 else 0, 0, accumulate, ws.ptr, wsb, None)
+        out = np.empty(n ** 3 * (cout if f32 else ld), np.float32 if f32 else np.uint16)
+        y.download(out)
+        return out.reshape(n ** 3, -1)[:, off:off + cout]
+
+    other = run(x, w, cout, accumulate=1)
+    y32 = run(x, w)
+    if n >= 96:
+        assert np.array_equal(to_bf16_bits(y32), other)
+        assert np.array_equal(run(x, w, cout + 4, 4), other)
+    mag = run(np.abs(x), np.abs(w))
+    bound = 2 * (27 * cin + 2) * 2.0 ** -24 * 1.001 * mag  # both orders' sums; then BF16 of each
+    for bits in (other, run(x, w, cout)):
+        assert np.all(np.abs(from_bf16_bits(bits) - y32) <= bound + 2.0 ** -8 * np.abs(y32) + 1e-30)
