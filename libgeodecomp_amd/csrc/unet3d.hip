@@ -1996,8 +1996,13 @@ ZmWgrad wgrad_zm_plan(int n, int cin, int cout) {
 
 // Voxels per chunk of the general kernel when the caller leaves it to the
 // library (chunk_vox <= 0): the largest power of two <= 4096 (and >= 128) that
-// still gives the launch 2048 waves (8 per CU) in its wave split, since each
-// wave marches its chunk 32 voxels per dependent step.
+// gives 2048 tasks.  A task is a wave's 16 columns of k, but for layers of whole
+// 16-channel tiles on n % 8 == 0 up to 4 x 4 tiles (a single one with 9 taps, few
+// with 3): their chunks stay 2 to 8 times shorter than 2048 waves would need, and
+// the shorter serial sums are both faster and nearer to the 64-bit sums.  MI355X,
+// chunks of this length / of 2048 waves, us and relative error: 64^3 16 -> 16 97,
+// 2.3e-7 / 115, 3.0e-7; 64^3 32 -> 32 213, 2.4e-7 / 288, 4.2e-7; 32^3 64 -> 64 90,
+// 1.5e-7 / 108, 2.2e-7; 32^3 192 -> 64 248, 2.2e-7 / 327, 4.1e-7.
 int wgrad_chunk(int n, int cin, int ksize, int cout) {
     const int64_t nvox = (int64_t)n * n * n;
     int64_t tasks = lgdhip_conv3d_kpad(cin, ksize) / 16;

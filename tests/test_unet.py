@@ -420,10 +420,10 @@ def test_conv_wgrad_default_chunk(hip, oracle, n, cin, cout, ksize):
 
 def test_conv_wgrad_default_chunk_sizes():
     """The library's chunk (chunk_vox = 0) for the U-Net's levels, read off
-    the workspace size: 4096 voxels while that gives 2048 waves (128^3, 48
-    -> 16 channels: 512 chunks x 9 waves), smaller elsewhere (128^3 16 ->
-    16, one wave per dz: 2048; 32^3 64 -> 64: 256; 16^3 128 -> 128: 128),
-    never below 128."""
+    the workspace size: the largest power of two from 128 to 4096 that gives
+    2048 tasks of up to 4 x 4 channel tiles (128^3: 16 -> 16 3 tasks a chunk,
+    2048 voxels, 48 -> 16 9 tasks, 4096; 32^3 64 -> 64: 256; 16^3 128 -> 128:
+    128)."""
     lib = lgdhip.load()
     for n, cin, cout, chunk in [(128, 16, 16, 2048), (128, 48, 16, 4096), (64, 32, 32, 1024), (32, 64, 64, 256),
                                 (16, 128, 128, 128), (128, 3, 16, 4096), (8, 16, 16, 128)]:
