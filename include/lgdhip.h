@@ -311,6 +311,12 @@ int lgdhip_life2d_packed_run(uint32_t *pa, uint32_t *pb, const lgdhip_grid *g,
 int lgdhip_life2d_packed_run_periodic(uint32_t *pa, uint32_t *pb, const lgdhip_grid *g, int edge_alive, int steps,
                                       int wrap_mask, const lgdhip_tile *tile, int *result_in_b,
                                       lgdhip_stream_t stream);
+/* The launch a run of `steps` generations resolves to: stacked waves per
+ * work-group, register rows per wave and generations per launch (a requested
+ * variant's, or the default's choice for the grid).  No device work; for
+ * tools.  No counterpart in the reference. */
+int lgdhip_life2d_plan(const lgdhip_grid *g, int steps, int wrap_mask, const lgdhip_tile *tile, int *waves, int *rows,
+                       int *generations);
 /* uint8 grid in, uint8 grid out (in place): pack -> packed_run -> unpack.
  * `workspace` must hold lgdhip_life2d_workspace_bytes(g) bytes. */
 size_t lgdhip_life2d_workspace_bytes(const lgdhip_grid *g);

@@ -499,9 +499,6 @@ int packed_launch(const uint32_t *src, uint32_t *dst, int nw, int ny, uint32_t l
     case 1: case 2: launch_rows<128>(src, dst, nw, ny, last_mask, edge, gens, halo_rows, variant == 1, wrap, s); break;
     case 3: case 4: launch_rows<64>(src, dst, nw, ny, last_mask, edge, gens, halo_rows, variant == 3, wrap, s); break;
     case 5: launch_stacked<64, 4>(src, dst, nw, ny, last_mask, edge, gens, halo_rows, wrap, s); break;
-    case 6: shape = LifeShape{8, 64, halo_rows}; break;
-    case 7: shape = LifeShape{8, 32, halo_rows}; break;
-    case 8: shape = LifeShape{16, 32, halo_rows}; break;
     default: break;
     }
 #define LGD_LIFE_CASE(NW, R)                                                                                    \
@@ -527,40 +524,53 @@ int check_life_grid(const lgdhip_grid *g) {
     return 0;
 }
 
-// K generations per launch over the packed words; wrap bits 1 (x) and 2 (y):
-// the axes taken periodic (x only when nx % 32 == 0: columns wrap word by word)
-int packed_run(uint32_t *pa, uint32_t *pb, const lgdhip_grid *g, int edge_alive, int steps, int wrap,
-               const lgdhip_tile *tile, int *result_in_b, lgdhip_stream_t stream) {
+// The variant and shape (waves, rows per wave, generations per launch) of a run.
+int packed_plan(const lgdhip_grid *g, int steps, int wrap, const lgdhip_tile *tile, int *variant, LifeShape *shape) {
     int rc = lgdhip::check_grid(g, 2, 1, 1);
     if (rc) return rc;
     if ((wrap & 1) && g->nx % 32 != 0)
         return lgdhip::set_error(LGDHIP_ERR_UNSUPPORTED, "a wrapped x axis needs nx % 32 == 0 (whole words)");
-    LGD_REQUIRE(pa && pb && pa != pb, "need two distinct device buffers");
     LGD_REQUIRE(steps >= 0, "steps must be >= 0");
-    LGD_REQUIRE(edge_alive == 0 || edge_alive == 1, "edge_alive must be 0 or 1");
-    int per_launch = 0, variant = 0;
+    int per_launch = 0;
+    *variant = 0;
     if (tile) {
         if (tile->steps_per_launch > 0) per_launch = tile->steps_per_launch;
-        variant = tile->variant;
+        *variant = tile->variant;
     }
-    if (variant < 0 || variant > kNumVariants) return lgdhip::set_error(LGDHIP_ERR_UNSUPPORTED, "unknown life variant");
-    if (variant != 0 && per_launch == 0) per_launch = kDefaultPerLaunch;
+    if (*variant < 0 || *variant > kNumVariants)
+        return lgdhip::set_error(LGDHIP_ERR_UNSUPPORTED, "unknown life variant");
+    if (*variant != 0 && per_launch == 0) per_launch = kDefaultPerLaunch;
     // a lane's neighbour word covers 32 cells, so at most 32 generations may
     // run before the halo lanes' garbage reaches an output column; the
     // register rows must keep at least one valid row per band
-    if (per_launch < 0 || per_launch > 32 || (variant != 0 && 2 * per_launch >= rows_per_group(variant)))
+    if (per_launch > 32 || (*variant != 0 && 2 * per_launch >= rows_per_group(*variant)))
         return lgdhip::set_error(LGDHIP_ERR_UNSUPPORTED,
                                  "steps_per_launch must be in [1, 32] and below half the register rows");
+    if (*variant == 0) {
+        *shape = life_plan((int)((g->nx + 31) / 32), (int)g->ny, wrap, steps, per_launch);
+    } else {
+        const int waves = *variant < 5 ? 1 : (*variant == 5 ? 4 : (*variant < 8 ? 8 : 16));
+        *shape = LifeShape{waves, rows_per_group(*variant) / waves, per_launch};
+    }
+    return 0;
+}
+
+// K generations per launch over the packed words; wrap bits 1 (x) and 2 (y):
+// the axes taken periodic (x only when nx % 32 == 0: columns wrap word by word)
+int packed_run(uint32_t *pa, uint32_t *pb, const lgdhip_grid *g, int edge_alive, int steps, int wrap,
+               const lgdhip_tile *tile, int *result_in_b, lgdhip_stream_t stream) {
+    LifeShape shape{};
+    int variant = 0;
+    int rc = packed_plan(g, steps, wrap, tile, &variant, &shape);
+    if (rc) return rc;
+    LGD_REQUIRE(pa && pb && pa != pb, "need two distinct device buffers");
+    LGD_REQUIRE(edge_alive == 0 || edge_alive == 1, "edge_alive must be 0 or 1");
+    const int per_launch = shape.gens;
     const int nw = (int)((g->nx + 31) / 32);
     const int rem = (int)(g->nx - 32 * (int64_t)(nw - 1));
     const uint32_t last_mask = rem >= 32 ? 0xFFFFFFFFu : ((1u << rem) - 1u);
     const uint32_t edge = edge_alive ? 0xFFFFFFFFu : 0u;
     hipStream_t s = lgdhip::as_stream(stream);
-    LifeShape shape{0, 0, per_launch};
-    if (variant == 0) {
-        shape = life_plan(nw, (int)g->ny, wrap, steps, per_launch);
-        per_launch = shape.gens;
-    }
     uint32_t *cur = pa, *nxt = pb;
     for (int done = 0; done < steps;) {
         const int gens = (steps - done < per_launch) ? (steps - done) : per_launch;
@@ -599,6 +609,20 @@ int lgdhip_life2d_u8_run(uint8_t *a, uint8_t *b, const lgdhip_grid *g, int steps
         nxt = tmp;
     }
     if (result_in_b) *result_in_b = (cur == b) ? 1 : 0;
+    return 0;
+}
+
+int lgdhip_life2d_plan(const lgdhip_grid *g, int steps, int wrap_mask, const lgdhip_tile *tile, int *waves, int *rows,
+                       int *generations) {
+    LGD_REQUIRE(waves && rows && generations, "NULL output pointer");
+    LGD_REQUIRE(wrap_mask >= 0 && wrap_mask <= 3, "wrap_mask must be a combination of bits 1, 2");
+    LifeShape shape{};
+    int variant = 0;
+    const int rc = packed_plan(g, steps, wrap_mask, tile, &variant, &shape);
+    if (rc) return rc;
+    *waves = shape.waves;
+    *rows = shape.rows;
+    *generations = shape.gens;
     return 0;
 }
 

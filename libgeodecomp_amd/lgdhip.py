@@ -145,6 +145,7 @@ SIGNATURES = {
     "lgdhip_life2d_pack": (_I, [_P, _GP, _P, _P]),
     "lgdhip_life2d_unpack": (_I, [_P, _GP, _P, _P]),
     "lgdhip_life2d_packed_run": (_I, [_P, _P, _GP, _I, _I, _TP, _IP, _P]),
+    "lgdhip_life2d_plan": (_I, [_GP, _I, _I, _TP, _IP, _IP, _IP]),
     "lgdhip_life2d_packed_run_periodic": (_I, [_P, _P, _GP, _I, _I, _I, _TP, _IP, _P]),
     "lgdhip_life2d_workspace_bytes": (_SZ, [_GP]),
     "lgdhip_life2d_run": (_I, [_P, _GP, _I, _I, _P, _SZ, _TP, _P]),

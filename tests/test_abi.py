@@ -188,6 +188,27 @@ def test_poisson_sweep_plan_without_gpu():
     assert plan([128] * 16, 5) == 5 and plan(ensemble, 3) == 3
 
 
+def test_life_plan_without_gpu():
+    """lgdhip_life2d_plan (host-only): the default's waves, rows and generations
+    per launch, a requested variant's and depth's, and the run's refusals."""
+    lib = lgdhip.load()
+
+    def plan(nx, ny, steps, wrap=0, **tile):
+        g = lgdhip.make_grid(2, nx, ny, 1, halo=1, elem_bytes=1)
+        t = lgdhip.tile(**tile) if tile else None
+        v = [C.c_int(-1) for _ in range(3)]
+        rc = lib.lgdhip_life2d_plan(C.byref(g), steps, wrap, C.byref(t) if t else None, *(C.byref(k) for k in v))
+        return rc if rc else tuple(k.value for k in v)
+
+    assert plan(16384, 16384, 1000) == (16, 20, 25)
+    assert plan(1000, 777, 100)[:2] == (8, 4)
+    assert plan(16384, 16384, 1000, steps_per_launch=31)[2] == 31
+    assert plan(300, 200, 40, variant=7) == (8, 32, 31)
+    assert plan(300, 200, 40, variant=1, steps_per_launch=9) == (1, 128, 9)
+    assert plan(300, 200, 40, steps_per_launch=33) == -2 and plan(300, 200, 40, variant=9) == -2
+    assert plan(300, 200, 40, wrap=1) == -2 and plan(300, 200, 40, wrap=4) == -1 and plan(300, 200, -1) == -1
+
+
 def test_new_entry_points_reject_bad_arguments_without_gpu():
     """Argument checks that return before any device work: the plan queries
     need their output pointers and valid problems; weighted sweeps need

@@ -8,7 +8,7 @@ errors on rho and j.
 import numpy as np
 import pytest
 
-from libgeodecomp_amd import synthetic
+from libgeodecomp_amd import lgdhip, synthetic
 from test_oracle import encode, jacobi_kat_expected, jacobi_kat_input, place
 
 pytestmark = pytest.mark.gpu
@@ -292,23 +292,79 @@ def test_life_packed_periodic_bit_exact(hip, oracle, shape):
 
 
 @pytest.mark.parametrize("nx,ny,steps,per_launch,wrap", [
-    (1000, 777, 100, 0, 0),     # low work-groups, two bands per wave
+    (1000, 777, 100, 0, 0),     # 8 waves x 4 rows, a span of 33 columns
     (1984, 40, 33, 0, 3),       # 62 words a row: a span of 64 columns, one band
     (1999, 2051, 60, 0, 2),     # ragged last word, bands cut at every column
-    (4096, 4100, 45, 0, 0),     # 16 stacked waves, low bands
-    (8190, 8193, 27, 0, 0),     # taller ones, the last band almost empty
+    (4096, 4100, 45, 0, 0),     # 16 x 4 rows
+    (8190, 8193, 27, 0, 0),     # 16 x 12 rows, the last band almost empty
     (8192, 8193, 27, 27, 1),    # images of the wrapped x axis inside a work-group
-    (16384, 16500, 26, 25, 0),  # the tallest work-groups
+    (16384, 16500, 26, 25, 0),  # 8 x 24 rows, a last launch of one generation
 ])
 def test_life_packed_default_shapes(hip, oracle, nx, ny, steps, per_launch, wrap):
-    """The default variant's work-group heights and launch depths on grids
-    from a fraction of the chip to several rounds of it, both edge states."""
+    """The default variant against the oracle on grids from a fraction of the
+    chip to several rounds of it, both edge states (every work-group shape:
+    test_life_packed_every_default_shape)."""
     say("life default", nx, ny, "steps", steps, "wrap", wrap)
     g0 = synthetic.life_initial(nx, ny, seed=nx + 11 * ny)
     edge = (nx + ny) % 2
     t = hip.tile(steps_per_launch=per_launch) if per_launch else None
     exp = oracle.life2d(g0, steps, edge=edge, threads=16, wrap=wrap)
     assert np.array_equal(gpu_life_packed_periodic(hip, g0, steps, wrap, edge=edge, tile=t), exp)
+
+
+# boards on which each shape of the default variant (waves, rows per wave) is
+# chosen: (waves, rows, nx, ny, steps, steps_per_launch, wrap)
+LIFE_PLAN_BOARDS = [
+    (8, 4, 263, 64, 70, 0, 0), (8, 4, 256, 64, 5, 0, 3), (8, 8, 105141, 405, 26, 14, 0),
+    (8, 8, 127488, 322, 70, 14, 3), (8, 12, 101872, 926, 17, 14, 0), (8, 12, 128736, 736, 70, 14, 3),
+    (8, 16, 102365, 1131, 26, 20, 0), (8, 16, 101920, 1155, 33, 20, 3), (8, 24, 130244, 1437, 26, 0, 0),
+    (8, 24, 24288, 7895, 40, 32, 3), (8, 32, 2702, 95556, 40, 32, 0), (8, 32, 2112, 120188, 70, 32, 3),
+    (8, 40, 5129, 62634, 70, 32, 0), (8, 40, 111968, 2886, 60, 32, 3), (8, 48, 73401, 5921, 70, 31, 0),
+    (8, 48, 104832, 4081, 70, 32, 3), (8, 64, 106895, 5861, 33, 31, 0), (8, 64, 31264, 20549, 70, 32, 3),
+    (8, 80, 107925, 4718, 70, 31, 0), (8, 80, 116064, 4361, 40, 32, 3), (16, 4, 266, 65, 40, 20, 0),
+    (16, 4, 256, 69, 26, 20, 3), (16, 6, 291, 65, 40, 32, 0), (16, 6, 288, 69, 70, 32, 3),
+    (16, 8, 128725, 106, 100, 31, 0), (16, 8, 288, 48037, 70, 32, 3), (16, 12, 265, 105288, 70, 32, 0),
+    (16, 12, 256, 106607, 60, 32, 3), (16, 16, 488, 124861, 100, 32, 0), (16, 16, 576, 105965, 70, 31, 3),
+    (16, 20, 103369, 787, 33, 31, 0), (16, 20, 127648, 616, 100, 31, 3), (16, 24, 113058, 1064, 40, 32, 0),
+    (16, 24, 85280, 1435, 100, 32, 3), (16, 32, 96226, 1950, 100, 31, 0), (16, 32, 1440, 130708, 40, 32, 3)
+]
+
+
+def life_plan(lib, g, steps, per_launch, wrap):
+    import ctypes as C
+    t = lgdhip.tile(steps_per_launch=per_launch) if per_launch else None
+    out = [C.c_int(-1) for _ in range(3)]
+    assert lib.lgdhip_life2d_plan(C.byref(g), steps, wrap, C.byref(t) if t else None, *(C.byref(v) for v in out)) == 0
+    return tuple(v.value for v in out)
+
+
+@pytest.mark.parametrize("waves,rows,nx,ny,steps,per_launch,wrap", LIFE_PLAN_BOARDS)
+def test_life_packed_every_default_shape(hip, waves, rows, nx, ny, steps, per_launch, wrap):
+    """Every work-group shape that the default variant chooses from, on a board
+    where it does, plain and on a torus: the packed words after the run equal
+    those of the independent-waves kernel (variant 1, which the oracle tests
+    cover), both edge states."""
+    import ctypes as C
+    g = hip.make_grid(2, nx, ny, 1, halo=1, elem_bytes=1)
+    assert life_plan(hip.load(), g, steps, per_launch, wrap)[:2] == (waves, rows)
+    nw = (nx + 31) // 32
+    rng = np.random.default_rng(nx + ny)
+    state = rng.integers(0, 2 ** 32, nw * ny, dtype=np.uint32)
+    pa, pb = hip.DeviceBuffer(state.nbytes), hip.DeviceBuffer(state.nbytes)
+    say("life shape", waves, rows, nx, ny, "steps", steps, per_launch, "wrap", wrap)
+    for edge in (0, 1):
+        got = []
+        for tile in (hip.tile(steps_per_launch=per_launch), hip.tile(variant=1, steps_per_launch=31)):
+            pa.upload(state)
+            in_b = C.c_int(-1)
+            hip.call("lgdhip_life2d_packed_run_periodic", pa.ptr, pb.ptr, C.byref(g), edge, steps, wrap, C.byref(tile),
+                     C.byref(in_b), None)
+            out = np.empty_like(state)
+            (pb if in_b.value else pa).download(out)
+            if nx % 32:
+                out[nw - 1::nw] &= np.uint32((1 << nx % 32) - 1)
+            got.append(out)
+        assert np.array_equal(*got), edge
 
 
 def test_life_glider_on_gpu(hip):
