@@ -438,9 +438,13 @@ LifeShape life_plan(int nw, int ny, int wrap, int steps, int per_launch) {
     // launch on 256 x 200 .. 16384^2 grids; the model's choice is within 3% of
     // the best on each).  A launch's fixed cost and its one pass over the state:
     const double launch_us = 2.0 + 8.0 * nw * ny / 5.5e6;
+    // no deeper than the run: a launch of fewer generations would carry halo rows
+    // for nothing, and a run of one generation would spend 3.3 us of host time here
+    const int deepest = std::min(32, std::max(1, steps));
     for (const auto &shape : kLifeShapes) {
         const int rows = shape.waves * shape.rows;
-        for (int gens = per_launch > 0 ? per_launch : 4; gens <= 32 && 2 * gens < rows; ++gens) {
+        for (int gens = per_launch > 0 ? per_launch : std::min(4, deepest);
+             gens <= (per_launch > 0 ? per_launch : deepest) && 2 * gens < rows; ++gens) {
             const int64_t groups = life_groups(nw, ny, wrap, rows, gens);
             if (groups <= INT32_MAX / kOutCols - 2) {
                 // A generation costs its exchange and barrier (0.25 us) and
@@ -455,7 +459,6 @@ LifeShape life_plan(int nw, int ny, int wrap, int steps, int per_launch) {
                     best = LifeShape{shape.waves, shape.rows, gens};
                 }
             }
-            if (per_launch > 0) break;
         }
     }
     return best;

@@ -204,6 +204,9 @@ def test_life_plan_without_gpu():
     assert plan(1000, 777, 100)[:2] == (8, 4)
     assert plan(16384, 16384, 1000, steps_per_launch=31)[2] == 31
     assert plan(300, 200, 40, variant=7) == (8, 32, 31)
+    # no deeper than the run, unless the caller asks for it
+    assert all(plan(nx, ny, k)[2] <= max(1, k) for nx, ny in ((1000, 777), (16384, 16384)) for k in range(40))
+    assert plan(300, 200, 3, steps_per_launch=9)[2] == 9
     assert plan(300, 200, 40, variant=1, steps_per_launch=9) == (1, 128, 9)
     assert plan(300, 200, 40, steps_per_launch=33) == -2 and plan(300, 200, 40, variant=9) == -2
     assert plan(300, 200, 40, wrap=1) == -2 and plan(300, 200, 40, wrap=4) == -1 and plan(300, 200, -1) == -1

@@ -293,6 +293,9 @@ def test_life_packed_periodic_bit_exact(hip, oracle, shape):
 
 @pytest.mark.parametrize("nx,ny,steps,per_launch,wrap", [
     (1000, 777, 100, 0, 0),     # 8 waves x 4 rows, a span of 33 columns
+    (97, 61, 1, 0, 0),          # runs shorter than the default's shallowest launch
+    (4096, 300, 2, 0, 3),
+    (333, 1000, 3, 0, 2),
     (1984, 40, 33, 0, 3),       # 62 words a row: a span of 64 columns, one band
     (1999, 2051, 60, 0, 2),     # ragged last word, bands cut at every column
     (4096, 4100, 45, 0, 0),     # 16 x 4 rows
