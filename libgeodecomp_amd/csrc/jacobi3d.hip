@@ -517,8 +517,9 @@ __global__ __launch_bounds__(64 * TY) void jacobi3d_f64_tb2(const double *__rest
 // default blocks 4 sweeps per
 // launch with variant 6 or 10, whichever the launch cost model rates cheaper
 // for the grid (10 from 96^3, 6 at 64^3, the faster ones there on MI355X);
-// step counts not divisible by K finish with single sweeps of
-// kSingleSweepVariant.
+// step counts not divisible by K finish with one blocked launch of the remaining
+// sweeps (remainder_plan; a remainder of one may be a single sweep), those of a
+// requested variant with single sweeps of kSingleSweepVariant.
 constexpr int kJacobiDefaultVariant = 6;
 constexpr int kSingleSweepVariant = 13;
 constexpr int kPairVariant = 13;
@@ -541,7 +542,13 @@ TbShape tb_shape(int variant) {
     }
 }
 constexpr int kJacobiVariants = 13;
-constexpr int64_t kSingleRestCells = int64_t(1) << 24;
+// Periodic runs end a remainder of one with a single sweep after a halo refresh
+// from this many cells on, with one blocked launch of one sweep below.  MI355X, all
+// axes wrapped, us blocked / single: 128^3 9.9 / 10.7, 160^3 12.7 / 21.3, 256^3
+// 48.8 / 62.4, 320^3 108 / 137, 384^3 220 / 207, 448^3 365 / 372, 512^3 535 / 487:
+// the memory traffic of the blocked tiles' overlap outweighs the refresh once the
+// grid has left the last-level cache.
+constexpr int64_t kSingleRestCells = int64_t(1) << 25;
 constexpr int kJacobiTallVariant = 10;  // the default's choice for grids that fill several rounds
 
 struct JacobiLaunch {
@@ -691,13 +698,13 @@ int launch_tb(const double *src, double *dst, const lgdhip_grid &g, const Jacobi
 }
 
 // The blocked launch of the default's last r = steps mod 4 sweeps (one row
-// per thread, the z chunk by tb_cost), or no launch (k 0) where single sweeps
-// are the faster ones.  Two or three single sweeps move two or three times the
-// memory of one launch; one single sweep is as fast as a blocked one, but on a
-// periodic grid it needs a halo refresh first.
-JacobiLaunch remainder_plan(const lgdhip_grid &g, int r, bool periodic) {
+// per thread, the z chunk by tb_cost).  Two or three single sweeps move two or
+// three times the memory of one launch.  For r = 1 the callers decide: a single
+// sweep of a Cube grid is as fast, on a periodic one it needs a halo refresh first
+// (kSingleRestCells).
+JacobiLaunch remainder_plan(const lgdhip_grid &g, int r) {
     lgdhip_tile t{};
-    t.variant = r == 3 ? 5 : (r == 2 ? 4 : (periodic ? 11 : kSingleSweepVariant));
+    t.variant = r == 3 ? 5 : (r == 2 ? 4 : 11);
     return plan(g, &t);
 }
 
@@ -793,7 +800,7 @@ extern "C" int lgdhip_jacobi3d_f64_run(double *a, double *b, const lgdhip_grid *
             nxt = tmp;
         }
         if (steps - t > 1 && (!tile || tile->variant == 0)) {
-            rc = launch_tb(cur, nxt, *g, remainder_plan(*g, steps - t, false), s);
+            rc = launch_tb(cur, nxt, *g, remainder_plan(*g, steps - t), s);
             if (rc) return rc;
             std::swap(cur, nxt);
             t = steps;
@@ -852,9 +859,8 @@ extern "C" int lgdhip_jacobi3d_f64_run_periodic(double *a, double *b, const lgdh
     double *cur = a, *nxt = b;
     int t = 0;
     // The default runs its remainder blocked too, but for one last sweep where a
-    // single one after a halo refresh is as fast: on large grids (512^3 all
-    // periodic: 480 us against 535; 128^3: 14 against 12), and as the only sweep
-    // of a call that refreshes halos anyway.
+    // single one after a halo refresh is as fast: on large grids, and as the only
+    // sweep of a call that refreshes halos anyway.
     const bool one_single = steps % 4 == 1 && (g->nx * g->ny * g->nz >= kSingleRestCells ||
                                                (steps == 1 && wrap_mask != 7));
     const bool blocked_rest = k > 0 && (!tile || tile->variant == 0) && !one_single;
@@ -872,7 +878,7 @@ extern "C" int lgdhip_jacobi3d_f64_run_periodic(double *a, double *b, const lgdh
             nxt = tmp;
         }
         if (t < steps && blocked_rest) {
-            rc = launch_tb(cur, nxt, *g, remainder_plan(*g, steps - t, true), s, wrap_mask, edge_at);
+            rc = launch_tb(cur, nxt, *g, remainder_plan(*g, steps - t), s, wrap_mask, edge_at);
             if (rc) return rc;
             std::swap(cur, nxt);
             t = steps;

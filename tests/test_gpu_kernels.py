@@ -141,10 +141,10 @@ def test_jacobi_periodic_bit_exact(hip, oracle, shape, steps):
 
 
 @pytest.mark.parametrize("shape,steps", [((70, 45, 40), (1, 2, 3, 6, 7)), ((129, 33, 9), (2, 7)), ((5, 3, 8), (3, 5)),
-                                         ((257, 256, 256), (1, 5))])
+                                         ((257, 256, 256), (1, 5)), ((330, 320, 320), (5,))])
 def test_jacobi_default_remainders_bit_exact(hip, oracle, shape, steps):
     """The default's last launch of 1, 2 or 3 sweeps on Cube and periodic grids
-    (the fourth shape is large enough to end with a single sweep after a halo
+    (the last shape is large enough to end with a single sweep after a halo
     refresh instead)."""
     nx, ny, nz = shape
     a = synthetic.jacobi_initial(nx, ny, nz, seed=nx + ny)
