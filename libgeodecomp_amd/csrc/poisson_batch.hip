@@ -782,7 +782,7 @@ constexpr int kSmallSweepVariant = 3;
 constexpr int64_t kTallMinTiles = 2048;
 constexpr int kSweepVariants = 6;
 constexpr int kSlabVariant = 7;  // named by the plan only
-TbShape tb_shape(int variant) {
+constexpr TbShape tb_shape(int variant) {
     switch (variant) {
     case 2: return {2, 16, 1};
     case 3: return {4, 16, 1};
@@ -835,6 +835,15 @@ int tb_zchunk(const lgdhip_poisson_problem *probs, const std::vector<int> &set, 
 // Slab shapes, all of 4 sweeps: output planes, lanes and rows per thread.
 constexpr TbShape kSlabShapes[] = {{4, 16, 1, 8, 32}, {4, 16, 1, 2, 32}, {4, 16, 3, 4, 64},
                                    {4, 16, 3, 2, 64}, {4, 16, 4, 4, 64}, {4, 16, 4, 2, 64}};
+
+// every shape the default chooses from advances the same number of sweeps per
+// launch, so a solve's chunks hold for whichever its active set gets
+constexpr bool default_shapes_alike() {
+    for (const TbShape &sh : kSlabShapes)
+        if (sh.k != tb_shape(kDefaultSweepVariant).k) return false;
+    return tb_shape(kSmallSweepVariant).k == tb_shape(kDefaultSweepVariant).k;
+}
+static_assert(default_shapes_alike());
 
 // The blocked sweep shape of a launch over the problems in `set`: the
 // requested variant, or for 0 the default by launch size: a slab shape where it
@@ -1345,7 +1354,8 @@ int lgdhip_poisson_batch_solve(double *u, const float *f, const lgdhip_poisson_p
     const bool graphs = opt->use_graph != 0 && s != nullptr;
     const double theta = opt->inner_reduction > 0 ? opt->inner_reduction : 1e-2;
     // the blocked shape is chosen per active set (sweep_shape); the default's
-    // two candidates both run K = 4, so the chunk length below holds for any
+    // candidates all run the same K (default_shapes_alike), so the chunk length
+    // below holds for any
     TbShape sh = sweep_shape(opt->sweep_variant, probs, std::vector<int>());
     // sweeps per chunk: even (plain) or a multiple of 2K (blocked), so every
     // chunk leaves the correction in the same buffer
