@@ -440,7 +440,8 @@ def poisson_sweep_kernel(stream, e0, e1, f, probs, count, ws, ws_bytes, cells, s
     """The roofline of the Poisson solver's sweep kernel: temporal blocking,
     4 sweeps per launch (12 B per sweep-LUP, so 4 x 12 B x cells per launch);
     variant 0 is the library default (6, three rows per thread, on large
-    launches, else 3, one row).  Returns (roofline, planned variant)."""
+    launches; 7, whole planes on chip, for sets of small problems; else 3, one
+    row).  Returns (roofline, planned variant)."""
     k, sweeps = 4, 48
     in_b = C.c_int(0)
     tile = lgdhip.tile(variant=variant)
@@ -448,7 +449,8 @@ def poisson_sweep_kernel(stream, e0, e1, f, probs, count, ws, ws_bytes, cells, s
                                            C.byref(tile), ws.ptr, ws_bytes, C.byref(in_b), stream.h))
     planned = C.c_int(0)  # the library resolves the default by launch size
     lgdhip.call("lgdhip_poisson_sweep_plan", probs, count, variant, C.byref(planned))
-    name = "poisson_sweep_tb2" if planned.value in (4, 5, 6) else "poisson_sweep_tb"
+    name = {4: "poisson_sweep_tb2", 5: "poisson_sweep_tb2", 6: "poisson_sweep_tb2",
+            7: "poisson_sweep_slab"}.get(planned.value, "poisson_sweep_tb")
     return roofline(name, shape, ms / (sweeps // k), k * 12.0 * cells, k), planned.value
 
 

@@ -639,7 +639,7 @@ int lgdhip_life2d_pack(const uint8_t *grid, const lgdhip_grid *g, uint32_t *pack
     if (rc) return rc;
     LGD_REQUIRE(grid && packed, "NULL pointer");
     const int nw = (int)((g->nx + 31) / 32);
-    LGD_REQUIRE(g->ny <= 65535, "ny must be <= 65535 (one grid row per launch row)");
+    LGD_REQUIRE(g->ny <= 65535, "ny must be <= 65535");
     const dim3 block = pack_block(nw), grd(lgdhip::ceil_div(nw, block.x), lgdhip::ceil_div(g->ny, block.y));
     life_pack<<<grd, block, 0, lgdhip::as_stream(stream)>>>(grid, packed, (int)g->nx, (int)g->ny, nw, g->sx,
                                                          lgdhip::origin_index(*g));
@@ -651,7 +651,7 @@ int lgdhip_life2d_unpack(const uint32_t *packed, const lgdhip_grid *g, uint8_t *
     int rc = check_life_grid(g);
     if (rc) return rc;
     LGD_REQUIRE(grid && packed, "NULL pointer");
-    LGD_REQUIRE(g->ny <= 65535, "ny must be <= 65535 (one grid row per launch row)");
+    LGD_REQUIRE(g->ny <= 65535, "ny must be <= 65535");
     const int nw = (int)((g->nx + 31) / 32);
     const dim3 block = pack_block(nw), grd(lgdhip::ceil_div(nw, block.x), lgdhip::ceil_div(g->ny, block.y));
     life_unpack<<<grd, block, 0, lgdhip::as_stream(stream)>>>(packed, grid, (int)g->nx, (int)g->ny, nw, g->sx,

@@ -43,8 +43,8 @@ def test_jacobi_128_cube_100_steps_bit_exact(hip, oracle, variant):
 
 
 def test_jacobi_512_cube_bit_exact(hip, oracle):
-    """The HBM-bound shape, 10 steps (two 4-sweep launches and two single
-    sweeps of the default plan)."""
+    """The HBM-bound shape, 10 steps (two 4-sweep launches and one 2-sweep
+    launch of the default plan)."""
     a = synthetic.jacobi_initial(512, 512, 512, seed=5)
     say("jacobi 512^3 x 10")
     exp = oracle.jacobi3d(a, 10, edge=0.0, threads=8)
@@ -76,8 +76,8 @@ def life_input():
 @pytest.mark.parametrize("tile", [dict(steps_per_launch=31, variant=7), None, dict(steps_per_launch=16, variant=3)])
 @pytest.mark.parametrize("generations", [31, 1000])
 def test_life_16384_square_against_fixture(hip, life_input, tile, generations):
-    """The headline run (the bench's tile: 31 generations per launch,
-    stacked-wave kernel; the library default; a one-row-per-thread
+    """The headline run (8 stacked waves x 32 rows at 31 generations per
+    launch; the library default, which the bench runs; an independent-waves
     variant) ends in exactly the oracle's state: SHA-256 of all 268 M cells
     and their popcount."""
     fx = life_fixture()["checkpoints"][str(generations)]
