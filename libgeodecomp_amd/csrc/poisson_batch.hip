@@ -821,15 +821,18 @@ void append_tb_tiles(std::vector<Tile> *out, int p, int n, TbShape sh, int zchun
 // one rounding tile per (problem, xy tile), itself under kTbMinGroups).
 constexpr int64_t kTbMinGroups = 512;  // two one-row work-groups per CU
 constexpr int64_t kTbSmallListTiles = 3 * kTbMinGroups;
-int tb_zchunk(const lgdhip_poisson_problem *probs, const std::vector<int> &set, TbShape sh) {
-    auto tiles = [&](int zc) {
-        int64_t t = 0;
-        for (int k : set) t += tb_tiles_of(probs[k].n, sh, zc);
-        return t;
-    };
+template <typename Tiles>  // tiles(zc): the launch's tiles in chunks of zc planes
+int tb_zchunk_of(TbShape sh, Tiles tiles) {
     int zc = sh.slab ? sh.slab : kTbZ;
     while (!sh.slab && zc > 4 && tiles(zc) < kTbMinGroups) zc /= 2;
     return zc;
+}
+int tb_zchunk(const lgdhip_poisson_problem *probs, const std::vector<int> &set, TbShape sh) {
+    return tb_zchunk_of(sh, [&](int zc) {
+        int64_t t = 0;
+        for (int k : set) t += tb_tiles_of(probs[k].n, sh, zc);
+        return t;
+    });
 }
 
 // Slab shapes, all of 4 sweeps: output planes, lanes and rows per thread.
@@ -853,6 +856,13 @@ static_assert(default_shapes_alike());
 // 14.3 / 20.0, 16 x 63^3 21.6 / 32.8, but 1 x 40^3 11.9 / 9.4, 1 x 63^3
 // 13.6 / 9.5.  8 sweeps per launch in 18 planes took 16.0 us at 16 x 31^3, no
 // less per sweep.
+//
+// Slabs of 64-lane rows in more than one round of the CUs win or lose by a third
+// (32 x 40^3 21.8 / 23.7, 16 x 60^3 18.1 / 30.3, but 40 x 52^3 41.2 / 34.2, 105 x
+// 53^3 86 / 64, 128 x 32^3 38 / 31), which the estimates above cannot tell; there
+// both kernels' times come from a fit to 131 measured sets (slabs within 4 % rms,
+// one row 6 %; 4 of those sets then run 2 to 8 % slower than with one row, 15 run
+// 2 to 10 % slower than with slabs).
 TbShape sweep_shape(int requested, const lgdhip_poisson_problem *probs, const std::vector<int> &set) {
     if (requested >= 1 && requested <= kSweepVariants) return tb_shape(requested);
     const TbShape tall = tb_shape(kDefaultSweepVariant), flat = tb_shape(kSmallSweepVariant);
@@ -864,18 +874,26 @@ TbShape sweep_shape(int requested, const lgdhip_poisson_problem *probs, const st
     }
     if (tiles >= kTallMinTiles) return tall;
     if (set.empty() || nmax >= 64) return flat;
+    // problems of each size, so that a large set costs the host no more
+    int64_t count[64] = {};
+    for (int k : set) ++count[probs[k].n];
+    auto sum = [&](auto of) {
+        int64_t t = 0;
+        for (int n = 1; n <= nmax; ++n)
+            if (count[n]) t += count[n] * of(n);
+        return t;
+    };
+    auto tiles_in = [&](TbShape sh, int zc) { return sum([&](int n) { return tb_tiles_of(n, sh, zc); }); };
     // the one-row kernel: 0.65 us a plane step, 0.9 us with two work-groups on
     // a CU, which holds no more
-    const int zc = tb_zchunk(probs, set, flat);
-    int64_t groups = 0;
-    for (int k : set) groups += tb_tiles_of(probs[k].n, flat, zc);
+    const int zc = tb_zchunk_of(flat, [&](int c) { return tiles_in(flat, c); });
+    const int64_t groups = tiles_in(flat, zc);
     TbShape best = flat;
     double best_us = 1.5 + (double)((groups + 2 * lgdhip::kCUs - 1) / (2 * lgdhip::kCUs)) * (zc + 2 * flat.k) *
                                (groups > (int64_t)lgdhip::kCUs ? 0.9 : 0.65);
     for (const TbShape &sh : kSlabShapes) {
         if (nmax >= std::min(sh.lanes, 16 * sh.rows * 64 / sh.lanes)) continue;
-        int64_t slabs = 0;
-        for (int k : set) slabs += tb_tiles_of(probs[k].n, sh);
+        const int64_t slabs = tiles_in(sh, 0);
         if (slabs > kTbSmallListTiles && sh.slab < 8) continue;  // the tile lists' capacity
         // a slab kernel: one work-group per CU; loads, levels' barriers and
         // the planes of all levels at 0.09 us per 1024 cells
@@ -886,6 +904,28 @@ TbShape sweep_shape(int requested, const lgdhip_poisson_problem *probs, const st
             best_us = us;
             best = sh;
         }
+    }
+    const int64_t slabs = best.slab ? tiles_in(best, 0) : 0;
+    if (best.lanes == 64 && slabs > lgdhip::kCUs) {
+        // slabs: rounds of levels (all waves' barriers, the live ones' sums), the
+        // planes read and written, less what the last round leaves free
+        const double rounds = (double)((slabs + lgdhip::kCUs - 1) / lgdhip::kCUs);
+        const double work = (best.k * best.slab + best.k * (best.k - 1)) * best.rows;
+        const double live = sum([&](int n) {
+            return tb_tiles_of(n, best) * std::min(16, (n + best.rows - 1) / best.rows);
+        }) / (16.0 * (double)slabs);
+        const double mb = 4e-6 * (3 * best.slab + 4 * best.k - 2) *
+                          (double)sum([&](int n) { return tb_tiles_of(n, best) * n * n; });
+        const double slab_us = 3.4 + rounds * (1.86 + work * (0.056 + 0.0159 * live)) + 0.0716 * mb -
+                               0.83 * (double)slabs / lgdhip::kCUs;
+        // one row: the longest march, and the mean one for the work-groups beyond
+        // the first round
+        const double steps = (double)sum([&](int n) {
+            return tb_tiles_of(n, flat, n) * (n + 2 * flat.k * (int64_t)((n + zc - 1) / zc));
+        });
+        const double flat_us = 4.6 + 0.75 * (std::min(zc, nmax) + 2 * flat.k) +
+                               0.54 * std::max(0.0, (double)groups / (2 * lgdhip::kCUs) - 0.93) * steps / groups;
+        if (slab_us > 0.98 * flat_us) best = flat;
     }
     return best;
 }
@@ -1089,10 +1129,13 @@ int run_sweeps_in(float *ea, float *eb, const float *r, const lgdhip_poisson_pro
     std::vector<Tile> tiles;
     rc = upload_set(w, probs, all, &tiles, s);
     if (rc) return rc;
-    const TbShape sh = sweep_shape(tile ? tile->variant : 0, probs, all);
+    const int requested = tile ? tile->variant : 0;
+    // sweeps per launch of any shape that the request may resolve to
+    const int k = tb_shape(requested >= 1 && requested <= kSweepVariants ? requested : kDefaultSweepVariant).k;
     float *cur = ea, *nxt = eb;
     int t = 0;
-    if (sh.k > 0 && sweeps >= sh.k) {
+    if (k > 0 && sweeps >= k) {
+        const TbShape sh = sweep_shape(requested, probs, all);
         int64_t ntb = 0;
         int zc = kTbZ;
         rc = upload_tb_set(w, probs, all, sh, &ntb, &zc, s);

@@ -186,6 +186,12 @@ def test_poisson_sweep_plan_without_gpu():
     assert plan(ensemble) == 6
     assert plan([128] * 16) == 3
     assert plan([128] * 16, 5) == 5 and plan(ensemble, 3) == 3
+    # whole planes on chip (7) for small sets and short rows, one row where more
+    # than a round of 64-lane planes was measured slower
+    for sizes in ([31], [31] * 16, [8] * 300, [60] * 16, [36] * 48, [40] * 48, [16] * 500):
+        assert plan(sizes) == 7, sizes
+    for sizes in ([52] * 40, [56] * 64, [53] * 105, [47] * 128, [32] * 128, [56] * 20):
+        assert plan(sizes) == 3, sizes
 
 
 def test_life_plan_without_gpu():
