@@ -60,6 +60,12 @@ struct SolveState {
     int32_t outer_iters, done, refresh, pad;
 };
 
+// What a sweep launch is: plain, damped, or plain in a solve, where it skips the
+// problems that are done.  A kind of its own, because the look at the states
+// splits the scalar loads at a kernel's start into a longer chain (2 x 50^3 6.6 ->
+// 6.9 us where every launch tested for states).
+enum SweepKind { kPlainSweep, kDampedSweep, kSolveSweep };
+
 __device__ __forceinline__ double block_sum(double v, double *lds) {
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
@@ -112,10 +118,10 @@ __global__ __launch_bounds__(kThreads) void poisson_residual_f64(const double *_
 // + e[y+1] + e[z+1] + r) * (1/6), summed in that order; when `partial` is
 // given, also the per-tile sum of the FP64 square of the residual of the
 // input iterate, r + sum_nb e - 6 e (= 6 (e' - e) up to rounding).
-// DAMPED: weighted Jacobi e' = e + omega (J(e) - e), which damps the
+// kDampedSweep: weighted Jacobi e' = e + omega (J(e) - e), which damps the
 // highest-frequency error modes by |1 - 2 omega| per sweep instead of
 // plain Jacobi's cos(pi/(n+1)) (used to smooth a predicted initial guess).
-template <bool DAMPED>
+template <SweepKind KIND>
 __global__ __launch_bounds__(kThreads) void poisson_sweep_f32(const float *__restrict__ e, float *__restrict__ e2,
                                                               const float *__restrict__ r,
                                                               const Tile *__restrict__ tiles,
@@ -124,7 +130,8 @@ __global__ __launch_bounds__(kThreads) void poisson_sweep_f32(const float *__res
                                                               const SolveState *__restrict__ state) {
     __shared__ double lds[kThreads / 64];
     const Tile t = tiles[blockIdx.x];
-    if (state && state[t.p].done) return;
+    if (KIND == kSolveSweep && state[t.p].done) return;
+    constexpr bool DAMPED = KIND == kDampedSweep;
     const ProblemDev P = probs[t.p];
     const int n = P.n;
     const int x = t.x0 + (int)(threadIdx.x % kTX);
@@ -185,7 +192,7 @@ __device__ __forceinline__ float lane_next(float v) {
 // launch equals K launches of that kernel bit for bit.  With `partial`, the
 // last level adds the FP64 square of the residual of its input iterate over
 // the written cells into one partial per tile.
-template <int K, int TY, bool DAMPED>
+template <int K, int TY, SweepKind KIND>
 __global__ __launch_bounds__(64 * TY) void poisson_sweep_tb(const float *__restrict__ e, float *__restrict__ e2,
                                                             const float *__restrict__ r,
                                                             const Tile *__restrict__ tiles,
@@ -202,7 +209,8 @@ __global__ __launch_bounds__(64 * TY) void poisson_sweep_tb(const float *__restr
     const unsigned tid = lgdhip::xcd_tile(blockIdx.x, per, true);
     if (tid >= ntiles) return;  // whole work-group, before any barrier
     const Tile t = tiles[tid];
-    if (state && state[t.p].done) return;
+    if (KIND == kSolveSweep && state[t.p].done) return;
+    constexpr bool DAMPED = KIND == kDampedSweep;
     const ProblemDev P = probs[t.p];
     const int n = P.n;
     const int tx = threadIdx.x, ty = threadIdx.y;
@@ -324,8 +332,8 @@ __global__ __launch_bounds__(64 * TY) void poisson_sweep_tb(const float *__restr
 // and last row for the neighbouring threads, and the taller tile recomputes
 // a smaller overlap ring.  Cells, sum order, rings, ramp and residual
 // partials as in poisson_sweep_tb: bit-exact with K launches of
-// poisson_sweep_f32 (DAMPED: of its weighted form).
-template <int K, int TY, int R, bool DAMPED>
+// poisson_sweep_f32 (kDampedSweep: of its weighted form).
+template <int K, int TY, int R, SweepKind KIND>
 __global__ __launch_bounds__(64 * TY) void poisson_sweep_tb2(const float *__restrict__ e, float *__restrict__ e2,
                                                              const float *__restrict__ r,
                                                              const Tile *__restrict__ tiles,
@@ -342,7 +350,8 @@ __global__ __launch_bounds__(64 * TY) void poisson_sweep_tb2(const float *__rest
     const unsigned tid = lgdhip::xcd_tile(blockIdx.x, per, true);
     if (tid >= ntiles) return;  // whole work-group, before any barrier
     const Tile t = tiles[tid];
-    if (state && state[t.p].done) return;
+    if (KIND == kSolveSweep && state[t.p].done) return;
+    constexpr bool DAMPED = KIND == kDampedSweep;
     const ProblemDev P = probs[t.p];
     const int n = P.n;
     const int tx = threadIdx.x, ty = threadIdx.y;
@@ -495,7 +504,7 @@ __global__ __launch_bounds__(64 * TY) void poisson_sweep_tb2(const float *__rest
 // dependent plane steps per launch, each with its barrier and level chain,
 // this one K levels with one barrier each (one more where the planes do not
 // fit LDS twice), every level's planes independent of each other.
-template <int LX, int RY, int NP, int K, bool DAMPED>
+template <int LX, int RY, int NP, int K, SweepKind KIND>
 __global__ __launch_bounds__(1024) void poisson_sweep_slab(const float *__restrict__ e, float *__restrict__ e2,
                                                            const float *__restrict__ r,
                                                            const Tile *__restrict__ tiles,
@@ -511,7 +520,8 @@ __global__ __launch_bounds__(1024) void poisson_sweep_slab(const float *__restri
     const unsigned tid = lgdhip::xcd_tile(blockIdx.x, per, true);
     if (tid >= ntiles) return;  // whole work-group, before any barrier
     const Tile t = tiles[tid];
-    if (state && state[t.p].done) return;
+    if (KIND == kSolveSweep && state[t.p].done) return;
+    constexpr bool DAMPED = KIND == kDampedSweep;
     const ProblemDev P = probs[t.p];
     const int n = P.n;
     const int lane = threadIdx.x & 63;
@@ -1033,13 +1043,13 @@ int upload_tb_set(const Workspace &w, const lgdhip_poisson_problem *probs, const
     return 0;
 }
 
-template <bool DAMPED>
+template <SweepKind KIND>
 void launch_tb_kind(TbShape sh, const float *a, float *b, const float *r, const Workspace &w, int64_t ntiles,
                     int zchunk, double *partial, float omega, const SolveState *state, hipStream_t s) {
     const unsigned nt = (unsigned)ntiles, per = lgdhip::xcd_per(nt), groups = lgdhip::xcd_groups(nt);
 #define LGD_SLAB_CASE(K, ZS, LX, RY)                                                                           \
-    if (sh.k == K && sh.slab == ZS && sh.lanes == LX && sh.rows == RY) {                                                   \
-        poisson_sweep_slab<LX, RY, ZS + 2 * K, K, DAMPED><<<groups, 1024, 0, s>>>(a, b, r, w.tb_tiles, w.probs, \
+    if (sh.k == K && sh.slab == ZS && sh.lanes == LX && sh.rows == RY) {                                \
+        poisson_sweep_slab<LX, RY, ZS + 2 * K, K, KIND><<<groups, 1024, 0, s>>>(a, b, r, w.tb_tiles, w.probs, \
                                                                                   partial, nt, per, omega,     \
                                                                                   state);                      \
         return;                                                                                                \
@@ -1048,19 +1058,19 @@ void launch_tb_kind(TbShape sh, const float *a, float *b, const float *r, const 
     LGD_SLAB_CASE(4, 2, 64, 4) LGD_SLAB_CASE(4, 4, 64, 3) LGD_SLAB_CASE(4, 2, 64, 3)
 #undef LGD_SLAB_CASE
     if (sh.rows == 3)
-        poisson_sweep_tb2<4, 16, 3, DAMPED><<<groups, dim3(64, 16), 0, s>>>(a, b, r, w.tb_tiles, w.probs, partial,
+        poisson_sweep_tb2<4, 16, 3, KIND><<<groups, dim3(64, 16), 0, s>>>(a, b, r, w.tb_tiles, w.probs, partial,
                                                                             zchunk, nt, per, omega, state);
     else if (sh.rows == 2 && sh.ty == 16)
-        poisson_sweep_tb2<4, 16, 2, DAMPED><<<groups, dim3(64, 16), 0, s>>>(a, b, r, w.tb_tiles, w.probs, partial,
+        poisson_sweep_tb2<4, 16, 2, KIND><<<groups, dim3(64, 16), 0, s>>>(a, b, r, w.tb_tiles, w.probs, partial,
                                                                             zchunk, nt, per, omega, state);
     else if (sh.rows == 2)
-        poisson_sweep_tb2<4, 8, 2, DAMPED><<<groups, dim3(64, 8), 0, s>>>(a, b, r, w.tb_tiles, w.probs, partial, zchunk,
+        poisson_sweep_tb2<4, 8, 2, KIND><<<groups, dim3(64, 8), 0, s>>>(a, b, r, w.tb_tiles, w.probs, partial, zchunk,
                                                                           nt, per, omega, state);
     else if (sh.k == 2)
-        poisson_sweep_tb<2, 16, DAMPED><<<groups, dim3(64, 16), 0, s>>>(a, b, r, w.tb_tiles, w.probs, partial, zchunk, nt,
+        poisson_sweep_tb<2, 16, KIND><<<groups, dim3(64, 16), 0, s>>>(a, b, r, w.tb_tiles, w.probs, partial, zchunk, nt,
                                                                         per, omega, state);
     else
-        poisson_sweep_tb<4, 16, DAMPED><<<groups, dim3(64, 16), 0, s>>>(a, b, r, w.tb_tiles, w.probs, partial, zchunk, nt,
+        poisson_sweep_tb<4, 16, KIND><<<groups, dim3(64, 16), 0, s>>>(a, b, r, w.tb_tiles, w.probs, partial, zchunk, nt,
                                                                         per, omega, state);
 }
 
@@ -1071,9 +1081,11 @@ void launch_tb(TbShape sh, const float *a, float *b, const float *r, const Works
                int zchunk, double *partial, hipStream_t s, float omega = 0.0f, const SolveState *state = nullptr) {
     if (ntiles <= 0) return;
     if (omega > 0.0f)
-        launch_tb_kind<true>(sh, a, b, r, w, ntiles, zchunk, partial, omega, state, s);
+        launch_tb_kind<kDampedSweep>(sh, a, b, r, w, ntiles, zchunk, partial, omega, state, s);
+    else if (state)
+        launch_tb_kind<kSolveSweep>(sh, a, b, r, w, ntiles, zchunk, partial, 0.0f, state, s);
     else
-        launch_tb_kind<false>(sh, a, b, r, w, ntiles, zchunk, partial, 0.0f, state, s);
+        launch_tb_kind<kPlainSweep>(sh, a, b, r, w, ntiles, zchunk, partial, 0.0f, nullptr, s);
 }
 
 // chunks of a solve enqueued between two looks at the problems' states
@@ -1148,10 +1160,10 @@ int run_sweeps_in(float *ea, float *eb, const float *r, const lgdhip_poisson_pro
     }
     for (; t < sweeps; ++t) {
         if (omega > 0.0f)
-            poisson_sweep_f32<true>
+            poisson_sweep_f32<kDampedSweep>
                 <<<(unsigned)tiles.size(), kThreads, 0, s>>>(cur, nxt, r, w.tiles, w.probs, nullptr, omega, nullptr);
         else
-            poisson_sweep_f32<false>
+            poisson_sweep_f32<kPlainSweep>
                 <<<(unsigned)tiles.size(), kThreads, 0, s>>>(cur, nxt, r, w.tiles, w.probs, nullptr, 1.0f, nullptr);
         LGD_LAUNCHED("poisson_sweep_f32");
         std::swap(cur, nxt);
@@ -1465,7 +1477,7 @@ int lgdhip_poisson_batch_solve(double *u, const float *f, const lgdhip_poisson_p
                 }
             }
             for (; t < smooth; ++t) {
-                poisson_sweep_f32<true><<<(unsigned)tiles.size(), kThreads, 0, s>>>(
+                poisson_sweep_f32<kDampedSweep><<<(unsigned)tiles.size(), kThreads, 0, s>>>(
                     ecur, enxt, w.r, w.tiles, w.probs, nullptr, opt->smooth_omega, nullptr);
                 LGD_LAUNCHED("poisson_sweep_f32");
                 std::swap(ecur, enxt);
@@ -1513,7 +1525,7 @@ int lgdhip_poisson_batch_solve(double *u, const float *f, const lgdhip_poisson_p
                 }
             } else {
                 for (int t = 0; t < C; ++t) {
-                    poisson_sweep_f32<false><<<nt, kThreads, 0, s>>>(a, b, w.r, w.tiles, w.probs,
+                    poisson_sweep_f32<kSolveSweep><<<nt, kThreads, 0, s>>>(a, b, w.r, w.tiles, w.probs,
                                                                      t == C - 1 ? w.partial : nullptr, 1.0f, w.state);
                     std::swap(a, b);
                 }
