@@ -1080,13 +1080,12 @@ bool gemm_applies(int n, int cin, int ksize, int cout) {
 // fragments' registers allow), columns and z planes per chunk
 struct ZmPlan {
     int nt, slices, bx, by, bz, zchunk;
+    double steps;  // modelled length of the launch in plane steps
 };
-ZmPlan zm_plan(int n, int groups, int cout) {
+ZmPlan zm_plan_of(int n, int groups, int tiles, int nt) {
     ZmPlan z;
-    const int tiles = cout / 16;
-    z.nt = std::max(1, std::min(3, 4 / groups));
+    z.nt = nt;
     const int resident = zm_waves(groups, z.nt) >= 2 ? 2 : 1;
-    while (tiles % z.nt) --z.nt;
     z.slices = tiles / z.nt;
     z.bx = (n + 15) / 16;
     z.by = (n + 7) / 8;
@@ -1094,7 +1093,7 @@ ZmPlan zm_plan(int n, int groups, int cout) {
     // where two work-groups share a CU, a step of one that has the CU alone
     // takes 0.6 of a step of two (0.8 from 5 input groups on); a chunk reads
     // two planes beyond its own and starts in about one step more.
-    double best = 1e300;
+    z.steps = 1e300;
     for (int chunks = 1; chunks <= n; ++chunks) {
         const int zc = (n + chunks - 1) / chunks;
         if ((n + zc - 1) / zc != chunks) continue;
@@ -1102,11 +1101,26 @@ ZmPlan zm_plan(int n, int groups, int cout) {
         double rounds = resident == 1 ? (double)on_cu : (double)((on_cu + 1) / 2);
         if (resident == 2 && on_cu == 1) rounds = groups <= 4 ? 0.6 : 0.8;
         const double steps = rounds * (zc + 3);
-        if (steps < best) {
-            best = steps;
+        if (steps < z.steps) {
+            z.steps = steps;
             z.zchunk = zc;
             z.bz = chunks;
         }
+    }
+    return z;
+}
+ZmPlan zm_plan(int n, int groups, int cout, bool masked) {
+    const int tiles = cout / 16;
+    int nt = std::max(1, std::min(3, 4 / groups));
+    while (tiles % nt) --nt;
+    const ZmPlan z = zm_plan_of(n, groups, tiles, nt);
+    // a masked row's weights are loaded value by value, 56 nt of them a lane before
+    // the march begins: one tile per slice where the launch gets no longer than that
+    // by it (us with nt tiles / one: 16^3 3 -> 48 11.4 / 6.2, 31^3 3 -> 48 11.8 / 8.2,
+    // 24^3 3 -> 32 8.9 / 7.0; 16^3 and 17^3 3 -> 48 took 9 in conv3d_fwd_mfma)
+    if (masked && nt > 1) {
+        const ZmPlan one = zm_plan_of(n, groups, tiles, 1);
+        if (one.steps <= z.steps + 1.25 * (nt - 1)) return one;
     }
     return z;
 }
@@ -2098,7 +2112,7 @@ int conv3d_forward(const void *x, int n, int ldx, int offx, int cin, int ksize, 
             split = p.slices;
         }
         if (groups >= 1 && (groups <= 6 || (groups <= 8 && (split || cout == 16))) && split <= 2) {
-            const ZmPlan z = zm_plan(n, groups, cout);
+            const ZmPlan z = zm_plan(n, groups, cout, masked);
             const unsigned wgs = (unsigned)((int64_t)z.bx * z.by * z.bz * z.slices), per = lgdhip::xcd_per(wgs);
             // the mask is compiled for square layers of 16, 32 and 64 channels,
             // those with a ReLU on both sides in a network

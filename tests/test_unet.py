@@ -1003,7 +1003,7 @@ def test_conv_wgrad_infinite_activations(hip, n, cin, cout):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("n,cin,cout", [(97, 16, 48), (96, 40, 64), (20, 3, 48)])
+@pytest.mark.parametrize("n,cin,cout", [(97, 16, 48), (96, 40, 64), (20, 3, 48), (48, 3, 48)])
 def test_conv_zm_other_orders(hip, n, cin, cout):
     """Layers whose plain 16-byte-aligned launch sums in another k order than
     the kernel of their accumulating launch: more than 32 output channels on
