@@ -2106,13 +2106,19 @@ int conv3d_forward(const void *x, int n, int ldx, int offx, int cin, int ksize, 
         const bool gemm_order = groups > 1 && (n < kZmGroupOrderN || groups > 6 || !plain) &&
                                 gemm_applies(n, cin, ksize, cout);
         int split = 0;
+        double gemm_us = 1e300;
         if (gemm_order) {
             const GemmPlan p = gemm_plan(n, cin, cout, workspace != nullptr);
             if (workspace && workspace_bytes < gemm_workspace_bytes(n, p)) return small_workspace();
             split = p.slices;
+            gemm_us = 22 + 0.0245 * (double)p.mblocks * p.nblocks;
         }
-        if (groups >= 1 && (groups <= 6 || (groups <= 8 && (split || cout == 16))) && split <= 2) {
-            const ZmPlan z = zm_plan(n, groups, cout, masked);
+        const bool fits = groups >= 1 && (groups <= 6 || (groups <= 8 && (split || cout == 16))) && split <= 2;
+        const ZmPlan z = fits ? zm_plan(n, groups, cout, masked) : ZmPlan{};
+        // 7 groups in tap-major order take 3.15 us a plane step, where 8 take 2.6: the
+        // GEMM-tiled kernel keeps the launches that this makes too long (33^3 56 -> 96
+        // 62 us, there 46; 96^3 56 -> 64 415, there 365; but 63^3 56 -> 32 60, there 116)
+        if (fits && !(groups == 7 && 3.15 * z.steps > gemm_us)) {
             const unsigned wgs = (unsigned)((int64_t)z.bx * z.by * z.bz * z.slices), per = lgdhip::xcd_per(wgs);
             // the mask is compiled for square layers of 16, 32 and 64 channels,
             // those with a ReLU on both sides in a network

@@ -236,7 +236,7 @@ def test_conv_zm_slices(hip, oracle, cout, ld, off):
     (17, 48, 16, 16, 0), (65, 5, 32, 32, 0), (19, 56, 16, 16, 0), (16, 64, 16, 16, 0), (64, 64, 32, 32, 0),
     (42, 16, 32, 32, 0), (43, 24, 48, 52, 4), (41, 32, 32, 32, 0), (42, 40, 32, 32, 0), (41, 48, 64, 64, 0),
     (41, 56, 32, 32, 0), (42, 64, 32, 32, 0), (33, 24, 32, 32, 0), (32, 32, 64, 64, 0), (36, 16, 48, 48, 0),
-    (37, 40, 48, 48, 0), (35, 48, 32, 32, 0), (33, 56, 48, 48, 0), (32, 64, 64, 64, 0)])
+    (37, 40, 48, 48, 0), (35, 48, 32, 32, 0), (33, 56, 48, 48, 0), (33, 56, 96, 96, 0), (32, 64, 64, 64, 0)])
 def test_conv_zm_same_bits(hip, oracle, n, cin, cout, ld, off):
     """The z-marching kernel over its input groups, output tiles per slice and
     the three k orders, on edges that leave part of a column and a chunk of
