@@ -1518,29 +1518,34 @@ __global__ __launch_bounds__(64 * TI * TO * KS, TI * TO * KS == 4 ? 3 : 1) void 
 
 // dW[co][k] = sum over chunks of P (fixed order) for k < K; the padding
 // columns k >= K stay zero
-// A work-group of 64 x 16 threads takes 64 consecutive outputs; thread row j
-// sums the chunks j, j + 16, j + 32, ... (eight loads in flight, coalesced
+// A work-group of 64 x ROWS threads takes 64 consecutive outputs; thread row j
+// sums the chunks j, j + ROWS, j + 2 ROWS, ... (eight loads in flight, coalesced
 // across the 64 outputs) and the row sums are added in row order: a fixed
-// order for every output.  (With 4 rows the 108 work-groups of a 16 -> 16
-// layer's 512 chunks took 20.5 us.)
-constexpr int kWgradReduceOutputs = 64, kWgradReduceRows = 16;
-__global__ __launch_bounds__(kWgradReduceOutputs * kWgradReduceRows) void conv3d_wgrad_reduce(const float *__restrict__ P, int chunks, int cout, int Kp,
-                                                           int K, float *__restrict__ dW, int accumulate) {
-    __shared__ float part[kWgradReduceRows][kWgradReduceOutputs];
+// order for every output.  16 rows where the outputs are fewer than two
+// work-groups per CU (16 -> 16: 112 of them; 128^3 40.1 us with the column kernel,
+// 44.1 with 4 rows), else 4: wide layers have few chunks on small volumes, and
+// rows without one cost their launch (16^3 128 -> 128 21.3 us, 32.0 with 16 rows).
+constexpr int kWgradReduceOutputs = 64;
+template <int ROWS>
+__global__ __launch_bounds__(kWgradReduceOutputs *ROWS) void conv3d_wgrad_reduce(const float *__restrict__ P,
+                                                                                 int chunks, int cout, int Kp, int K,
+                                                                                 float *__restrict__ dW,
+                                                                                 int accumulate) {
+    __shared__ float part[ROWS][kWgradReduceOutputs];
     const int total = cout * Kp;  // < 2^31: cout <= 192, Kp <= 27 * 192 + 31
     const int o = (int)blockIdx.x * kWgradReduceOutputs + (int)threadIdx.x;
     const int j = (int)threadIdx.y;
     float s = 0.0f;
     if (o < total && o % Kp < K) {
 #pragma unroll 8
-        for (int c = j; c < chunks; c += kWgradReduceRows) s += P[(int64_t)c * total + o];
+        for (int c = j; c < chunks; c += ROWS) s += P[(int64_t)c * total + o];
     }
     part[j][threadIdx.x] = s;
     __syncthreads();
     if (j != 0 || o >= total) return;
     float r = part[0][threadIdx.x];
 #pragma unroll
-    for (int k = 1; k < kWgradReduceRows; ++k) r += part[k][threadIdx.x];
+    for (int k = 1; k < ROWS; ++k) r += part[k][threadIdx.x];
     if (o % Kp >= K) {  // padding columns stay zero
         dW[o] = accumulate ? dW[o] : 0.0f;
         return;
@@ -2339,9 +2344,11 @@ int lgdhip_conv3d_bf16_wgrad(const void *x, int n, int ldx, int offx, int cin, i
 #undef LGD_WG_CASE
         LGD_LAUNCHED("conv3d_wgrad_mfma");
     }
-    conv3d_wgrad_reduce<<<(unsigned)((cout * Kp + kWgradReduceOutputs - 1) / kWgradReduceOutputs),
-                              dim3(kWgradReduceOutputs, kWgradReduceRows), 0, s>>>(P, parts, cout, Kp, K, dw,
-                                                                                    accumulate);
+    const unsigned outs = (unsigned)((cout * Kp + kWgradReduceOutputs - 1) / kWgradReduceOutputs);
+    if (outs >= 2 * lgdhip::kCUs)
+        conv3d_wgrad_reduce<4><<<outs, dim3(kWgradReduceOutputs, 4), 0, s>>>(P, parts, cout, Kp, K, dw, accumulate);
+    else
+        conv3d_wgrad_reduce<16><<<outs, dim3(kWgradReduceOutputs, 16), 0, s>>>(P, parts, cout, Kp, K, dw, accumulate);
     LGD_LAUNCHED("conv3d_wgrad_reduce");
     if (db) {
         const int bchunks = (int)((nvox + kBiasChunk - 1) / kBiasChunk);
