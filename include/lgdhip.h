@@ -510,8 +510,8 @@ int lgdhip_conv3d_bf16_dgrad_relu(const void *x, int n, int ldx, int offx, int c
                                   size_t workspace_bytes, lgdhip_stream_t stream);
 /* dw[co][k] (+)= sum_v dy[v][co] x[v+tap(k)][ci(k)] (FP32, fixed-order
  * reduction over voxel chunks), db[co] = sum_v dy[v][co] (if non-NULL).
- * 3x3x3 layers of aligned 8-channel rows are reduced over column chunks of
- * the library's choice; the others over chunks of chunk_vox voxels, a multiple
+ * 3x3x3 layers of aligned 8-channel rows, but for the smallest, are reduced
+ * over column chunks of the library's choice; the others over chunks of chunk_vox voxels, a multiple
  * of 32 (<= 0: the library's choice, a power of two from 128 to 4096).  Pass the
  * same value to the workspace query. */
 size_t lgdhip_conv3d_wgrad_workspace_bytes(int n, int cin, int ksize, int cout, int chunk_vox);

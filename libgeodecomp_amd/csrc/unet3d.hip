@@ -2035,6 +2035,21 @@ int wgrad_chunk(int n, int cin, int ksize, int cout) {
     return c;
 }
 
+// Modelled time (us) of the general kernel on small volumes, its reduction
+// included: what a wave's steps over its output tiles take, and the waves beyond
+// the few that run for nothing.  The column kernel takes 13 us on the smallest (14
+// with a masked row), its march and the epilogue of 27 taps.  Below that the general
+// kernel is the faster one (within 10 % where it measures less than 18; 4^3 64 -> 64
+// 10.0 against 12.8, 12^3 32 -> 16 10.2 / 12.7, 16^3 3 -> 16 9.3 / 13.3, 17^3 16 -> 16
+// 10.8 / 13.4, but 16^3 64 -> 16 14.6 / 13.2, 16^3 64 -> 64 28 / 18).
+double wgrad_gather_us(int n, int cin, int cout, int chunk_vox) {
+    const int64_t nvox = (int64_t)n * n * n;
+    const int tiles = (cout + 15) / 16;
+    const double steps = (double)((std::min<int64_t>(chunk_vox, nvox) + 31) / 32);
+    const double waves = (double)((nvox + chunk_vox - 1) / chunk_vox) * (lgdhip_conv3d_kpad(cin, 3) / 16);
+    return 8.3 + 0.33 * tiles * steps + 0.0014 * waves * (1 + 0.2 * (tiles - 1));
+}
+
 int check_tensor(int n, int ld, int off, int c) {
     if (n < 1 || ld < 1 || off < 0 || c < 1 || off + c > ld)
         return lgdhip::set_error(LGDHIP_ERR_INVALID_ARG, "bad tensor shape (n, ld, off, c)");
@@ -2296,7 +2311,8 @@ int lgdhip_conv3d_bf16_wgrad(const void *x, int n, int ldx, int offx, int cin, i
     int parts = chunks;
     const bool zm = wgrad_zm_shape(cin, ksize, cout) && ldx % 8 == 0 && offx % 8 == 0 && ldy % 8 == 0 &&
                     offy % 8 == 0 && (cin >= 8 || offx + 8 <= ldx) && (uintptr_t)x % 16 == 0 &&
-                    (uintptr_t)dy % 16 == 0 && (int64_t)n * n * std::max(ldx, ldy) < INT32_MAX;
+                    (uintptr_t)dy % 16 == 0 && (int64_t)n * n * std::max(ldx, ldy) < INT32_MAX &&
+                    wgrad_gather_us(n, cin, cout, chunk_vox) > (cin < 8 ? 14 : 13);
     if (zm) {
         const ZmWgrad w = wgrad_zm_plan(n, cin, cout);
         parts = w.chunks;

@@ -461,12 +461,12 @@ def run_wgrad_case(hip, oracle, n, cin, cout, ksize, chunk):
 @pytest.mark.gpu
 @pytest.mark.parametrize("n,cin,cout", [(17, 16, 16), (13, 24, 40), (33, 3, 16), (20, 3, 48), (31, 64, 128), (53, 192, 48),
                                         (30, 96, 128), (35, 64, 128), (45, 48, 128), (47, 64, 128), (68, 64, 96),
-                                        (1, 16, 16)])
+                                        (1, 16, 16), (25, 16, 16), (30, 24, 16), (49, 3, 16), (37, 3, 48)])
 def test_conv_wgrad_columns_vs_gather(hip, n, cin, cout):
     """The column kernel (every tile grouping, ragged columns and z chunks,
     channel counts that fill half a tile, one masked row) against the gather
     kernel, which the same values in rows of an odd stride take, with a second
-    call accumulating."""
+    call accumulating; the smallest layers take the gather kernel either way."""
     print("[case] conv wgrad columns", n, cin, cout, flush=True)
     rng = np.random.default_rng(n * cin + cout)
     x = rng.standard_normal((n ** 3, cin)).astype(np.float32)
@@ -957,7 +957,8 @@ def test_conv_zm_infinite_activations(hip, n, cin, cout):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("n,cin,cout", [(16, 16, 16), (17, 16, 16), (13, 24, 40), (33, 3, 16), (20, 3, 48), (31, 64, 128),
-                                        (32, 64, 32), (30, 96, 128), (45, 48, 128), (64, 32, 16), (1, 16, 16)])
+                                        (32, 64, 32), (30, 96, 128), (45, 48, 128), (64, 32, 16), (1, 16, 16),
+                                        (25, 16, 16), (30, 24, 16), (49, 3, 16), (37, 3, 48)])
 def test_conv_wgrad_infinite_activations(hip, n, cin, cout):
     """An infinite activation makes the weight gradients of its channel infinite
     (by the sign of the output gradient) for the taps that reach it inside the
