@@ -1980,6 +1980,22 @@ constexpr struct {
 // 3x3x3 layers whose 8-channel pieces are whole (or, for the network's first
 // layer, one masked row); the partials index rows of channels with 32 bits
 bool wgrad_zm_shape(int cin, int ksize, int cout) { return ksize == 3 && (cin % 8 == 0 || cin < 8) && cout % 8 == 0; }
+// Bytes of a voxel's c channels that groups of `tiles` 16-channel tiles read among
+// them when each group fetches whole 128-byte lines anew (a row below 128 bytes is
+// read whole by each).
+int wgrad_row_bytes(int c, int tiles) {
+    int lines = 0;
+    for (int a = 0; a < c; a += 16 * tiles) lines += (std::min(c, a + 16 * tiles) + 63) / 64 - a / 64;
+    return lines * std::min(128, 2 * c);
+}
+// Bytes of a voxel's c channels that the groups fetch beyond one row: none while
+// the volume stays in the L2s between the groups that share its lines; past 28 MB
+// of their 32 most of each line (0.65: the least total time over 425 layers timed
+// in every grouping, 2 % above the best of each; 11 % without).
+double wgrad_refetch(int n, int c, int tiles) {
+    const double row = 2.0 * c;
+    return row * n * n * n > 28e6 ? 0.65 * std::max(0.0, wgrad_row_bytes(c, tiles) - row) : 0.0;
+}
 ZmWgrad wgrad_zm_plan(int n, int cin, int cout) {
     const int cit = (cin + 15) / 16, cot = (cout + 15) / 16;
     ZmWgrad best{};
@@ -1989,6 +2005,12 @@ ZmWgrad wgrad_zm_plan(int n, int cin, int cout) {
         if (cin < 8 && c.to > 2) continue;
         ZmWgrad w{c.ti, c.to, c.ks, (cit + c.ti - 1) / c.ti, (cot + c.to - 1) / c.to, (n + 15) / 16, (n + 7) / 8, 0, 0};
         const int waves = c.ti * c.to * c.ks, resident = waves == 4 ? 3 : 1;
+        // what the groups' shares of a 128-byte line cost on top (us): a part of the
+        // grouping alone, the chunk length is chosen by the rest.  MI355X, us, without
+        // it / with it: 72^3 64 -> 64 404 / 114, 72^3 64 -> 32 148 / 59, 88^3 64 -> 16
+        // 120 / 71, 120^3 3 -> 128 383 / 232; it costs 108^3 3 -> 128 230 / 243.
+        const double lines =
+            (double)n * n * n * (w.go * wgrad_refetch(n, cin, c.ti) + w.gi * wgrad_refetch(n, cout, c.to)) / 4.5e6;
         for (int zc = 2; zc <= 64; zc *= 2) {
             w.zchunk = zc;
             w.chunks = w.bx * w.by * ((n + zc - 1) / zc);
@@ -2003,7 +2025,7 @@ ZmWgrad wgrad_zm_plan(int n, int cin, int cout) {
             const double march = rounds * ((zc + 2) * std::max(0.7, products) + 4.0);
             const double partials = 2.0 * w.chunks * cout * lgdhip_conv3d_kpad(cin, 3) * 4 / 4e6;
             const double tensors = 2.0 * n * n * n * (1.4 * (zc + 2) / zc * w.go * cin + (double)w.gi * cout) / 4.5e6;
-            const double us = std::max(march, tensors) + partials;
+            const double us = std::max(march, tensors) + partials + lines;
             if (us < best_us) {
                 best_us = us;
                 best = w;
