@@ -2059,17 +2059,30 @@ int wgrad_chunk(int n, int cin, int ksize, int cout) {
 
 // Modelled time (us) of the general kernel on small volumes, its reduction
 // included: what a wave's steps over its output tiles take, and the waves beyond
-// the few that run for nothing.  The column kernel takes 13 us on the smallest (14
-// with a masked row), its march and the epilogue of 27 taps.  Below that the general
-// kernel is the faster one (within 10 % where it measures less than 18; 4^3 64 -> 64
-// 10.0 against 12.8, 12^3 32 -> 16 10.2 / 12.7, 16^3 3 -> 16 9.3 / 13.3, 17^3 16 -> 16
-// 10.8 / 13.4, but 16^3 64 -> 16 14.6 / 13.2, 16^3 64 -> 64 28 / 18).
+// the few that run for nothing.
 double wgrad_gather_us(int n, int cin, int cout, int chunk_vox) {
     const int64_t nvox = (int64_t)n * n * n;
     const int tiles = (cout + 15) / 16;
     const double steps = (double)((std::min<int64_t>(chunk_vox, nvox) + 31) / 32);
     const double waves = (double)((nvox + chunk_vox - 1) / chunk_vox) * (lgdhip_conv3d_kpad(cin, 3) / 16);
     return 8.3 + 0.33 * tiles * steps + 0.0014 * waves * (1 + 0.2 * (tiles - 1));
+}
+
+// The column kernel takes 14 us on the smallest layers (with a masked row 0.55 more
+// for each further output tile), its march and the epilogue of 27 taps.  Below that
+// the general kernel is the faster one (4^3 64 -> 64 10.0 against 12.8, 12^3 32 -> 16
+// 10.2 / 12.7, 16^3 3 -> 16 9.3 / 13.3, 17^3 16 -> 16 10.8 / 13.4, 16^3 24 -> 32 12.4
+// / 14.3, 24^3 1 -> 64 14.4 / 16.8; over 0.75 to 1 beyond the line 13.8 on average
+// against 13.9, over 1 to 1.5 15.8 / 14.5; 16^3 64 -> 64 28 / 18).
+// A single input channel is 27 columns of k, two tiles for the general kernel, and a
+// masked row with 27 taps for the column kernel.  With 4 output tiles or more the
+// latter's groups re-fetch dY's lines on middle volumes, whose columns also leave
+// many of its waves short (us, general / column: 68^3 1 -> 64 46 / 49, 88^3 1 -> 64
+// 77 / 80, 68^3 1 -> 128 62 / 74, 88^3 1 -> 128 107 / 134; 64^3 1 -> 128 52 / 39,
+// 96^3 1 -> 128 146 / 135).
+bool wgrad_columns_pay(int n, int cin, int cout, int chunk_vox) {
+    if (cin == 1 && cout > 48 && n > 64 && n < 96) return false;
+    return wgrad_gather_us(n, cin, cout, chunk_vox) > 14 + (cin < 8 ? 0.55 * ((cout - 1) / 16) : 0);
 }
 
 int check_tensor(int n, int ld, int off, int c) {
@@ -2334,7 +2347,7 @@ int lgdhip_conv3d_bf16_wgrad(const void *x, int n, int ldx, int offx, int cin, i
     const bool zm = wgrad_zm_shape(cin, ksize, cout) && ldx % 8 == 0 && offx % 8 == 0 && ldy % 8 == 0 &&
                     offy % 8 == 0 && (cin >= 8 || offx + 8 <= ldx) && (uintptr_t)x % 16 == 0 &&
                     (uintptr_t)dy % 16 == 0 && (int64_t)n * n * std::max(ldx, ldy) < INT32_MAX &&
-                    wgrad_gather_us(n, cin, cout, chunk_vox) > (cin < 8 ? 14 : 13);
+                    wgrad_columns_pay(n, cin, cout, chunk_vox);
     if (zm) {
         const ZmWgrad w = wgrad_zm_plan(n, cin, cout);
         parts = w.chunks;

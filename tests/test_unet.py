@@ -462,7 +462,8 @@ def run_wgrad_case(hip, oracle, n, cin, cout, ksize, chunk):
 @pytest.mark.parametrize("n,cin,cout", [(17, 16, 16), (13, 24, 40), (33, 3, 16), (20, 3, 48), (31, 64, 128), (53, 192, 48),
                                         (30, 96, 128), (35, 64, 128), (45, 48, 128), (47, 64, 128), (68, 64, 96),
                                         (1, 16, 16), (25, 16, 16), (30, 24, 16), (49, 3, 16), (37, 3, 48),
-                                        (61, 3, 64), (67, 64, 64), (61, 64, 16)])
+                                        (61, 3, 64), (67, 64, 64), (61, 64, 16),
+                                        (65, 1, 64), (24, 3, 64)])
 def test_conv_wgrad_columns_vs_gather(hip, n, cin, cout):
     """The column kernel (every tile grouping, ragged columns and z chunks,
     channel counts that fill half a tile, one masked row) against the gather
