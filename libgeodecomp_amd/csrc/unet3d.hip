@@ -1522,9 +1522,11 @@ __global__ __launch_bounds__(64 * TI * TO * KS, TI * TO * KS == 4 ? 3 : 1) void 
 // sums the chunks j, j + ROWS, j + 2 ROWS, ... (eight loads in flight, coalesced
 // across the 64 outputs) and the row sums are added in row order: a fixed
 // order for every output.  16 rows where the outputs are fewer than two
-// work-groups per CU (16 -> 16: 112 of them; 128^3 40.1 us with the column kernel,
+// work-groups per CU and have more than 16 chunks (16 -> 16: 112 of them; 128^3 40.1 us with the column kernel,
 // 44.1 with 4 rows), else 4: wide layers have few chunks on small volumes, and
 // rows without one cost their launch (16^3 128 -> 128 21.3 us, 32.0 with 16 rows).
+// The same holds for 16 chunks or fewer: 1^3 7.9 us with 4 rows, 9.6 with 16, 4^3
+// 9.2 / 10.3, 8^3 11.2 / 11.8 (mean over 48 layers; alike with 16 to 64 chunks).
 constexpr int kWgradReduceOutputs = 64;
 template <int ROWS>
 __global__ __launch_bounds__(kWgradReduceOutputs *ROWS) void conv3d_wgrad_reduce(const float *__restrict__ P,
@@ -2396,7 +2398,7 @@ int lgdhip_conv3d_bf16_wgrad(const void *x, int n, int ldx, int offx, int cin, i
         LGD_LAUNCHED("conv3d_wgrad_mfma");
     }
     const unsigned outs = (unsigned)((cout * Kp + kWgradReduceOutputs - 1) / kWgradReduceOutputs);
-    if (outs >= 2 * lgdhip::kCUs)
+    if (outs >= 2 * lgdhip::kCUs || parts <= 16)
         conv3d_wgrad_reduce<4><<<outs, dim3(kWgradReduceOutputs, 4), 0, s>>>(P, parts, cout, Kp, K, dw, accumulate);
     else
         conv3d_wgrad_reduce<16><<<outs, dim3(kWgradReduceOutputs, 16), 0, s>>>(P, parts, cout, Kp, K, dw, accumulate);
