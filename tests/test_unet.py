@@ -468,7 +468,8 @@ def test_conv_wgrad_columns_vs_gather(hip, n, cin, cout):
     """The column kernel (every tile grouping, ragged columns and z chunks,
     channel counts that fill half a tile, one masked row) against the gather
     kernel, which the same values in rows of an odd stride take, with a second
-    call accumulating; the smallest layers take the gather kernel either way."""
+    call accumulating; the smallest layers and 65^3 1 -> 64 take the gather kernel
+    either way."""
     print("[case] conv wgrad columns", n, cin, cout, flush=True)
     rng = np.random.default_rng(n * cin + cout)
     x = rng.standard_normal((n ** 3, cin)).astype(np.float32)
